@@ -44,27 +44,9 @@
 #include <string>
 #include <type_traits>
 
-#include "cbx_core.hpp"
-#include "cbx_host.hpp"
+#include "cbx_draw.hpp"
 
 namespace cbx {
-
-template <typename T>
-struct Segment {
-    int32_t line;
-    int32_t c[2];   // walk position at the segment's first column
-    int32_t ncols;  // long-axis columns covered from c[axis] in the walk direction
-    T Te, Ne;       // walk errors at that position
-    int32_t lo, hi; // short-axis pixel range the fills can reach, clipped to the frame
-};
-
-struct Geometry {
-    int64_t n_frames;
-    int32_t H, W;
-    int32_t tile, seg;
-    int32_t ntx, nty;
-    int32_t skip_neg = 0;   // 1: a line with a negative frame draws nothing (accumulate_lines term batches)
-};
 
 // ---------------------------------------------------------------------------
 // segment pre-passes
@@ -97,6 +79,25 @@ __device__ __forceinline__ bool setup_line(const T *__restrict__ lines, const I 
     }
     L.frame = (int32_t)f;
     return L.valid;
+}
+
+__device__ __forceinline__ LineLite line_lite(const LineSetup<float> &L)
+{
+    const int a = L.axis, b = 1 - a;
+    LineLite r;
+    r.t[0] = L.t[0];
+    r.t[1] = L.t[1];
+    r.LL = L.LL;
+    r.ea = L.ea;
+    r.nlim = L.nlim;
+    // A fill visits at most J = nlim / |t_a| + 2 steps from its column, each
+    // moving Te by |t_b| and rounding it by at most half an ulp of LL + cap.
+    const float J = L.nlim / m_abs(pick(L.t, a)) + 2.0f;
+    r.cap = J * (m_abs(pick(L.t, b)) * 1.00001f + L.LL * 2.4e-7f);
+    r.meta = a | (pick(L.st, a) > 0 ? FR_SA : 0) | (pick(L.st, b) > 0 ? FR_SB : 0) | (L.safe ? FR_SAFE : 0) |
+             ((int)(uint8_t)L.kid << 8);
+    r.pad = 0;
+    return r;
 }
 
 // Most segments a line's walk can make: one per SEG-column block of the
@@ -145,6 +146,9 @@ __device__ __forceinline__ void walk_segments(const LineSetup<T> &L, int64_t l, 
         if (lo > hi) return;
         cur.lo = lo;
         cur.hi = hi;
+        // every long-axis step emits the column it leaves: the emitted columns
+        // are the block's first nem
+        cur.ncols = nem;
         on_seg(cur, tl);
     };
 
@@ -195,7 +199,6 @@ __device__ __forceinline__ void walk_segments(const LineSetup<T> &L, int64_t l, 
         cur.c[1] = s.c[1];
         cur.Te = s.Te;
         cur.Ne = s.Ne;
-        cur.ncols = (sa > 0) ? (b_hi - c0) : (c0 - b_lo + 1);
         // One exit test per step: the long-axis coordinate moves by 0 or sa
         // per step and starts inside the block [b_lo, b_hi), which lies
         // inside the frame, so the block (and the frame) is left exactly at
@@ -300,7 +303,7 @@ template <typename T, typename I>
 __global__ void __launch_bounds__(256)
 k_setup_lines(const T *__restrict__ lines, const I *__restrict__ idxs, const uint8_t *__restrict__ kernels,
               int kernel, int64_t n_lines, Geometry g, LineSetup<T> *__restrict__ setup,
-              unsigned long long *__restrict__ counters, int *__restrict__ flags)
+              LineLite *__restrict__ lite, unsigned long long *__restrict__ counters, int *__restrict__ flags)
 {
     const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int ub = 0;
@@ -308,6 +311,7 @@ k_setup_lines(const T *__restrict__ lines, const I *__restrict__ idxs, const uin
         LineSetup<T> L;
         setup_line(lines, idxs, kernels, kernel, l, g, L, flags);
         setup[l] = L;
+        if constexpr (sizeof(T) == 4) lite[l] = line_lite(L);
         ub = segment_bound(L, g);
     }
 #pragma unroll
@@ -319,18 +323,6 @@ k_setup_lines(const T *__restrict__ lines, const I *__restrict__ idxs, const uin
     if ((threadIdx.x & 63) == 0 && ub) atomicAdd(&bsum, (unsigned long long)ub);
     __syncthreads();
     if (threadIdx.x == 0 && bsum) atomicAdd(&counters[0], bsum);
-}
-
-// The unordered plan's item list of tile t is split into LIST_SUBS sub-lists
-// by the binning wave (slot / 64 mod LIST_SUBS), so that the cursor atomics
-// of a dense tile spread over LIST_SUBS counters; the sub-lists are
-// contiguous: tile t's items are [tile_off[t * LIST_SUBS],
-// tile_off[(t + 1) * LIST_SUBS]).
-constexpr int LIST_SUBS = 8;
-
-__device__ __forceinline__ int64_t list_index(int64_t tile, int64_t slot)
-{
-    return tile * LIST_SUBS + ((slot >> 6) & (LIST_SUBS - 1));
 }
 
 // Records per thread in the walk's LDS ring: 2 (16 KB per 256 threads; a
@@ -560,581 +552,6 @@ k_bin_slots(int64_t n_slots, Geometry g, const LineSetup<T> *__restrict__ setup,
         if (act && lane == leader) b = atomicAdd(&cur[key], __popcll(grp));
         b = __shfl(b, leader, 64);
         if (act) pairs[tile_off[key] + b + __popcll(grp & below)] = item;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// shared pieces of the tile kernels
-// ---------------------------------------------------------------------------
-template <typename T>
-struct ColRec {
-    int32_t s; // short-axis centre, INT_MIN when the column is not emitted
-    T Te, Ne;
-};
-
-struct ItemHdr {
-    int32_t seg;
-    int32_t line;
-};
-
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Phase 1: replay a segment's walk from its checkpoint and record, for each
-// of its columns, the centre and errors at which the reference emits it, in
-// the column slots i * SEG + k of item i of rr.
-template <typename T, int SEG>
-__device__ __forceinline__ void walk_columns(const LineSetup<T> &L, const Segment<T> &sg, ColRec<T> *rr, int i,
-                                             int *flags)
-{
-    for (int k = 0; k < SEG; k++) rr[i * SEG + k].s = INT_MIN;
-    const int a = L.axis, b = 1 - a, sa = pick(L.st, a);
-    WalkState<T> s;
-    s.c[0] = sg.c[0];
-    s.c[1] = sg.c[1];
-    s.Te = sg.Te;
-    s.Ne = sg.Ne;
-    const int c0 = pick(s.c, a);
-    int it = 0;
-    for (; it < 4 * SEG + 16; it++) {
-        if (walk_done(L, s)) break;
-        const int k = (pick(s.c, a) - c0) * sa;
-        if (k >= sg.ncols) break;
-        bool nx, ny;
-        walk_next(L, s.Ne, nx, ny);
-        if ((a == 0) ? nx : ny) {
-            ColRec<T> &r = rr[i * SEG + k];
-            r.s = pick(s.c, b);
-            r.Te = s.Te;
-            r.Ne = s.Ne;
-        }
-        walk_step(L, s, nx, ny);
-    }
-    if (it == 4 * SEG + 16) atomicOr(flags, FLAG_STUCK);
-}
-
-// Phase 2: the orthogonal fills of one emitted column (bresenham.hpp:364-380),
-// restricted to the short-axis window [s_lo, s_hi); emit(s, err) is called
-// for every pixel of the window the reference would hand to draw_pixel.
-template <typename T, typename Emit>
-__device__ __forceinline__ void fill_column(const LineSetup<T> &L, const ColRec<T> &cr, int s_lo, int s_hi,
-                                            Emit &&emit)
-{
-    const int b = 1 - L.axis;
-    if (cr.s >= s_lo && cr.s < s_hi) emit(cr.s, cr.Te, cr.Ne);
-    const T tb = pick(L.t, b), nb = pick(L.nv, b);
-    const int sb = pick(L.st, b);
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-        const int dir = half ? -sb : sb;
-        const T dT = (dir > 0) ? tb : -tb, dN = (dir > 0) ? nb : -nb;
-        int s = cr.s;
-        T Te = cr.Te, Ne = cr.Ne;
-        for (;;) {
-            s += dir;
-            Te += dT;
-            Ne += dN;
-            if (!(nsq_of(L, Ne) < L.w2)) break;
-            if (s >= s_lo && s < s_hi) emit(s, Te, Ne);
-            else if ((dir > 0) ? (s >= s_hi) : (s < s_lo)) break;
-        }
-    }
-}
-
-// LDS accumulator of the tile kernel, by accumulation mode OV:
-//   0  sums in double (on gfx950 ds_add_f64 sustains ~20x the lane rate of
-//      ds_add_f32; the tile is rounded to the image type once, at the flush)
-//   1  max overlap, as order-preserving unsigned codes (ds_max)
-//   2  float sums in 32-bit fixed point (ds_add_u32, the fastest LDS atomic,
-//      at half the LDS of double; see k_tiles)
-template <typename T, int OV>
-struct AccType {
-    using type = double;
-};
-template <>
-struct AccType<float, 1> {
-    using type = uint32_t;
-};
-template <>
-struct AccType<double, 1> {
-    using type = unsigned long long;
-};
-template <>
-struct AccType<float, 2> {
-    using type = uint32_t;
-};
-
-// Adds one pixel value to the LDS tile.  For OV = 2, v is the profile value
-// already scaled by the round's 2^F; exact zeros only mark the pixel touched.
-// POS: v is known to be positive (and, for OV = 2, at least 1).
-template <int OV, bool POS = false, typename Acc, typename V>
-__device__ __forceinline__ void tile_put(Acc *img, uint32_t *zb, int idx, V v)
-{
-    if constexpr (OV == 0) {
-        atomicAdd(&img[idx], (Acc)v);
-    } else if constexpr (OV == 1) {
-        if (v == v) atomicMax(&img[idx], ord_enc(v));
-    } else if constexpr (POS) {
-        atomicAdd(&img[idx], __float2uint_rn((float)v));
-    } else {
-        if (v > 0.0f) atomicAdd(&img[idx], max(1u, __float2uint_rn((float)v)));
-        else atomicOr(&zb[idx >> 5], 1u << (idx & 31));
-    }
-}
-
-// ---------------------------------------------------------------------------
-// 4. tile kernel (image mode)
-// ---------------------------------------------------------------------------
-// Per-item record in LDS, written by the phase-1 thread that replays the
-// item's walk (it holds the line's setup in registers) and read by the
-// phase-2 threads of its columns: the item's line and first long-axis
-// coordinate, and for float lines the fast path's constants, so the fills
-// need no global load (the exact error near the threshold reads the setup).
-struct alignas(16) FillRec {
-    float LL, ea, nlim;
-    float tb, nb;     // tangent and normal components along the short axis b
-    int32_t c0;       // long-axis coordinate of the item's first column
-    int32_t line;
-    int32_t meta;     // FR_* bits, profile id in bits 8-15
-};
-constexpr int FR_AXIS = 1, FR_SA = 2, FR_SB = 4, FR_SAFE = 8;
-
-template <typename T>
-__device__ __forceinline__ FillRec fill_rec(const LineSetup<T> &L, int c0, int line)
-{
-    FillRec r;
-    const int a = L.axis, b = 1 - a;
-    r.c0 = c0;
-    r.line = line;
-    r.meta = a | (pick(L.st, a) > 0 ? FR_SA : 0) | (pick(L.st, b) > 0 ? FR_SB : 0) |
-             (sizeof(T) == 4 && L.safe ? FR_SAFE : 0) | ((int)L.kid << 8);
-    r.LL = (float)L.LL;
-    r.ea = L.ea;
-    r.nlim = L.nlim;
-    r.tb = (float)pick(L.t, b);
-    r.nb = (float)pick(L.nv, b);
-    return r;
-}
-
-// The fills of one column half for the float fast path (lines with L.safe):
-// the band test |Ne| < nlim, the one-product error estimate (err_fast), the
-// profile's constant folded into the column's value scale and the tile window
-// turned into a skip count and a trip count, with the LDS index stepped per
-// pixel.  The errors advance by the same FP32 additions as the reference's
-// loop.  Lg is the line's setup in global memory, read only for exact errors
-// near the threshold.  vscale is max_val (OV 0, 1) or the fixed-point scale
-// 2^F (OV 2: F >= 20, so positive profiles give values of at least 1).
-template <int K, int OV, typename Acc>
-__device__ __forceinline__ void fill_half_fast(Acc *img, uint32_t *zb, const FillRec &R,
-                                               const LineSetup<float> &Lg, int cs, float Te, float Ne, int half,
-                                               int cbase, int sstride, int s_lo, int s_hi, float vscale)
-{
-    constexpr bool POS = (OV == 2) && fast_positive<K>();
-    const float LL = R.LL, ea = R.ea, nlim = R.nlim;
-    const int kid = R.meta >> 8;
-    const int sb = (R.meta & FR_SB) ? 1 : -1;
-    const int dir = half ? -sb : sb;
-    const float dT = (dir > 0) ? R.tb : -R.tb, dN = (dir > 0) ? R.nb : -R.nb;
-    const float c = fast_scale<K>(kid, vscale);
-    auto put = [&](int idx, float T, float N) {
-        const float e = err_fast(Lg, LL, ea, T, N);
-        if (e <= 1.0f) tile_put<OV, POS>(img, zb, idx, fast_value<K>(kid, e, c));
-    };
-    wait_lds_loads();
-    if (half == 0 && cs >= s_lo && cs < s_hi) put(cbase + (cs - s_lo) * sstride, Te, Ne);
-    // steps to the last in-window pixel in the direction of travel, and the
-    // first step that lands inside the window
-    const int nsteps = (dir > 0) ? (s_hi - 1 - cs) : (cs - s_lo);
-    if (nsteps < 1) return;
-    const int jin = max(1, (dir > 0) ? (s_lo - cs) : (cs - s_hi + 1));
-    for (int j = 1; j < jin; j++) {
-        Te += dT;
-        Ne += dN;
-        if (!(__builtin_fabsf(Ne) < nlim)) return;
-    }
-    const int step = dir * sstride;
-    int idx = cbase + (cs + jin * dir - s_lo) * sstride;
-    for (int j = jin; j <= nsteps; j++, idx += step) {
-        Te += dT;
-        Ne += dN;
-        if (!(__builtin_fabsf(Ne) < nlim)) return;
-        put(idx, Te, Ne);
-    }
-}
-
-// Value a fixed-point tile pixel adds to the image: acc * max_val * 2^-F, or
-// max_val * 0 (the sign rules of adding exact zeros) if only zeros touched
-// it.  has = false: the pixel was not touched.
-__device__ __forceinline__ double fix_value(uint32_t acc, const uint32_t *zb, int i, double scale, float max_val,
-                                            bool &has)
-{
-    has = acc != 0u || ((zb[i >> 5] >> (i & 31)) & 1u);
-    return acc ? (double)acc * scale : (double)(max_val * 0.0f);
-}
-
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-// fix_value for a pixel already in a register, in float: o + (acc 2^-F)
-// max_val (or + zero, the value of exact zeros, when only zeros touched it:
-// zbit set), or o untouched.  acc 2^-F is exact (p2 = 2^-F); the rounding of
-// acc to 24 bits and of the two operations stays below 2e-7 of the pixel's
-// value, far inside the fixed-point terms' own error (<= 2^-F max_val each).
-__device__ __forceinline__ float fold_fix(float o, uint32_t acc, uint32_t zbit, float p2, float max_val, float zero)
-{
-    const float add = acc ? ((float)acc * p2) * max_val : zero;
-    return (acc | zbit) ? o + add : o;
-}
-
-// LDS row pitch of the adjoint's gradient tile, in words: 4 words of padding
-// per row.  The lanes of one item read the same short-axis coordinate in 8 or
-// 16 consecutive rows (steep lines); with a pitch of TILE (a multiple of the
-// bank count) those reads fall in one bank, with TILE + 4 in distinct banks.
-// (The tile kernel keeps a pitch of TILE: its padded variants measured slower,
-// see k_tiles.)
-template <int TILE>
-constexpr int tile_pitch() { return TILE + 4; }
-
-// Tile kernel.  The workgroup takes its tile's items ((segment, line) pairs)
-// in chunks of CH <= NT: phase 1 gives each of CH threads one item (the walk
-// replay, column records into LDS); phase 2 gives each thread one (item,
-// column, half) unit of the fills at a time.  The first chunk's loads and
-// (256-thread float sum tiles) the tile's current values in `out` are
-// requested before the LDS tile is cleared, so their latency overlaps.
-//
-// Fixed-point sums (OV = 2): an item (one segment in one tile) adds at most
-// one value per pixel, so a round of n items adds at most n values of at most
-// 2^F with F = clz(n): the sum stays below 2^32.  Each value p > 0 adds
-// max(1, rn(p 2^F)) (absolute error <= 2^-F max_val per term, so a touched
-// pixel stays non-zero); exact zeros set a bit in zb.  Tiles of more than
-// FIX_ROUND items take several rounds, folded into the running pixel values.
-constexpr int FIX_ROUND = 4095;
-
-// (at least 5 waves per SIMD: the fastest register budget measured)
-template <typename T, int K, int OV, int TILE, int SEG, int NT, int CH, bool FAST>
-__global__ void __launch_bounds__(NT, 5)
-k_tiles(T *__restrict__ out, Geometry g, const int *__restrict__ tile_off, const int2 *__restrict__ pairs,
-        const Segment<T> *__restrict__ segs, const LineSetup<T> *__restrict__ setup, T max_val,
-        int *__restrict__ flags)
-{
-    using Acc = typename AccType<T, OV>::type;
-    static_assert(OV != 2 || (FAST && sizeof(T) == 4), "fixed-point sums are the float fast path");
-    // LDS pitch TILE: the bank conflicts of the fills (steep lines write one
-    // bank from consecutive rows, the two halves of a column share a bank) and
-    // of the strided item records cost less than removing them did (a padded
-    // pitch and rotated record slots spilled registers at 5 waves per SIMD or
-    // dropped to 4)
-    constexpr int PITCH = TILE;
-    constexpr int LDS_PX = TILE * PITCH;   // LDS words of the tile (pixel (y, x) at y * PITCH + x)
-    __shared__ alignas(16) Acc img[LDS_PX];
-    __shared__ uint32_t zb[OV == 2 ? LDS_PX / 32 : 1];
-    static_assert(CH <= NT, "one phase-1 thread per item");
-    __shared__ int32_t rs[CH * SEG + CH];   // + one sink slot per phase-1 lane
-    __shared__ T rT[CH * SEG + CH];
-    __shared__ T rN[CH * SEG + CH];
-    __shared__ FillRec frec[CH];
-
-    const int tile = blockIdx.x;
-    // (one round trip for the item range and the error flags: a plan's draw
-    // reports errors afterwards and leaves `out` untouched then)
-    const int beg = tile_off[tile * LIST_SUBS], end = tile_off[(tile + 1) * LIST_SUBS];
-    const int fl = *flags;
-    if (fl || beg == end) return;
-    const int per_frame = g.ntx * g.nty;
-    const int64_t f = tile / per_frame;
-    const int r = tile - (int)f * per_frame;
-    const int ty = r / g.ntx, tx = r - ty * g.ntx;
-    const int X0 = tx * TILE, Y0 = ty * TILE;
-    const int X1 = min(X0 + TILE, g.W), Y1 = min(Y0 + TILE, g.H);
-    const int tid = threadIdx.x;
-    T *fo = out + (f * g.H) * (int64_t)g.W;
-    constexpr int V = 4;
-    const bool full = (X1 - X0 == TILE) && ((g.W & (V - 1)) == 0) && (((uintptr_t)out & 15) == 0);
-
-    // the tile's current values, for the flush (float sums, 256 threads:
-    // 4 float4 per thread), requested first
-    constexpr bool PREF = (OV != 1) && sizeof(T) == 4 && NT == 256 && TILE == 64;
-    constexpr int PV = PREF ? (TILE * TILE) / (NT * V) : 1;
-    float4 pre[PV];
-    if constexpr (PREF) {
-        if (full) {
-#pragma unroll
-            for (int j = 0; j < PV; j++) {
-                const int i = (tid + j * NT) * V;
-                const int y = Y0 + i / TILE, x = X0 + (i % TILE);
-                if (y < Y1) {
-                    const v4f q = __builtin_nontemporal_load(reinterpret_cast<const v4f *>(fo + (int64_t)y * g.W + x));
-                    pre[j] = make_float4(q.x, q.y, q.z, q.w);
-                }
-            }
-        }
-    }
-    // first chunk's item loads (after the tile's loads, which do not wait on them)
-    Segment<T> sg0;
-    LineSetup<T> L0;
-    if (tid < min(CH, end - beg)) {
-        const int2 it = pairs[beg + tid];
-        sg0 = segs[it.x];
-        L0 = setup[it.y];
-    }
-
-    auto clear = [&]() {
-        if constexpr (OV != 0 && sizeof(Acc) == 4) {
-            // zero words (below every max code / empty fixed-point sum), 16 bytes per store
-            static_assert(LDS_PX % 4 == 0, "whole 16-byte stores");
-            uint4 *p = reinterpret_cast<uint4 *>(img);
-            for (int i = tid; i < LDS_PX / 4; i += NT) p[i] = make_uint4(0u, 0u, 0u, 0u);
-        } else {
-            for (int i = tid; i < LDS_PX; i += NT) {
-                if constexpr (OV == 0) img[i] = Acc(-0.0); // additive identity, keeps -0.0 pixels intact
-                else img[i] = Acc(0);                      // below every max code
-            }
-        }
-        if constexpr (OV == 2)
-            for (int i = tid; i < LDS_PX / 32; i += NT) zb[i] = 0u;
-    };
-    clear();
-
-    // rounds [rb, re): one for OV 0 / 1, FIX_ROUND items each for OV 2
-    for (int rb = beg, re; rb < end; rb = re) {
-        re = (OV == 2) ? rb + min(FIX_ROUND, end - rb) : end;
-        const int F = (OV == 2) ? __clz(re - rb) : 0;
-        // value scale: max_val, or 2^F for fixed-point sums
-        const T vscale = (OV == 2) ? (T)__int_as_float((127 + F) << 23) : max_val;
-        if (rb != beg) {
-            __syncthreads();
-            clear();
-        }
-        for (int first = rb; first < re; first += CH) {
-            const int n = min(CH, re - first);
-            // (phase 1 writes only the item records: the first chunk needs no
-            // barrier after the clear)
-            if (first != beg) __syncthreads();
-            // phase 1: replay the walk of one item from its checkpoint and
-            // record the centre and errors of every emitted column
-            if (tid < n) {
-                Segment<T> sg;
-                LineSetup<T> L;
-                if (first == beg) {
-                    sg = sg0;
-                    L = L0;
-                } else {
-                    const int2 it = pairs[first + tid];
-                    sg = segs[it.x];
-                    L = setup[it.y];
-                }
-                const int a = L.axis, sa = pick(L.st, a);
-                const int c0 = pick(sg.c, a);
-                // per-line profiles: the wave's items take their record slots
-                // grouped by profile, so the fills of a wave mostly share one
-                // (fixed-point sums do not depend on the item order)
-                int dst = tid;
-                if constexpr (K == K_MIXED) {
-                    const int kc = (L.kid >= 0 && L.kid < K_TRIANGULAR) ? L.kid : K_TRIANGULAR;
-                    const uint64_t below = (1ull << (tid & 63)) - 1ull;
-                    int off = 0, rank = 0;
-#pragma unroll
-                    for (int k = 0; k <= K_TRIANGULAR; k++) {
-                        const uint64_t m = __ballot(kc == k);
-                        if (kc == k) rank = off + __popcll(m & below);
-                        off += __popcll(m);
-                    }
-                    dst = (tid & ~63) + rank;
-                }
-                frec[dst] = fill_rec(L, c0, sg.line);
-#pragma unroll
-                for (int k = 0; k < SEG; k++) rs[dst * SEG + k] = INT_MIN;
-                WalkState<T> s;
-                s.c[0] = sg.c[0];
-                s.c[1] = sg.c[1];
-                s.Te = sg.Te;
-                s.Ne = sg.Ne;
-                // a loop uniform over the wave: lanes whose walk has ended are
-                // masked by predicates and store into their sink slot
-                bool act = true;
-                for (int it = 0; it < 4 * SEG + 16; it++) {
-                    act = act && !walk_done(L, s);
-                    const int k = (pick(s.c, a) - c0) * sa;
-                    act = act && k < sg.ncols;
-                    if (__ballot(act) == 0) break;
-                    bool nx, ny;
-                    walk_next(L, s.Ne, nx, ny);
-                    const bool rec = act && ((a == 0) ? nx : ny);
-                    const int slot = rec ? dst * SEG + k : CH * SEG + tid;
-                    rs[slot] = pick(s.c, 1 - a);
-                    rT[slot] = s.Te;
-                    rN[slot] = s.Ne;
-                    walk_step(L, s, act && nx, act && ny);
-                }
-                if (act) atomicOr(flags, FLAG_STUCK);   // still walking after the step budget
-            }
-            __syncthreads();
-            // phase 2: one thread per (item, column, half); the centre goes
-            // with the half that steps in +st[b] (bresenham.hpp:364-380)
-            for (int u = tid; u < n * SEG * 2; u += NT) {
-                const int i = u / (2 * SEG), rem = u - i * (2 * SEG);
-                const int k = rem >> 1, half = rem & 1;
-                const int slot = i * SEG + k;
-                const int cs = rs[slot];
-                if (cs == INT_MIN) continue;
-                const FillRec R = frec[i];
-                const int a = R.meta & FR_AXIS, b = 1 - a;
-                const int c = R.c0 + ((R.meta & FR_SA) ? k : -k);
-                const int s_lo = (a == 0) ? Y0 : X0, s_hi = (a == 0) ? Y1 : X1;
-                // LDS stride of the short axis and offset of the long-axis column
-                const int sstride = (a == 0) ? PITCH : 1;
-                const int cbase = (a == 0) ? (c - X0) : (c - Y0) * PITCH;
-                T Te = rT[slot], Ne = rN[slot];
-                if constexpr (FAST && sizeof(T) == 4) {
-                    if (R.meta & FR_SAFE) {
-                        fill_half_fast<K, OV>(img, zb, R, setup[R.line], cs, Te, Ne, half, cbase, sstride, s_lo,
-                                              s_hi, (float)vscale);
-                        continue;
-                    }
-                }
-                const LineSetup<T> L = setup[R.line];
-                auto put = [&](int s, T Te_, T nsq) {
-                    T v;
-                    if (!pixel_eval<FAST, K>(L, Te_, nsq, vscale, v)) return;
-                    tile_put<OV>(img, zb, cbase + (s - s_lo) * sstride, v);
-                };
-                if (half == 0 && cs >= s_lo && cs < s_hi) put(cs, Te, nsq_of(L, Ne));
-                const int sb = pick(L.st, b);
-                const int dir = half ? -sb : sb;
-                const T tb = pick(L.t, b), nb = pick(L.nv, b);
-                const T dT = (dir > 0) ? tb : -tb, dN = (dir > 0) ? nb : -nb;
-                int s = cs;
-                for (;;) {
-                    s += dir;
-                    Te += dT;
-                    Ne += dN;
-                    const T nsq = nsq_of(L, Ne);
-                    if (!(nsq < L.w2)) break;
-                    if (s >= s_lo && s < s_hi) put(s, Te, nsq);
-                    else if ((dir > 0) ? (s >= s_hi) : (s < s_lo)) break;
-                }
-            }
-        }
-        if constexpr (OV == 2) {
-            // fold the round into the pixel values (registers or `out`)
-            __syncthreads();
-            const double scale = ldexp((double)max_val, -F);
-            bool has;
-            if (PREF && full) {
-                // all LDS reads first (4 pixels and their zero bits per read),
-                // then branch-free updates
-                const float zero = (float)max_val * 0.0f;
-                const float p2 = __int_as_float((127 - F) << 23);   // 2^-F, F <= 31
-                uint4 acc[PV];
-                uint32_t zw[PV];
-#pragma unroll
-                for (int j = 0; j < PV; j++) {
-                    const int i = (tid + j * NT) * V;
-                    const int li = (i / TILE) * PITCH + (i % TILE);
-                    acc[j] = *reinterpret_cast<const uint4 *>(&img[li]);
-                    zw[j] = zb[li >> 5] >> (li & 31);
-                }
-#pragma unroll
-                for (int j = 0; j < PV; j++) {
-                    pre[j].x = fold_fix(pre[j].x, acc[j].x, zw[j] & 1u, p2, (float)max_val, zero);
-                    pre[j].y = fold_fix(pre[j].y, acc[j].y, zw[j] & 2u, p2, (float)max_val, zero);
-                    pre[j].z = fold_fix(pre[j].z, acc[j].z, zw[j] & 4u, p2, (float)max_val, zero);
-                    pre[j].w = fold_fix(pre[j].w, acc[j].w, zw[j] & 8u, p2, (float)max_val, zero);
-                }
-            } else {
-                for (int i = tid; i < TILE * TILE; i += NT) {
-                    const int y = Y0 + i / TILE, x = X0 + (i % TILE);
-                    if (y >= Y1 || x >= X1) continue;
-                    const int li = (i / TILE) * PITCH + (i % TILE);
-                    const double add = fix_value(img[li], zb, li, scale, (float)max_val, has);
-                    T *o = fo + (int64_t)y * g.W + x;
-                    if (has) *o = (T)((double)*o + add);
-                }
-            }
-        }
-    }
-    if constexpr (OV == 2) {
-        if (PREF && full) {
-#pragma unroll
-            for (int j = 0; j < PV; j++) {
-                const int i = (tid + j * NT) * V;
-                const int y = Y0 + i / TILE, x = X0 + (i % TILE);
-                if (y < Y1) {
-                    // written once per draw: non-temporal
-                    const v4f q = {pre[j].x, pre[j].y, pre[j].z, pre[j].w};
-                    __builtin_nontemporal_store(q, reinterpret_cast<v4f *>(fo + (int64_t)y * g.W + x));
-                }
-            }
-        }
-        return;
-    }
-    __syncthreads();
-
-    // flush: one coalesced read-modify-write of the tile, 4 pixels per access
-    // where the tile row lies inside the frame
-    if constexpr (PREF) {
-        if (full) {
-#pragma unroll
-            for (int j = 0; j < PV; j++) {
-                const int i = (tid + j * NT) * V;
-                const int y = Y0 + i / TILE, x = X0 + (i % TILE);
-                if (y >= Y1) continue;
-                const int li = (i / TILE) * PITCH + (i % TILE);
-                float4 ov = pre[j];
-                ov.x = (float)((double)ov.x + img[li]);
-                ov.y = (float)((double)ov.y + img[li + 1]);
-                ov.z = (float)((double)ov.z + img[li + 2]);
-                ov.w = (float)((double)ov.w + img[li + 3]);
-                *reinterpret_cast<float4 *>(fo + (int64_t)y * g.W + x) = ov;
-            }
-            return;
-        }
-    }
-    for (int i = tid * V; i < TILE * TILE; i += NT * V) {
-        const int y = Y0 + i / TILE, x = X0 + (i % TILE);
-        if (y >= Y1) continue;
-        T *o = fo + (int64_t)y * g.W + x;
-        const int li = (i / TILE) * PITCH + (i % TILE);
-        if (full) {
-            if constexpr (OV == 0) {
-                if constexpr (sizeof(T) == 4) {
-                    float4 ov = *reinterpret_cast<float4 *>(o);
-                    ov.x = (float)((double)ov.x + img[li]);
-                    ov.y = (float)((double)ov.y + img[li + 1]);
-                    ov.z = (float)((double)ov.z + img[li + 2]);
-                    ov.w = (float)((double)ov.w + img[li + 3]);
-                    *reinterpret_cast<float4 *>(o) = ov;
-                } else {
-                    for (int j = 0; j < V; j++) o[j] = o[j] + img[li + j];
-                }
-            } else {
-                for (int j = 0; j < V; j++) {
-                    const Acc e = img[li + j];
-                    if (e != Acc(0)) {
-                        const T m = ord_dec(e);
-                        const T ov = o[j];
-                        o[j] = (ov < m) ? m : ov; // std::max(out, value)
-                    }
-                }
-            }
-        } else {
-            for (int j = 0; j < V; j++) {
-                if (x + j >= X1) break;
-                if constexpr (OV == 0) {
-                    o[j] = (T)((double)o[j] + img[li + j]);
-                } else {
-                    const Acc e = img[li + j];
-                    if (e != Acc(0)) {
-                        const T m = ord_dec(e);
-                        const T ov = o[j];
-                        o[j] = (ov < m) ? m : ov;
-                    }
-                }
-            }
-        }
     }
 }
 
@@ -1531,6 +948,15 @@ __device__ __forceinline__ void pixel_grad(const GradConst &C, int x, int y, dou
     acc[4] = __builtin_fma(gw, C.cw, acc[4]);
 }
 
+// LDS row pitch of the adjoint's gradient tile, in words: 4 words of padding
+// per row.  The lanes of one item read the same short-axis coordinate in 8 or
+// 16 consecutive rows (steep lines); with a pitch of TILE (a multiple of the
+// bank count) those reads fall in one bank, with TILE + 4 in distinct banks.
+// (The tile kernel keeps a pitch of TILE: its padded variants measured slower,
+// see k_tiles.)
+template <int TILE>
+constexpr int tile_pitch() { return TILE + 4; }
+
 // The fills of one column for the float fast path (both halves and the
 // centre), with the forward's band test and inclusion decisions (err_fast);
 // lines with L.safe only.
@@ -1714,20 +1140,6 @@ k_line_grad(const int64_t *__restrict__ line_base, const LineSetup<T> *__restric
 // ---------------------------------------------------------------------------
 // host pipeline
 // ---------------------------------------------------------------------------
-template <typename T>
-struct SegmentPlan {
-    Geometry g;
-    int64_t n_lines = 0;
-    int64_t n_segs = 0;
-    int64_t n_items = 0;
-    int64_t n_tiles = 0;
-    DevBuf<LineSetup<T>> setup;
-    DevBuf<int> seg_cnt, seg_off, tile_cnt, tile_off, tile_cur, items, flags;
-    DevBuf<int2> pairs; // unordered plan: per-tile (segment, line) lists
-    DevBuf<int> slot_tiles; // unordered plan, when asked for: tiles per segment slot (the adjoint's)
-    DevBuf<Segment<T>> segs;
-};
-
 static int check_common(int64_t n_frames, int64_t H, int64_t W, int64_t n_lines, bool have_idxs, int kernel,
                         int overlap)
 {
@@ -1765,10 +1177,7 @@ static int build_plan(SegmentPlan<T> &P, const T *lines, const I *idxs, int kern
     g.n_frames = n_frames;
     g.H = (int32_t)H;
     g.W = (int32_t)W;
-    g.tile = tile;
-    g.seg = seg;
-    g.ntx = (int32_t)((W + tile - 1) / tile);
-    g.nty = (int32_t)((H + tile - 1) / tile);
+    set_tiles(g, tile, seg);
     P.n_lines = n_lines;
     P.n_tiles = bin ? n_frames * g.ntx * g.nty : 0;
     if (P.n_tiles >= (int64_t(1) << 31)) return fail(CBX_EVALUE, "too many tiles");
@@ -1852,10 +1261,7 @@ static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs
     g.n_frames = n_frames;
     g.H = (int32_t)H;
     g.W = (int32_t)W;
-    g.tile = tile;
-    g.seg = seg;
-    g.ntx = (int32_t)((W + tile - 1) / tile);
-    g.nty = (int32_t)((H + tile - 1) / tile);
+    set_tiles(g, tile, seg);
     P.n_lines = n_lines;
     P.n_tiles = n_frames * g.ntx * g.nty;
     if (P.n_tiles >= (int64_t(1) << 31) / LIST_SUBS) return fail(CBX_EVALUE, "too many tiles");
@@ -1863,6 +1269,7 @@ static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs
 
     DevBuf<unsigned long long> counters;
     CBX_HIP(P.setup.alloc(n_lines, st));
+    if (sizeof(T) == 4) CBX_HIP(P.lite.alloc(n_lines, st));
     CBX_HIP(P.flags.alloc(1, st));
     CBX_HIP(counters.alloc(2, st));
     CBX_HIP(P.tile_cnt.alloc(n_lists, st));
@@ -1876,7 +1283,7 @@ static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs
     }
     const int blk = 256;
     k_setup_lines<T, I><<<grid_for(n_lines, blk), blk, 0, st>>>(lines, idxs, kernels, kernel, n_lines, g,
-                                                               P.setup.ptr, counters.ptr, P.flags.ptr);
+                                                               P.setup.ptr, P.lite.ptr, counters.ptr, P.flags.ptr);
     CBX_HIP(hipGetLastError());
     uint64_t hv[3];
     int fl = 0, rc = 0;
@@ -1959,56 +1366,6 @@ static int check_opts(int tile, int seg)
     if (!(tile == 32 || tile == 64)) return fail(CBX_EVALUE, "tile must be 32 or 64");
     if (!(seg == 8 || seg == 16)) return fail(CBX_EVALUE, "seg must be 8 or 16");
     return CBX_OK;
-}
-
-template <typename T, int K, int OV, int TILE, int SEG>
-static void launch_tiles(T *out, const SegmentPlan<T> &P, T max_val, int threads, int chunk, bool fast,
-                         hipStream_t st)
-{
-#define CBX_TILES(NT, CH, FST)                                                                                  \
-    k_tiles<T, K, OV, TILE, SEG, NT, CH, FST><<<(unsigned)P.n_tiles, NT, 0, st>>>(                             \
-        out, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, max_val, P.flags.ptr)
-    if constexpr (OV == 2) {
-        if (threads == 64) CBX_TILES(64, 64, true);
-        else if (threads == 128) CBX_TILES(128, 64, true);
-        else if (chunk == 64) CBX_TILES(256, 64, true);
-        else CBX_TILES(256, 256, true);
-    } else if (fast) {
-        if (threads == 64) CBX_TILES(64, 64, true);
-        else if (threads == 128) CBX_TILES(128, 64, true);
-        else if (chunk == 64) CBX_TILES(256, 64, true);
-        else CBX_TILES(256, 256, true);
-    } else {
-        if (threads == 64) CBX_TILES(64, 64, false);
-        else if (threads == 128) CBX_TILES(128, 64, false);
-        else if (chunk == 64) CBX_TILES(256, 64, false);
-        else CBX_TILES(256, 256, false);
-    }
-#undef CBX_TILES
-}
-
-template <typename T, int K, int OV>
-static void launch_tiles_k(T *out, const SegmentPlan<T> &P, T max_val, int threads, int chunk, bool fast,
-                           hipStream_t st)
-{
-    if (P.g.tile == 64 && P.g.seg == 16) launch_tiles<T, K, OV, 64, 16>(out, P, max_val, threads, chunk, fast, st);
-    else if (P.g.tile == 64) launch_tiles<T, K, OV, 64, 8>(out, P, max_val, threads, chunk, fast, st);
-    else if (P.g.seg == 16) launch_tiles<T, K, OV, 32, 16>(out, P, max_val, threads, chunk, fast, st);
-    else launch_tiles<T, K, OV, 32, 8>(out, P, max_val, threads, chunk, fast, st);
-}
-
-template <typename T, int OV>
-static void launch_tiles_ov(int kernel, T *out, const SegmentPlan<T> &P, T max_val, int threads, int chunk,
-                            bool fast, hipStream_t st)
-{
-    switch (kernel) {
-    case K_BIWEIGHT: launch_tiles_k<T, K_BIWEIGHT, OV>(out, P, max_val, threads, chunk, fast, st); break;
-    case K_GAUSSIAN: launch_tiles_k<T, K_GAUSSIAN, OV>(out, P, max_val, threads, chunk, fast, st); break;
-    case K_PARABOLIC: launch_tiles_k<T, K_PARABOLIC, OV>(out, P, max_val, threads, chunk, fast, st); break;
-    case K_RECTANGULAR: launch_tiles_k<T, K_RECTANGULAR, OV>(out, P, max_val, threads, chunk, fast, st); break;
-    case K_TRIANGULAR: launch_tiles_k<T, K_TRIANGULAR, OV>(out, P, max_val, threads, chunk, fast, st); break;
-    default: launch_tiles_k<T, K_MIXED, OV>(out, P, max_val, threads, chunk, fast, st); break;
-    }
 }
 
 template <typename T, bool WRITE>
@@ -2177,19 +1534,14 @@ template <typename T>
 static void run_tiles(T *out, const SegmentPlan<T> &P, int kernel, int overlap, T max_val, const cbx_draw_opts *opts,
                       hipStream_t st)
 {
-    const int threads = (opts && opts->threads) ? opts->threads : 256;
-    const bool fast = !(opts && opts->exact_values);
-    const int chunk = (opts && opts->chunk) ? opts->chunk : 64;
-    // float sums on the fast path accumulate in fixed point, unless max_val
-    // is not finite (inf * 0 must stay NaN, as in the reference)
-    if constexpr (sizeof(T) == 4) {
-        if (overlap == 0 && fast && std::isfinite(max_val)) {
-            launch_tiles_ov<T, 2>(kernel, out, P, max_val, threads, chunk, fast, st);
-            return;
-        }
+    switch (kernel) {
+    case K_BIWEIGHT: run_tiles_profile<T, K_BIWEIGHT>(out, P, max_val, overlap, opts, st); break;
+    case K_GAUSSIAN: run_tiles_profile<T, K_GAUSSIAN>(out, P, max_val, overlap, opts, st); break;
+    case K_PARABOLIC: run_tiles_profile<T, K_PARABOLIC>(out, P, max_val, overlap, opts, st); break;
+    case K_RECTANGULAR: run_tiles_profile<T, K_RECTANGULAR>(out, P, max_val, overlap, opts, st); break;
+    case K_TRIANGULAR: run_tiles_profile<T, K_TRIANGULAR>(out, P, max_val, overlap, opts, st); break;
+    default: run_tiles_profile<T, K_MIXED>(out, P, max_val, overlap, opts, st); break;
     }
-    if (overlap == 0) launch_tiles_ov<T, 0>(kernel, out, P, max_val, threads, chunk, fast, st);
-    else launch_tiles_ov<T, 1>(kernel, out, P, max_val, threads, chunk, fast, st);
 }
 
 template <typename T, typename I>
@@ -2589,10 +1941,7 @@ static int plan_create(cbx_plan **out_plan, int64_t n_frames, int64_t H, int64_t
     g.n_frames = n_frames;
     g.H = (int32_t)H;
     g.W = (int32_t)W;
-    g.tile = tile;
-    g.seg = seg;
-    g.ntx = (int32_t)((W + tile - 1) / tile);
-    g.nty = (int32_t)((H + tile - 1) / tile);
+    set_tiles(g, tile, seg);
     P.n_lines = n_lines;
     P.n_tiles = n_frames * g.ntx * g.nty;
     const int64_t n_lists = P.n_tiles * LIST_SUBS;
@@ -2609,6 +1958,7 @@ static int plan_create(cbx_plan **out_plan, int64_t n_frames, int64_t H, int64_t
     };
     // owned allocations (no workspace is open here)
     take(P.setup.alloc(n_lines, st));
+    take(P.lite.alloc(n_lines, st));
     take(P.flags.alloc(1, st));
     take(P.segs.alloc(slot_cap, st));
     take(P.slot_tiles.alloc(slot_cap, st));
@@ -2625,7 +1975,7 @@ static int plan_create(cbx_plan **out_plan, int64_t n_frames, int64_t H, int64_t
         delete pl;
         return fail(CBX_ERUNTIME, std::string("plan allocation: ") + hipGetErrorString(e));
     }
-    pl->bytes = (int64_t)((sizeof(LineSetup<float>) + sizeof(int64_t)) * n_lines +
+    pl->bytes = (int64_t)((sizeof(LineSetup<float>) + sizeof(LineLite) + sizeof(int64_t)) * n_lines +
                           (sizeof(Segment<float>) + sizeof(int)) * slot_cap +
                           sizeof(int2) * item_cap + 3 * sizeof(int) * n_lists + sizeof(int) +
                           sizeof(unsigned long long) * scan_words);
@@ -2650,7 +2000,8 @@ static int plan_draw(cbx_plan *pl, float *out, const float *lines, int64_t n_lin
                                                          P.tile_cur.ptr, pl->scan_state.ptr,
                                                          (int64_t)pl->scan_state.n);
     k_setup_lines<float, int32_t><<<grid_for(n_lines, blk), blk, 0, st>>>(lines, idxs, kernels, kernel, n_lines, g,
-                                                                         P.setup.ptr, pl->counters.ptr, P.flags.ptr);
+                                                                         P.setup.ptr, P.lite.ptr, pl->counters.ptr,
+                                                                         P.flags.ptr);
     k_walk_lines<float><<<grid_for(n_lines, blk), blk, 0, st>>>(n_lines, g, P.setup.ptr, P.segs.ptr, P.n_segs,
                                                                 pl->counters.ptr, P.tile_cnt.ptr, P.flags.ptr,
                                                                 pl->line_base.ptr);

@@ -1,0 +1,198 @@
+// Types of the 2D draw pipeline shared by its translation units: segments,
+// line records, the plan of a draw, the walk replay and the column fills.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <climits>
+
+#include "cbx_core.hpp"
+#include "cbx_host.hpp"
+
+namespace cbx {
+
+template <typename T>
+struct Segment {
+    int32_t line;
+    int32_t c[2];   // walk position at the segment's first column
+    int32_t ncols;  // emitted long-axis columns, consecutive from c[axis] in the walk direction
+    T Te, Ne;       // walk errors at that position
+    int32_t lo, hi; // short-axis pixel range the fills can reach, clipped to the frame
+};
+
+// What the float tile kernel needs of a line (32 bytes, two 16-byte loads; the
+// whole LineSetup is read only for exact errors next to the threshold and for
+// the lines that are not FR_SAFE).
+struct alignas(16) LineLite {
+    float t[2];       // tangent (the normal components are t[1], -t[0])
+    float LL, ea;     // as in LineSetup
+    float nlim;       // band limit
+    float cap;        // a column with cap < Te < LL - cap has no tangential overshoot at any of its pixels
+    int32_t meta;     // FR_* bits, profile id in bits 8-15
+    int32_t pad;
+};
+constexpr int FR_AXIS = 1, FR_SA = 2, FR_SB = 4, FR_SAFE = 8;
+
+struct Geometry {
+    int64_t n_frames;
+    int32_t H, W;
+    int32_t tile, seg;
+    int32_t ntx, nty;
+    uint32_t m_frame = 0, m_ntx = 0;   // tile_coords: 2^32 / (tiles per frame), 2^32 / ntx, rounded down
+    int32_t skip_neg = 0;   // 1: a line with a negative frame draws nothing (accumulate_lines term batches)
+};
+
+// The unordered plan's item list of tile t is split into LIST_SUBS sub-lists
+// by the binning wave (slot / 64 mod LIST_SUBS), so that the cursor atomics
+// of a dense tile spread over LIST_SUBS counters; the sub-lists are
+// contiguous: tile t's items are [tile_off[t * LIST_SUBS],
+// tile_off[(t + 1) * LIST_SUBS]).
+constexpr int LIST_SUBS = 8;
+
+// n / d (remainder in r) from m = floor(2^32 / d) (2^32 - 1 for d = 1): the product
+// is at most one too small.  Scalar instructions for a uniform n, where the
+// compiler's integer division takes about 20 vector ones.
+__host__ __device__ __forceinline__ uint32_t div_magic(uint32_t d)
+{
+    return d <= 1 ? 0xffffffffu : (uint32_t)((uint64_t(1) << 32) / d);
+}
+__device__ __forceinline__ int div_by(int n, int d, uint32_t m, int &r)
+{
+    int q = (int)__umulhi((uint32_t)n, m);
+    r = n - q * d;
+    if (r >= d) {
+        q++;
+        r -= d;
+    }
+    return q;
+}
+
+// frame and tile column / row of a tile index
+__device__ __forceinline__ void tile_coords(const Geometry &g, int tile, int64_t &f, int &tx, int &ty)
+{
+    int r;
+    f = div_by(tile, g.ntx * g.nty, g.m_frame, r);
+    ty = div_by(r, g.ntx, g.m_ntx, tx);
+}
+
+inline void set_tiles(Geometry &g, int tile, int seg)
+{
+    g.tile = tile;
+    g.seg = seg;
+    g.ntx = (int32_t)((g.W + tile - 1) / tile);
+    g.nty = (int32_t)((g.H + tile - 1) / tile);
+    g.m_frame = div_magic((uint32_t)((int64_t)g.ntx * g.nty));
+    g.m_ntx = div_magic((uint32_t)g.ntx);
+}
+
+__device__ __forceinline__ int64_t list_index(int64_t tile, int64_t slot)
+{
+    return tile * LIST_SUBS + ((slot >> 6) & (LIST_SUBS - 1));
+}
+
+// ---------------------------------------------------------------------------
+// shared pieces of the tile kernels
+// ---------------------------------------------------------------------------
+template <typename T>
+struct ColRec {
+    int32_t s; // short-axis centre, INT_MIN when the column is not emitted
+    T Te, Ne;
+};
+
+struct ItemHdr {
+    int32_t seg;
+    int32_t line;
+};
+
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Phase 1: replay a segment's walk from its checkpoint and record, for each
+// of its columns, the centre and errors at which the reference emits it, in
+// the column slots i * SEG + k of item i of rr.
+template <typename T, int SEG>
+__device__ __forceinline__ void walk_columns(const LineSetup<T> &L, const Segment<T> &sg, ColRec<T> *rr, int i,
+                                             int *flags)
+{
+    for (int k = 0; k < SEG; k++) rr[i * SEG + k].s = INT_MIN;
+    const int a = L.axis, b = 1 - a, sa = pick(L.st, a);
+    WalkState<T> s;
+    s.c[0] = sg.c[0];
+    s.c[1] = sg.c[1];
+    s.Te = sg.Te;
+    s.Ne = sg.Ne;
+    const int c0 = pick(s.c, a);
+    int it = 0;
+    for (; it < 4 * SEG + 16; it++) {
+        if (walk_done(L, s)) break;
+        const int k = (pick(s.c, a) - c0) * sa;
+        if (k >= sg.ncols) break;
+        bool nx, ny;
+        walk_next(L, s.Ne, nx, ny);
+        if ((a == 0) ? nx : ny) {
+            ColRec<T> &r = rr[i * SEG + k];
+            r.s = pick(s.c, b);
+            r.Te = s.Te;
+            r.Ne = s.Ne;
+        }
+        walk_step(L, s, nx, ny);
+    }
+    if (it == 4 * SEG + 16) atomicOr(flags, FLAG_STUCK);
+}
+
+// Phase 2: the orthogonal fills of one emitted column (bresenham.hpp:364-380),
+// restricted to the short-axis window [s_lo, s_hi); emit(s, err) is called
+// for every pixel of the window the reference would hand to draw_pixel.
+template <typename T, typename Emit>
+__device__ __forceinline__ void fill_column(const LineSetup<T> &L, const ColRec<T> &cr, int s_lo, int s_hi,
+                                            Emit &&emit)
+{
+    const int b = 1 - L.axis;
+    if (cr.s >= s_lo && cr.s < s_hi) emit(cr.s, cr.Te, cr.Ne);
+    const T tb = pick(L.t, b), nb = pick(L.nv, b);
+    const int sb = pick(L.st, b);
+#pragma unroll
+    for (int half = 0; half < 2; half++) {
+        const int dir = half ? -sb : sb;
+        const T dT = (dir > 0) ? tb : -tb, dN = (dir > 0) ? nb : -nb;
+        int s = cr.s;
+        T Te = cr.Te, Ne = cr.Ne;
+        for (;;) {
+            s += dir;
+            Te += dT;
+            Ne += dN;
+            if (!(nsq_of(L, Ne) < L.w2)) break;
+            if (s >= s_lo && s < s_hi) emit(s, Te, Ne);
+            else if ((dir > 0) ? (s >= s_hi) : (s < s_lo)) break;
+        }
+    }
+}
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+template <typename T>
+struct SegmentPlan {
+    Geometry g;
+    int64_t n_lines = 0;
+    int64_t n_segs = 0;
+    int64_t n_items = 0;
+    int64_t n_tiles = 0;
+    DevBuf<LineSetup<T>> setup;
+    DevBuf<LineLite> lite;   // unordered float plan
+    DevBuf<int> seg_cnt, seg_off, tile_cnt, tile_off, tile_cur, items, flags;
+    DevBuf<int2> pairs; // unordered plan: per-tile (segment, line) lists
+    DevBuf<int> slot_tiles; // unordered plan, when asked for: tiles per segment slot (the adjoint's)
+    DevBuf<Segment<T>> segs;
+};
+
+// The tile kernel of one profile (CBX_PROFILE of cbx_tiles.hip; K_MIXED: per-line
+// profiles) over a built unordered plan.
+template <typename T, int K>
+void run_tiles_profile(T *out, const SegmentPlan<T> &P, T max_val, int overlap, const cbx_draw_opts *opts,
+                       hipStream_t st);
+
+} // namespace cbx
