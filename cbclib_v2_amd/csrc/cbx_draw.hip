@@ -110,134 +110,114 @@ __device__ __forceinline__ int segment_bound(const LineSetup<T> &L, const Geomet
     const int a = L.axis, da = (a == 0) ? g.W : g.H;
     const int c0 = pick(L.m0, a), c1 = pick(L.m1, a);
     const int lo = max(min(c0, c1), 0), hi = min(max(c0, c1), da - 1);
-    return (lo > hi) ? 0 : hi / g.seg - lo / g.seg + 1;
+    return (lo > hi) ? 0 : (hi >> g.seg_log) - (lo >> g.seg_log) + 1;
+}
+
+// Short-axis pixels from a column's centre that its fills can reach.  A fill of
+// j steps has |N_j| >= j |t_a| - |N_0| and stops once |N| / len >= w; at an emitted
+// column |N_0| <= max(|N at m0|, |t_a| / 2): every step takes the candidate of
+// smallest |N|, and one of them moves N against its sign by at most |t_a|.
+// (2^-23 per step: the rounding of the fill's running sums.)
+template <typename T>
+__device__ __forceinline__ int fill_reach(const LineSetup<T> &L)
+{
+    const double ta = (double)m_abs(pick(L.t, L.axis));
+    const double n0 = (double)m_abs(L.e0[1]), half = 0.50001 * ta;
+    const double j = ((double)L.w * (double)L.len + (n0 > half ? n0 : half)) / ta;
+    const double r = j * (1.00001 + 1.2e-7 * j) + 1.0;
+    return r < 1073741824.0 ? (int)r : 1073741824;   // 2^30: added to a coordinate (below 1e9) it stays an int
 }
 
 // Replays line l's walk (bresenham.hpp:352-383) and cuts it into segments of
 // <= SEG long-axis columns inside the frame.  For each segment whose fills
 // can reach the frame, on_seg(cur, tl) gets the checkpoint (with the reach
 // range lo..hi set) and the tile column tl along the long axis.
+//
+// The steps are a serial chain (each FP32 sum rounds), so the time of a draw of
+// few lines is the instructions of one step times the longest line, and the
+// loop holds little else: the next |N| is one of the three candidates, both
+// coordinates move by selects, one test ends the block.  Emission needs no bookkeeping: every long-axis
+// step emits the column it leaves, so a block's emitted columns are its first
+// ones, their centres lie between the block's first and last short-axis
+// positions and their errors below a bound of the whole line (fill_reach).
+// 19 vector instructions per step: the walk of 1000 lines of up to 720 px takes
+// 71 us (131 with the bookkeeping in the step and a store ring), of 128 000
+// lines of up to 400 px 86 us (126).
 template <typename T, typename OnSeg>
 __device__ __forceinline__ void walk_segments(const LineSetup<T> &L, int64_t l, const Geometry &g,
                                               int *__restrict__ flags, OnSeg on_seg)
 {
     const int a = L.axis, b = 1 - a;
-    const bool ax0 = a == 0;
-    const int da = (a == 0) ? g.W : g.H, db = (a == 0) ? g.H : g.W;
-    const int sa = pick(L.st, a);
-    const double ta = (double)m_abs(pick(L.t, a));
-    const double wl = (double)L.w * (double)L.len;
+    const bool ax = a == 1;
+    const int da = ax ? g.H : g.W, db = ax ? g.W : g.H;
+    const int sa = pick(L.st, a), sb = pick(L.st, b);
+    const int R = fill_reach(L);
+    // signed increments along x and y
+    const T dx = (L.st[0] > 0) ? L.nv[0] : -L.nv[0], dy = (L.st[1] > 0) ? L.nv[1] : -L.nv[1];
+    const T ux = (L.st[0] > 0) ? L.t[0] : -L.t[0], uy = (L.st[1] > 0) ? L.t[1] : -L.t[1];
+    T Te = L.e0[0], Ne = L.e0[1];
+    int c = pick(L.m0, a), s = pick(L.m0, b);
+    int left = (pick(L.m1, a) - c) * sa, side = (pick(L.m1, b) - s) * sb;   // steps to the walk's end along each axis
+    wait_vm_loads();
 
-    WalkState<T> s;
-    s.c[0] = L.m0[0];
-    s.c[1] = L.m0[1];
-    s.Te = L.e0[0];
-    s.Ne = L.e0[1];
-
-    int b_lo = 0, b_hi = 0, tl = 0, nem = 0, smin = 0, smax = 0;
-    T maxN = T(0);   // the largest |N| at an emitted column (exact in T)
-    Segment<T> cur;
-
-    auto close = [&]() {
-        if (nem == 0) return;
-        // fills stop once |N| / len >= w; |N| grows by |t_a| per short step
-        int R = (int)((wl + (double)maxN) / ta) + 2;
-        int lo = max(smin - R, 0), hi = min(smax + R, db - 1);
-        if (lo > hi) return;
-        cur.lo = lo;
-        cur.hi = hi;
-        // every long-axis step emits the column it leaves: the emitted columns
-        // are the block's first nem
-        cur.ncols = nem;
-        on_seg(cur, tl);
+    // steps until k (> 0) long-axis steps are done or `side` (> 0) short-axis
+    // steps are left no more; returns the long-axis steps left.  Every step moves
+    // along one of the axes at least, so the loop ends.
+    auto advance = [&](int k) {
+        bool go;
+        do {
+            const T ex = Ne + dx, ey = Ne + dy, exy = ex + dy;
+            const bool yb = m_abs(ey) < m_abs(ex);
+            const T m = yb ? ey : ex;
+            const bool both = m_abs(exy) < m_abs(m);
+            Te += (both | !yb) ? ux : T(0);
+            Te += (both | yb) ? uy : T(0);
+            Ne = both ? exy : m;
+            side -= (both | (yb != ax)) ? 1 : 0;
+            k -= (both | (yb == ax)) ? 1 : 0;
+            go = (k != 0) & (side != 0);
+        } while (go);
+        return k;
     };
 
-    // every step moves the walk; a walk takes at most one short-axis-only
-    // step per long-axis step, so this budget is never reached by a valid line
-    const int64_t budget = 4 * ((int64_t)abs(pick(L.m1, a) - pick(L.m0, a)) + abs(pick(L.m1, b) - pick(L.m0, b))) + 64;
-    // Loop structure: an outer loop over segments and an inner loop over the
-    // steps of one SEG-column block, so that the lanes of a wave close their
-    // segments together (a close inside the step loop would run, with a few
-    // lanes active, on almost every step).  The steps and decisions are those
-    // of one plain loop over the walk.
-    wait_vm_loads();
-    int64_t it = 0;
-    bool stop = false;
     // columns before the frame (the walk is monotone along the long axis)
-    for (;; it++) {
-        if (it == budget) {
-            atomicOr(flags, FLAG_STUCK);
-            stop = true;
-            break;
+    {
+        const int k0 = min(max(0, (sa > 0) ? -c : c - (da - 1)), left);
+        if (k0 > 0) {
+            const int q = side;
+            const int k = advance(k0);
+            c += sa * k0;
+            s += sb * (q - side);
+            left = (k != 0) ? 0 : left - k0;
         }
-        if (walk_done(L, s)) {
-            stop = true;
-            break;
-        }
-        const int c = pick(s.c, a);
-        if ((sa > 0) ? (c >= da) : (c < 0)) { // no in-frame column is left
-            stop = true;
-            break;
-        }
-        if (c >= 0 && c < da) break; // the first segment starts here
-        bool nx, ny;
-        walk_next(L, s.Ne, nx, ny);
-        walk_step(L, s, nx, ny);
     }
-    while (!stop) {
-        // open a segment at the current (in-frame) column
-        const int c0 = pick(s.c, a);
-        b_lo = (c0 / g.seg) * g.seg;
-        b_hi = min(b_lo + g.seg, da);
-        tl = c0 / g.tile;
-        nem = 0;
-        maxN = T(0);
-        smin = INT_MAX;
-        smax = INT_MIN;
-        cur.line = (int32_t)l;
-        cur.c[0] = s.c[0];
-        cur.c[1] = s.c[1];
-        cur.Te = s.Te;
-        cur.Ne = s.Ne;
-        // One exit test per step: the long-axis coordinate moves by 0 or sa
-        // per step and starts inside the block [b_lo, b_hi), which lies
-        // inside the frame, so the block (and the frame) is left exactly at
-        // c_end.  Steps are counted per block in 32 bits (at most two per
-        // column for a valid walk: kmax is never reached) and added to the
-        // walk's budget after it.  Why the block ended is sorted out after
-        // the loop, in the order the checks have in a plain loop: the step
-        // budget, the end of the walk, the frame edge, else the next block.
-        // Branch-free updates keep the step short.
-        const int c_end = (sa > 0) ? b_hi : b_lo - 1;
-        const int kmax = 4 * g.seg + 8;
-        int k = 0;
-        for (;; k++) {
-            if ((k == kmax) | (pick(s.c, a) == c_end) | walk_done(L, s)) break;
-            bool nx, ny;
-            walk_next(L, s.Ne, nx, ny);
-            // (lane masks combined with the loop-invariant axis mask; a NaN
-            // |N| leaves maxN, as fmax would)
-            const bool em = (nx && ax0) || (ny && !ax0);
-            const int sb = pick(s.c, b);
-            const T an = m_abs(s.Ne);
-            nem += em ? 1 : 0;
-            smin = em ? min(smin, sb) : smin;
-            smax = em ? max(smax, sb) : smax;
-            maxN = (em && an > maxN) ? an : maxN;
-            walk_step(L, s, nx, ny);
-        }
-        it += k;
-        if (k == kmax || it >= budget) {
-            atomicOr(flags, FLAG_STUCK);
-            stop = true;
-        } else if (walk_done(L, s)) {
-            stop = true;
-        } else {
-            const int c = pick(s.c, a);
-            if ((sa > 0) ? (c >= da) : (c < 0)) stop = true;
-        }
-        close();
+    left = (side > 0) ? min(left, (sa > 0) ? da - c : c + 1) : 0;   // columns inside the frame
+    const int seg = g.seg;
+    int most = 0;
+    Segment<T> cur;
+    cur.line = (int32_t)l;
+    while (left > 0) {
+        // a segment from the current column to the end of its block of SEG
+        const int in = c & (seg - 1);
+        const int k0 = min((sa > 0) ? seg - in : in + 1, left);
+        const int s0 = s, q = side, tl = c >> g.tile_log;
+        cur.c[0] = ax ? s : c;
+        cur.c[1] = ax ? c : s;
+        cur.Te = Te;
+        cur.Ne = Ne;
+        const int k = advance(k0);
+        most = max(most, q - side);
+        s += sb * (q - side);
+        c += sa * k0;
+        left = (side > 0) ? left - k0 : 0;
+        cur.ncols = k0 - k;
+        cur.lo = max(min(s0, s) - R, 0);
+        cur.hi = min(max(s0, s) + R, db - 1);
+        if ((cur.ncols > 0) & (cur.lo <= cur.hi)) on_seg(cur, tl);
     }
+    // (the tile kernels' replay stops after 4 SEG + 16 steps; a walk takes at
+    // most about two per column)
+    if (most > 3 * seg + 8) atomicOr(flags, FLAG_STUCK);
 }
 
 __device__ __forceinline__ int64_t tile_index(const Geometry &g, int frame, int axis, int tl, int tb)
@@ -277,7 +257,7 @@ k_segments(const T *__restrict__ lines, const I *__restrict__ idxs, int kernel, 
         const int sid = base + nseg;
         if (WRITE) segs[sid] = cur;
         if (BIN) {
-            for (int tb = cur.lo / g.tile; tb <= cur.hi / g.tile; tb++) {
+            for (int tb = cur.lo >> g.tile_log; tb <= cur.hi >> g.tile_log; tb++) {
                 const int64_t tid = tile_index(g, L.frame, L.axis, tl, tb);
                 if (!WRITE) atomicAdd(&tile_cnt[tid], 1);
                 else items[tile_off[tid] + atomicAdd(&tile_cur[tid], 1)] = sid;
@@ -324,11 +304,6 @@ k_setup_lines(const T *__restrict__ lines, const I *__restrict__ idxs, const uin
     __syncthreads();
     if (threadIdx.x == 0 && bsum) atomicAdd(&counters[0], bsum);
 }
-
-// Records per thread in the walk's LDS ring: 2 (16 KB per 256 threads; a
-// ring of 4 gave no faster walk on 128k lines and fewer resident workgroups
-// on 972k lines).
-constexpr int WALK_RING = 2;
 
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -410,47 +385,20 @@ k_walk_lines(int64_t n_lines, Geometry g, const LineSetup<T> *__restrict__ setup
     if (ub == 0 || (int64_t)(wbase + total) > slot_cap) return;
     const int64_t base = (int64_t)wbase + pre;
     int nseg = 0;
-    // Segments go through a per-thread ring of WALK_RING records in LDS and
-    // are written to memory WALK_RING at a time, all loads before all
-    // stores: a store's data registers cannot be reused before the store
-    // completes, so writing each segment from registers at its close would
-    // stall every close on the previous store.  The tile counts are atomics
-    // whose results the walk does not use (k_bin_slots places the items);
-    // their rate bounds the walk, so each lane adds up runs of items into
-    // the same list (consecutive segments of a line mostly share their
-    // tiles) in two pending counters and issues one atomic per run.
-    // (ring words [slot][word][thread]: a record moves as 32-bit words with
-    // constant indices, so it stays in registers)
-    constexpr int NW = (int)(sizeof(Segment<T>) / 4);
-    static_assert(sizeof(Segment<T>) % 8 == 0, "records move as 64-bit pairs");
-    __shared__ uint32_t ring[WALK_RING][NW][256];
-    const int t = threadIdx.x;
-    auto flush = [&](int first, int cnt) {   // records first .. first + cnt - 1, ring slots 0 .. cnt - 1
-        uint32_t w[WALK_RING][NW];
-#pragma unroll
-        for (int j = 0; j < WALK_RING; j++)
-#pragma unroll
-            for (int k = 0; k < NW; k++)
-                if (j < cnt) w[j][k] = ring[j][k][t];
-#pragma unroll
-        for (int j = 0; j < WALK_RING; j++) {
-            if (j < cnt && first + j < ub) {
-                uint2 *dst = reinterpret_cast<uint2 *>(segs + base + first + j);
-#pragma unroll
-                for (int k = 0; k < NW / 2; k++) dst[k] = make_uint2(w[j][2 * k], w[j][2 * k + 1]);
-            }
-        }
-    };
+    // The tile counts are atomics whose results the walk does not use
+    // (k_bin_slots places the items); each lane adds up runs of items into
+    // the same list (consecutive segments of a line mostly share their tiles)
+    // in two pending counters and issues one atomic per run.
     int pend_a = -1, pend_b = -1, n_a = 0, n_b = 0;   // pending list counts (list index, items)
+    Segment<T> *const dst = segs + base;
+    // (axis 0: the long axis runs along tile columns)
+    const int fbase = L.frame * (g.nty * g.ntx), ml = (L.axis == 0) ? 1 : g.ntx, mb = (L.axis == 0) ? g.ntx : 1;
     walk_segments(L, l, g, flags, [&](const Segment<T> &cur, int tl) {
-        uint32_t cw[NW];
-        __builtin_memcpy(cw, &cur, sizeof(cw));
-        const int slot = nseg % WALK_RING;
-#pragma unroll
-        for (int k = 0; k < NW; k++) ring[slot][k][t] = cw[k];
-        const int tb0 = cur.lo / g.tile, tb1 = cur.hi / g.tile;
-        for (int tb = tb0; tb <= tb1; tb++) {
-            const int li = (int)list_index(tile_index(g, L.frame, L.axis, tl, tb), base + nseg);
+        if (nseg < ub) dst[nseg] = cur;
+        const int tb0 = cur.lo >> g.tile_log, tb1 = cur.hi >> g.tile_log;
+        const int sub = (int)(((uint32_t)base + (uint32_t)nseg) >> 6) & (LIST_SUBS - 1);
+        int li = (fbase + tl * ml + tb0 * mb) * LIST_SUBS + sub;
+        for (int tb = tb0; tb <= tb1; tb++, li += mb * LIST_SUBS) {
             if (li == pend_a) {
                 n_a++;
             } else if (li == pend_b) {
@@ -464,14 +412,9 @@ k_walk_lines(int64_t n_lines, Geometry g, const LineSetup<T> *__restrict__ setup
             }
         }
         nseg++;
-        if (nseg % WALK_RING == 0) flush(nseg - WALK_RING, WALK_RING);
     });
     if (n_a) atomicAdd(&tile_cnt[pend_a], n_a);
     if (n_b) atomicAdd(&tile_cnt[pend_b], n_b);
-    if (nseg % WALK_RING) {
-        const int done = (nseg / WALK_RING) * WALK_RING;   // records flushed at closes
-        flush(done, nseg - done);
-    }
     if (nseg > ub) atomicOr(flags, FLAG_STUCK); // cannot happen: the bound holds for every walk
     for (int k = nseg; k < ub; k++) segs[base + k].ncols = 0;
 }
@@ -523,9 +466,9 @@ k_bin_slots(int64_t n_slots, Geometry g, const LineSetup<T> *__restrict__ setup,
         if (sg.ncols > 0) {
             axis = setup[sg.line].axis;
             frame = setup[sg.line].frame;
-            tl = pick(sg.c, axis) / g.tile;
-            tb0 = sg.lo / g.tile;
-            np = sg.hi / g.tile - tb0 + 1;
+            tl = pick(sg.c, axis) >> g.tile_log;
+            tb0 = sg.lo >> g.tile_log;
+            np = (sg.hi >> g.tile_log) - tb0 + 1;
             item = make_int2((int)i, sg.line);
         }
     }
@@ -1089,7 +1032,7 @@ k_adjoint_tiles(const T *__restrict__ grad, const T *__restrict__ lines, Geometr
                 const Segment<T> &sg = segs[sid];
                 const int a = setup[hdr[wave][i].line].axis;
                 const int tb = (a == 0) ? ty : tx;
-                double *p = partial + 5 * (int64_t)(slot_base[sid] + (tb - sg.lo / g.tile));
+                double *p = partial + 5 * (int64_t)(slot_base[sid] + (tb - (sg.lo >> g.tile_log)));
 #pragma unroll
                 for (int j = 0; j < 5; j++) p[j] = acc[j];
             }

@@ -37,6 +37,7 @@ struct Geometry {
     int64_t n_frames;
     int32_t H, W;
     int32_t tile, seg;
+    int32_t tile_log, seg_log;
     int32_t ntx, nty;
     uint32_t m_frame = 0, m_ntx = 0;   // tile_coords: 2^32 / (tiles per frame), 2^32 / ntx, rounded down
     int32_t skip_neg = 0;   // 1: a line with a negative frame draws nothing (accumulate_lines term batches)
@@ -79,6 +80,8 @@ inline void set_tiles(Geometry &g, int tile, int seg)
 {
     g.tile = tile;
     g.seg = seg;
+    g.tile_log = (tile == 64) ? 6 : 5;
+    g.seg_log = (seg == 16) ? 4 : 3;
     g.ntx = (int32_t)((g.W + tile - 1) / tile);
     g.nty = (int32_t)((g.H + tile - 1) / tile);
     g.m_frame = div_magic((uint32_t)((int64_t)g.ntx * g.nty));
