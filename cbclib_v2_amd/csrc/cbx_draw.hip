@@ -96,7 +96,7 @@ __device__ __forceinline__ LineLite line_lite(const LineSetup<float> &L)
     r.cap = J * (m_abs(pick(L.t, b)) * 1.00001f + L.LL * 2.4e-7f);
     r.meta = a | (pick(L.st, a) > 0 ? FR_SA : 0) | (pick(L.st, b) > 0 ? FR_SB : 0) | (L.safe ? FR_SAFE : 0) |
              ((int)(uint8_t)L.kid << 8);
-    r.pad = 0;
+    r.term = -1;
     return r;
 }
 
@@ -283,7 +283,8 @@ template <typename T, typename I>
 __global__ void __launch_bounds__(256)
 k_setup_lines(const T *__restrict__ lines, const I *__restrict__ idxs, const uint8_t *__restrict__ kernels,
               int kernel, int64_t n_lines, Geometry g, LineSetup<T> *__restrict__ setup,
-              LineLite *__restrict__ lite, unsigned long long *__restrict__ counters, int *__restrict__ flags)
+              LineLite *__restrict__ lite, const int32_t *__restrict__ line_term,
+              unsigned long long *__restrict__ counters, int *__restrict__ flags)
 {
     const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int ub = 0;
@@ -291,7 +292,11 @@ k_setup_lines(const T *__restrict__ lines, const I *__restrict__ idxs, const uin
         LineSetup<T> L;
         setup_line(lines, idxs, kernels, kernel, l, g, L, flags);
         setup[l] = L;
-        if constexpr (sizeof(T) == 4) lite[l] = line_lite(L);
+        if constexpr (sizeof(T) == 4) {
+            LineLite r = line_lite(L);
+            if (line_term) r.term = line_term[l];
+            lite[l] = r;
+        }
         ub = segment_bound(L, g);
     }
 #pragma unroll
@@ -1198,7 +1203,8 @@ static std::atomic<int64_t> g_slot_hint{0};
 template <typename T, typename I>
 static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs, const uint8_t *kernels,
                                 int kernel, int64_t n_lines, int64_t n_frames, int64_t H, int64_t W, int tile,
-                                int seg, hipStream_t st, int64_t *line_base = nullptr, bool slot_tiles = false)
+                                int seg, hipStream_t st, int64_t *line_base = nullptr, bool slot_tiles = false,
+                                const int32_t *line_term = nullptr)
 {
     Geometry &g = P.g;
     g.n_frames = n_frames;
@@ -1226,7 +1232,8 @@ static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs
     }
     const int blk = 256;
     k_setup_lines<T, I><<<grid_for(n_lines, blk), blk, 0, st>>>(lines, idxs, kernels, kernel, n_lines, g,
-                                                               P.setup.ptr, P.lite.ptr, counters.ptr, P.flags.ptr);
+                                                               P.setup.ptr, P.lite.ptr, line_term, counters.ptr,
+                                                               P.flags.ptr);
     CBX_HIP(hipGetLastError());
     uint64_t hv[3];
     int fl = 0, rc = 0;
@@ -1550,11 +1557,14 @@ static int draw_pixels_impl(int64_t n_frames, int64_t H, int64_t W, const T *lin
 // accumulate_lines, step 1: range checks of terms and frames (bad[0]: a term
 // outside [0, n_terms), bad[1]: a frame outside [0, n_frames)), the frame of
 // every term as int32 (frames32, n_terms entries) and, when comp != nullptr,
-// the frame of every line, comp[i] = frames[terms[i]].
+// the frame of every line, comp[i] = frames[terms[i]].  With cnt: also the lines
+// of every term (cnt), each line's place among them (rank, in no fixed order)
+// and the largest count (bad[2]).
 template <typename I>
 __global__ void k_term_frames(const I *__restrict__ terms, const I *__restrict__ frames, int64_t n_lines,
                               int64_t n_terms, int64_t n_frames, I *__restrict__ comp,
-                              int32_t *__restrict__ frames32, int *__restrict__ bad)
+                              int32_t *__restrict__ frames32, int *__restrict__ bad, int *__restrict__ cnt,
+                              int *__restrict__ rank)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i < n_terms) {
@@ -1569,7 +1579,66 @@ __global__ void k_term_frames(const I *__restrict__ terms, const I *__restrict__
         if (t < 0 || (int64_t)t >= n_terms) atomicOr(bad, 1);
         else f = frames[t];
         if (comp) comp[i] = (f < 0 || (int64_t)f >= n_frames) ? I(0) : f;
+        if (cnt && t >= 0 && (int64_t)t < n_terms) {
+            const int r = atomicAdd(&cnt[t], 1);
+            rank[i] = r;
+            if (r + 1 > __hip_atomic_load(bad + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(bad + 2, r + 1);
+        }
     }
+}
+
+// lines by term: order[off[t] + rank[i]] = i
+template <typename I>
+__global__ void k_term_order(const I *__restrict__ terms, const int *__restrict__ off, const int *__restrict__ rank,
+                             int64_t n_lines, int *__restrict__ order)
+{
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i < n_lines) order[off[terms[i]] + rank[i]] = (int)i;
+}
+
+// Squared distance of point (px, py) to the segment (ax, ay)-(bx, by).
+__device__ __forceinline__ double point_segment2(double px, double py, double ax, double ay, double bx, double by)
+{
+    const double ux = bx - ax, uy = by - ay, m = ux * ux + uy * uy;
+    double t = (m > 0.0) ? ((px - ax) * ux + (py - ay) * uy) / m : 0.0;
+    t = fmin(fmax(t, 0.0), 1.0);
+    const double dx = px - ax - t * ux, dy = py - ay - t * uy;
+    return dx * dx + dy * dy;
+}
+
+// line_term[i] = the term of line i if another line of it may draw one of line
+// i's pixels, else -1.  Every pixel of a line lies within its width of the
+// segment, up to the drift of the float walk: lines further apart than both
+// widths plus 1 px plus 1e-4 of their lengths share none.  (A line that draws
+// nothing, e.g. a NaN end point, touches none.)
+template <typename T, typename I>
+__global__ void k_term_touch(const T *__restrict__ lines, const I *__restrict__ terms, const int *__restrict__ off,
+                             const int *__restrict__ order, int64_t n_lines, int32_t *__restrict__ line_term)
+{
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= n_lines) return;
+    const int t = (int)terms[i];
+    const T *a = lines + 5 * i;
+    const double ax = a[0], ay = a[1], bx = a[2], by = a[3], wa = a[4];
+    const double la = fabs(bx - ax) + fabs(by - ay);
+    bool touch = false;
+    for (int k = off[t]; k < off[t + 1] && !touch; k++) {
+        const int j = order[k];
+        if (j == (int)i) continue;
+        const T *b = lines + 5 * (int64_t)j;
+        const double cx = b[0], cy = b[1], dx = b[2], dy = b[3];
+        const double r = wa + (double)b[4] + 1.0 + 1e-4 * (la + fabs(dx - cx) + fabs(dy - cy));
+        if (!(fmax(cx, dx) + r >= fmin(ax, bx) && fmin(cx, dx) - r <= fmax(ax, bx) && fmax(cy, dy) + r >= fmin(ay, by) &&
+              fmin(cy, dy) - r <= fmax(ay, by)))
+            continue;
+        // the segments cross, or the distance is an end point's
+        const double o1 = (bx - ax) * (cy - ay) - (by - ay) * (cx - ax), o2 = (bx - ax) * (dy - ay) - (by - ay) * (dx - ax);
+        const double o3 = (dx - cx) * (ay - cy) - (dy - cy) * (ax - cx), o4 = (dx - cx) * (by - cy) - (dy - cy) * (bx - cx);
+        const double d2 = fmin(fmin(point_segment2(ax, ay, cx, cy, dx, dy), point_segment2(bx, by, cx, cy, dx, dy)),
+                               fmin(point_segment2(cx, cy, ax, ay, bx, by), point_segment2(dx, dy, ax, ay, bx, by)));
+        touch = (o1 * o2 <= 0.0 && o3 * o4 <= 0.0) || d2 <= r * r;
+    }
+    line_term[i] = touch ? t : -1;
 }
 
 // The ids of the plan tiles that hold items (in no fixed order), one atomic
@@ -1609,7 +1678,10 @@ static void launch_accumulate(int kernel, T *out, const SegmentPlan<T> &P, T max
 // accumulate_lines (bresenham.cpp:151-256): lines grouped into terms, each
 // term reduced over its lines (in_overlap), terms reduced into frames
 // (out_overlap).  Equal overlaps compose to draw_lines with idxs =
-// frames[terms] on the tile path.  Mixed overlaps bin the lines by (term,
+// frames[terms] on the tile path.  So do mixed overlaps for every line that no
+// other line of its term can touch (k_term_touch), with out_overlap; the others
+// follow term by term in the same frame tiles (k_tiles_terms).  Double images
+// and terms of many lines (MAX_TERM_LINES) bin the lines by (term,
 // tile) and run the ordered tile kernel in accumulate mode: each term tile
 // is reduced in LDS in reference line order from zero, like the reference's
 // term buffer, and its touched pixels are combined into frame frames[term]
@@ -1617,6 +1689,11 @@ static void launch_accumulate(int kernel, T *out, const SegmentPlan<T> &P, T max
 // order, as under the reference's OpenMP loop over terms.
 // (term, tile) pairs of one mixed-overlap accumulate plan at most
 constexpr int64_t MAX_TERM_TILES = int64_t(1) << 24;
+// Mixed overlaps of float images whose terms hold at most this many lines go by
+// frame tiles (k_term_touch compares every pair of a term's lines: 256 x the
+// lines; 64 000 lines in 4000 terms of 16 and 16 frames of 512^2 take 1.37 ms by
+// (term, tile) lists and 0.23 ms by frame tiles).
+constexpr int64_t MAX_TERM_LINES = 256;
 
 // term of each line within the batch [t0, t1), or -1 (a line of another batch)
 template <typename I>
@@ -1651,23 +1728,35 @@ static int accumulate_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W,
     hipStream_t st = (hipStream_t)stream;
     const int64_t n_chk = n_lines > n_terms ? n_lines : n_terms;
     const bool same = in_overlap == out_overlap;
+    // different overlaps of float images: by frame tiles, unless a term is large
+    // (below), a tile index would not fit or max_val is not finite
+    bool by_tile = !same && sizeof(T) == 4 && std::isfinite(max_val) && n_lines > 0 && n_terms > 0 &&
+                   n_frames * ((H + 63) / 64) * ((W + 63) / 64) < (int64_t(1) << 31) / LIST_SUBS;
     DevBuf<I> comp;
     DevBuf<int32_t> frames32;
+    DevBuf<int> cnt, rank;
     if (n_chk > 0) {
         DevBuf<int> bad;
-        CBX_HIP(bad.alloc(2, st));
-        CBX_HIP(hipMemsetAsync(bad.ptr, 0, 2 * sizeof(int), st));
-        if (same && n_lines > 0) CBX_HIP(comp.alloc(n_lines, st));
+        CBX_HIP(bad.alloc(3, st));
+        if ((same || by_tile) && n_lines > 0) CBX_HIP(comp.alloc(n_lines, st));
         CBX_HIP(frames32.alloc(n_terms > 0 ? n_terms : 1, st));
+        if (by_tile) {
+            CBX_HIP(cnt.alloc(n_terms, st));
+            CBX_HIP(rank.alloc(n_lines, st));
+        }
+        void *const zp[2] = {bad.ptr, cnt.ptr};
+        const int64_t zw[2] = {3, by_tile ? n_terms : 0};
+        CBX_HIP(zero_words(st, 2, zp, zw));
         k_term_frames<I><<<grid_for(n_chk, 256), 256, 0, st>>>(terms, frames, n_lines, n_terms, n_frames,
-                                                                 comp.ptr, frames32.ptr, bad.ptr);
+                                                                 comp.ptr, frames32.ptr, bad.ptr, cnt.ptr, rank.ptr);
         CBX_HIP(hipGetLastError());
-        const void *src[2] = {bad.ptr, bad.ptr + 1};
-        const int nb[2] = {4, 4};
-        uint64_t hv[2] = {0, 0};
-        CBX_HIP(read_device_values(st, 2, src, nb, hv));
+        const void *src[3] = {bad.ptr, bad.ptr + 1, bad.ptr + 2};
+        const int nb[3] = {4, 4, 4};
+        uint64_t hv[3] = {0, 0, 0};
+        CBX_HIP(read_device_values(st, 3, src, nb, hv));
         if (hv[1]) return fail(CBX_EINDEX, "frames is outside of (0, n_frames)");
         if (hv[0]) return fail(CBX_EINDEX, "a term index is outside of (0, len(frames))");
+        by_tile = by_tile && (int64_t)hv[2] <= MAX_TERM_LINES;
     }
     if (n_lines == 0 || n_frames * H * W == 0) return CBX_OK;
     // max/max: the term buffer starts at zero and takes std::max(buffer, v),
@@ -1676,6 +1765,39 @@ static int accumulate_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W,
     if (same) return draw_lines_impl<T, I>(out, n_frames, H, W, lines, n_lines, comp.ptr,
                                            (in_overlap == 1 && max_val < T(0)) ? T(0) : max_val, kernel,
                                            in_overlap, opts, stream);
+
+    if constexpr (sizeof(T) == 4) {
+        if (by_tile) {
+            DevBuf<int> off, order;
+            DevBuf<int32_t> line_term;
+            CBX_HIP(off.alloc(n_terms + 1, st));
+            CBX_HIP(order.alloc(n_lines, st));
+            CBX_HIP(line_term.alloc(n_lines, st));
+            CBX_HIP(exclusive_scan_total_i32(cnt.ptr, nullptr, off.ptr, n_terms, st));
+            const unsigned grid = (unsigned)grid_for(n_lines, 256);
+            k_term_order<I><<<grid, 256, 0, st>>>(terms, off.ptr, rank.ptr, n_lines, order.ptr);
+            k_term_touch<T, I><<<grid, 256, 0, st>>>(lines, terms, off.ptr, order.ptr, n_lines, line_term.ptr);
+            CBX_HIP(hipGetLastError());
+            // a term's buffer starts at zero: with max_val < 0 its maximum is 0
+            const T mv = (in_overlap == 1 && max_val < T(0)) ? T(0) : max_val;
+            SegmentPlan<T> P;
+            if ((rc = build_plan_unordered<T, I>(P, lines, comp.ptr, nullptr, kernel, n_lines, n_frames, H, W, 64, 8, st,
+                                                 nullptr, false, line_term.ptr)))
+                return rc;
+            if (P.n_segs == 0) return CBX_OK;
+            KernelTimer timer("accumulate_tiles", st);
+            run_tiles<T>(out, P, kernel, out_overlap, mv, nullptr, st);
+            switch (kernel) {
+            case K_BIWEIGHT: run_tiles_terms<K_BIWEIGHT>(out, P, mv, in_overlap, st); break;
+            case K_GAUSSIAN: run_tiles_terms<K_GAUSSIAN>(out, P, mv, in_overlap, st); break;
+            case K_PARABOLIC: run_tiles_terms<K_PARABOLIC>(out, P, mv, in_overlap, st); break;
+            case K_RECTANGULAR: run_tiles_terms<K_RECTANGULAR>(out, P, mv, in_overlap, st); break;
+            default: run_tiles_terms<K_TRIANGULAR>(out, P, mv, in_overlap, st); break;
+            }
+            CBX_HIP(hipGetLastError());
+            return CBX_OK;
+        }
+    }
 
     // The plan's frames are terms: (term, tile) lists scale with n_terms.
     // Above MAX_TERM_TILES pairs the terms go in batches, each with a plan of
@@ -1943,7 +2065,7 @@ static int plan_draw(cbx_plan *pl, float *out, const float *lines, int64_t n_lin
                                                          P.tile_cur.ptr, pl->scan_state.ptr,
                                                          (int64_t)pl->scan_state.n);
     k_setup_lines<float, int32_t><<<grid_for(n_lines, blk), blk, 0, st>>>(lines, idxs, kernels, kernel, n_lines, g,
-                                                                         P.setup.ptr, P.lite.ptr, pl->counters.ptr,
+                                                                         P.setup.ptr, P.lite.ptr, nullptr, pl->counters.ptr,
                                                                          P.flags.ptr);
     k_walk_lines<float><<<grid_for(n_lines, blk), blk, 0, st>>>(n_lines, g, P.setup.ptr, P.segs.ptr, P.n_segs,
                                                                 pl->counters.ptr, P.tile_cnt.ptr, P.flags.ptr,

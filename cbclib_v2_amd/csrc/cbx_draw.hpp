@@ -29,7 +29,8 @@ struct alignas(16) LineLite {
     float nlim;       // band limit
     float cap;        // a column with cap < Te < LL - cap has no tangential overshoot at any of its pixels
     int32_t meta;     // FR_* bits, profile id in bits 8-15
-    int32_t pad;
+    int32_t term;     // accumulate_lines with different overlaps: the line's term when another line of it
+                      // may touch this one, else (and in every other draw) -1
 };
 constexpr int FR_AXIS = 1, FR_SA = 2, FR_SB = 4, FR_SAFE = 8;
 
@@ -197,5 +198,11 @@ struct SegmentPlan {
 template <typename T, int K>
 void run_tiles_profile(T *out, const SegmentPlan<T> &P, T max_val, int overlap, const cbx_draw_opts *opts,
                        hipStream_t st);
+
+// accumulate_lines with different overlaps, after run_tiles_profile has drawn the
+// lines alone in their pixels (LineLite::term < 0): the other lines, term by term
+// (k_tiles_terms; plans of 64-pixel tiles and 8-column segments).
+template <int K>
+void run_tiles_terms(float *out, const SegmentPlan<float> &P, float max_val, int in_overlap, hipStream_t st);
 
 } // namespace cbx
