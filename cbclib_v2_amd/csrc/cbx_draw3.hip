@@ -12,17 +12,21 @@
 // sqrt), so the emitted pixel set and the per-pixel values are the
 // reference's exactly.
 //
-// Four lanes walk one line (each replays the main-axis walk and fills one
-// quadrant of every orthogonal plane; the first also emits the main-axis
-// pixels) and apply its pixels to `out` with global atomics (add for sum,
-// compare-and-swap for max): sums land in no fixed order (within float
-// rounding of the single-threaded reference), max is exact.  A validation pass runs first, so a call that fails leaves `out`
-// untouched.
+// A draw records every line's planes (k_walk3_main, a lane per line) and fills
+// them (k_fill3, four lanes per plane); above MAX_PLANES planes, and for
+// accumulate_lines with different overlaps, four lanes walk a line instead
+// (each replays the main-axis walk and fills one quadrant of every orthogonal
+// plane; the first also emits the main-axis pixels).  Pixels are applied to
+// `out` with global atomics (add for sum, compare-and-swap for max): sums land
+// in no fixed order (within float rounding of the single-threaded reference),
+// max is exact.  A validation pass runs first, so a call that fails leaves
+// `out` untouched.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <climits>
 #include <string>
+#include <type_traits>
 
 #include "cbx_core.hpp"
 #include "cbx_host.hpp"
@@ -392,25 +396,6 @@ k_draw3(T *__restrict__ out, const T *__restrict__ lines, int64_t n_lines, const
 // as many steps each (one lane per line left most of a wave idle behind its
 // longest and widest line).
 
-// ub[i]: planes of line i at most (the long-axis span), 0 if it draws nothing;
-// ub[n_lines] = 0 (the scan's total)
-template <typename T>
-__global__ void __launch_bounds__(D3_NT)
-k_plane_bound(const T *__restrict__ lines, int64_t n_lines, int64_t *__restrict__ ub)
-{
-    const int64_t i = (int64_t)blockIdx.x * D3_NT + threadIdx.x;
-    if (i > n_lines) return;
-    int64_t n = 0;
-    if (i < n_lines) {
-        Line3<T> L;
-        if (line3_setup(lines + 7 * i, L) == 1) {
-            const int64_t sp = (L.axis == 0) ? L.m1[0] - L.m0[0] : ((L.axis == 1) ? L.m1[1] - L.m0[1] : L.m1[2] - L.m0[2]);
-            n = sp < 0 ? -sp : sp;
-        }
-    }
-    ub[i] = n;
-}
-
 template <typename T>
 __global__ void __launch_bounds__(D3_NT)
 k_walk3_main(const T *__restrict__ lines, int64_t n_lines, const int64_t *__restrict__ off,
@@ -444,37 +429,356 @@ k_walk3_main(const T *__restrict__ lines, int64_t n_lines, const int64_t *__rest
     for (; k < cap; k++) states[base + k].line = -1;
 }
 
-template <int AXIS, typename T, typename Emit>
-__device__ __forceinline__ void fill_plane(const Line3<T> &L, const Iter3<T> &it, int quad, int *flags, Emit &emit)
+// A line's constants for the fills of its planes: Line3's, and what turns their
+// divisions into products (a correctly rounded reciprocal and one correction
+// step give the IEEE quotient).
+template <typename T>
+struct alignas(16) Rec3 {
+    T t[3];              // p1 - p0: the pair normals are (t[b], -t[a])
+    T len, rlen, LL, w2;
+    T in, out;           // sum of the squared normal errors, times len^2: below `in` the pixel is within w, above `out` beyond
+    double rw2;          // 1 / (double)w2
+    int64_t frame;
+    int32_t ray_cap;
+    int32_t span[3];     // steps a plane's pixels lie from its centre along each axis (patch size: a few may lie further)
+    int8_t axis, step[3];
+};
+
+__device__ __forceinline__ float div3(float a, float b, float rb) { return div_rn(a, b, rb); }
+__device__ __forceinline__ double div3(double a, double b, double rb) { return div_rn(a, b, rb); }
+
+// it3_nerr with the reciprocal: the square of a float is exact in double, so one
+// FMA rounds like the reference's double addition
+__device__ __forceinline__ float nerr3(const Rec3<float> &L, const float *ne)
 {
-    if (quad == 0) emit(it.cur, it3_err(L, it));
-    fill3_quadrant<AXIS>(L, it, quad, flags, emit);
+    float e = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const double v = (double)div3(ne[q], L.len, L.rlen);
+        e = (float)__builtin_fma(v, v, (double)e);
+    }
+    return e;
 }
 
-template <typename T, typename I, int K, int OV>
-__global__ void __launch_bounds__(D3_NT)
-k_fill3(T *__restrict__ out, const T *__restrict__ lines, const PlaneState<T> *__restrict__ states, int64_t n_states,
-        int64_t n_lines, const I *__restrict__ idxs, Vol3 v, T max_val, int *__restrict__ flags)
+__device__ __forceinline__ double nerr3(const Rec3<double> &L, const double *ne)
 {
-    const int64_t u = (int64_t)blockIdx.x * D3_NT + threadIdx.x;
-    if (u >= 4 * n_states) return;
-    const PlaneState<T> ps = states[u >> 2];
-    if (ps.line < 0) return;
-    const int64_t i = ps.line;
-    Line3<T> L;
-    if (line3_setup(lines + 7 * i, L) != 1) return;
-    Iter3<T> it;
-    it3_from(L, ps, it);
-    const int64_t f = idxs ? (int64_t)idxs[i] : ((v.n_frames == 1) ? 0 : i);
-    T *fo = out + f * v.D * v.H * v.W;
-    auto emit = [&](const int64_t *p, T err) {
-        if (!(err <= T(1)) || p[0] < 0 || p[0] >= v.W || p[1] < 0 || p[1] >= v.H || p[2] < 0 || p[2] >= v.D) return;
-        apply_atomic<OV>(fo + (p[2] * v.H + p[1]) * v.W + p[0], pixel_value<K>(err, max_val));
+    double e = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const double v = div3(ne[q], L.len, L.rlen);
+        e = e + v * v;
+    }
+    return e;
+}
+
+__device__ __forceinline__ float err3(const Rec3<float> &L, float te, float nerr)
+{
+    const float a = -te, b = te - L.LL, m = (a < b) ? b : a, at = (m < 0.0f) ? 0.0f : m;
+    const double qt = (double)div3(at, L.len, L.rlen);
+    return (float)div_rn(__builtin_fma(qt, qt, (double)nerr), (double)L.w2, L.rw2);
+}
+
+__device__ __forceinline__ double err3(const Rec3<double> &L, double te, double nerr)
+{
+    const double a = -te, b = te - L.LL, m = (a < b) ? b : a, at = (m < 0.0) ? 0.0 : m;
+    const double qt = div3(at, L.len, L.rlen), qt2 = qt * qt;
+    return (qt2 + nerr) / L.w2;
+}
+
+// Validation (as k_check3), ub[i]: planes of line i at most (the long-axis span),
+// 0 if it draws nothing (ub[n_lines] = 0: the scan's total), and its record.
+template <typename T, typename I>
+__global__ void __launch_bounds__(D3_NT)
+k_setup3(const T *__restrict__ lines, int64_t n_lines, const I *__restrict__ idxs, Vol3 v, int *__restrict__ flags,
+         int64_t *__restrict__ ub, Rec3<T> *__restrict__ rec)
+{
+    const int64_t i = (int64_t)blockIdx.x * D3_NT + threadIdx.x;
+    if (i > n_lines) return;
+    int64_t n = 0;
+    if (i < n_lines) {
+        const int64_t f = idxs ? (int64_t)idxs[i] : ((v.n_frames == 1) ? 0 : i);
+        if (f < 0 || f >= v.n_frames) atomicOr(flags, FLAG_INDEX);
+        Line3<T> L;
+        const int rc = line3_setup(lines + 7 * i, L);
+        if (rc < 0) atomicOr(flags, FLAG_LONG);
+        if (rc == 1) {
+            const int a = L.axis;
+            const int64_t m0 = (a == 0) ? L.m0[0] : ((a == 1) ? L.m0[1] : L.m0[2]);
+            const int64_t m1 = (a == 0) ? L.m1[0] : ((a == 1) ? L.m1[1] : L.m1[2]);
+            n = (m1 > m0) ? m1 - m0 : m0 - m1;
+            Rec3<T> R;
+            for (int k = 0; k < 3; k++) {
+                R.t[k] = L.t[k];
+                R.step[k] = (int8_t)L.step[k];
+            }
+            R.len = L.len;
+            R.rlen = T(1) / L.len;
+            R.LL = L.len * L.len;
+            R.w2 = L.w2;
+            R.rw2 = 1.0 / (double)L.w2;
+            const double lim = (double)L.w2 * (double)L.len * (double)L.len, tol = sizeof(T) == 4 ? 4e-6 : 1e-13;
+            R.in = (T)(lim * (1.0 - tol));
+            R.out = (T)(lim * (1.0 + tol));
+            const T ta = (a == 0) ? L.t[0] : ((a == 1) ? L.t[1] : L.t[2]);
+            for (int k = 0; k < 3; k++) {
+                const float slope = (float)(L.t[k] / ta);
+                R.span[k] = (int32_t)fminf((float)lines[7 * i + 6] * sqrtf(1.0f + slope * slope) + 0.5f, 1e6f);
+            }
+            R.frame = f;
+            R.ray_cap = (int32_t)min(L.ray_cap, (int64_t)INT_MAX);
+            R.axis = (int8_t)a;
+            rec[i] = R;
+        }
+    }
+    ub[i] = n;
+}
+
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ uint32_t patch_bits(float v) { return __float_as_uint(v); }
+__device__ __forceinline__ unsigned long long patch_bits(double v) { return (unsigned long long)__double_as_longlong(v); }
+__device__ __forceinline__ float patch_value(uint32_t b) { return __uint_as_float(b); }
+__device__ __forceinline__ double patch_value(unsigned long long b) { return __longlong_as_double((long long)b); }
+
+// Fills of the recorded planes.  A wave takes FILL_PLANES consecutive planes, one
+// (plane, quadrant) per lane (fill3_quadrant's pixels: a walk away from the
+// line with, from each of its pixels, a ray along the other axis for each axis
+// that the next step moves).  Walk and rays are one loop, a candidate pixel of
+// every lane per turn, written in terms of the plane's axes P < Q, so that
+// lanes at different places of their walks and on different axes stay
+// together; the pixels inside go to the wave's queue, whose errors and profile
+// values 64 lanes compute at a time.
+//
+// The volume is updated with global atomics, whose rate is one request per 64
+// bytes and instruction: 13 M float additions take 621 us at random places, 189
+// us in runs of 4 along x, 81 us in runs of 16.  So the values of a plane
+// across y or z first go to a patch of the plane in LDS, whose rows along x are
+// then added by neighbouring lanes; planes across x (their pixels at one place
+// of consecutive planes are neighbours in x, and in the queue) and pixels
+// outside the patch are added directly.
+//
+// Bound by the loop's vector instructions (191 M wave instructions, 310 us at
+// the issue rate, for 50 000 lines of widths 1 to 3, 13 M voxels, in 16 volumes
+// of 64 x 128 x 128).  A wave's patch and queue limit the waves in flight: with
+// patches of 1536, 1024, 768, 640 values 526, 433, 387, 381 us (planes that
+// find no room in the patch are added directly, so not smaller still).
+// One lane per (plane, quadrant) with atomics for every pixel took 623 us.
+constexpr int FILL_PLANES = 16, FILL_NT = 256, FILL_QUEUE = 128;
+
+template <typename T, int K, int OV>
+__global__ void __launch_bounds__(FILL_NT)
+k_fill3(T *__restrict__ out, const Rec3<T> *__restrict__ rec, const PlaneState<T> *__restrict__ states,
+        int64_t n_states, Vol3 v, T max_val, int *__restrict__ flags)
+{
+    constexpr int NW = FILL_NT / 64, PATCH = sizeof(T) == 4 ? 768 : 512;
+    using Bits = typename std::conditional<sizeof(T) == 4, uint32_t, unsigned long long>::type;
+    struct Entry {   // a pixel to draw: its errors, its plane (4 bits) and offsets from the centre along P, Q (14 bits each)
+        T te, ne[3];
+        uint32_t at;
     };
-    const int quad = (int)(u & 3);
-    if (L.axis == 0) fill_plane<0>(L, it, quad, flags, emit);
-    else if (L.axis == 1) fill_plane<1>(L, it, quad, flags, emit);
-    else fill_plane<2>(L, it, quad, flags, emit);
+    struct Plane {
+        int64_t centre;   // index of its centre in `out`
+        int32_t line, patch, spanP, spanQ;
+        int32_t sP, sQ;   // strides along P, Q
+    };
+    __shared__ Entry queue[NW][FILL_QUEUE];
+    __shared__ Bits patch[NW][PATCH];
+    __shared__ Plane plane[NW][FILL_PLANES];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int64_t first = ((int64_t)blockIdx.x * NW + wave) * FILL_PLANES;
+    const int pl = lane & (FILL_PLANES - 1), quad = lane / FILL_PLANES;
+    const bool have = first + pl < n_states;
+    PlaneState<T> ps;
+    ps.line = -1;
+    if (have) ps = states[first + pl];
+    bool go = ps.line >= 0;
+
+    T te = T(0), ne[3], xte = T(0), xne[3], s_in = T(0), s_out = T(0), stP = T(0), stQ = T(0);
+    T iP[3], iQ[3];   // changes of the three normal errors per step along P, Q (one of them zero each)
+    int count = 0, walks = 0, cap = 0, plane_q = 0;   // count, walks: steps of the ray, of the walk
+    // offsets from the centre along P, Q (of the candidate, of the walk), steps, offsets inside the volume
+    int oP = 0, oQ = 0, xP = 0, xQ = 0, dP = 0, dQ = 0, loP = 0, hiP = -1, loQ = 0, hiQ = -1, side = 0;
+    bool second = false, alongP = false, flat = false;
+    const Rec3<T> *L = rec;
+    for (int k = 0; k < 3; k++) ne[k] = xne[k] = iP[k] = iQ[k] = T(0);
+    if (go) {
+        L = rec + ps.line;
+        const int a = L->axis;
+        const int P = (a == 0) ? 1 : 0, Q = (a == 2) ? 1 : 2;
+        const T t0 = L->t[0], t1 = L->t[1], t2 = L->t[2];
+        const T tP = (P == 0) ? t0 : t1, tQ = (Q == 1) ? t1 : t2;
+        const bool flip1 = quad & 1, flip2 = quad >> 1;   // of axes (a + 1) % 3, (a + 2) % 3
+        dP = ((P == 0) ? L->step[0] : L->step[1]) * (((a == 1) ? flip2 : flip1) ? -1 : 1);
+        dQ = ((Q == 1) ? L->step[1] : L->step[2]) * (((a == 1) ? flip1 : flip2) ? -1 : 1);
+        const T fP = (T)dP, fQ = (T)dQ;
+        stP = fP * tP;
+        stQ = fQ * tQ;
+        // pairs (0,1), (0,2), (1,2): normals (t[b], -t[a])
+        iP[0] = fP * ((P == 0) ? t1 : -t0);
+        iP[1] = (P == 0) ? fP * t2 : T(0);
+        iP[2] = (P == 0) ? T(0) : fP * t2;
+        iQ[0] = (Q == 1) ? fQ * -t0 : T(0);
+        iQ[1] = (Q == 1) ? T(0) : fQ * -t0;
+        iQ[2] = (Q == 1) ? fQ * t2 : fQ * -t1;
+        plane_q = (a == 0) ? 2 : ((a == 1) ? 1 : 0);
+        s_in = L->in;
+        s_out = L->out;
+        cap = L->ray_cap;
+        const int64_t ca = (a == 0) ? ps.cur[0] : ((a == 1) ? ps.cur[1] : ps.cur[2]);
+        const int64_t da = (a == 0) ? v.W : ((a == 1) ? v.H : v.D);
+        const int cP = (P == 0) ? ps.cur[0] : ps.cur[1], cQ = (Q == 1) ? ps.cur[1] : ps.cur[2];
+        const int64_t nP = (P == 0) ? v.W : v.H, nQ = (Q == 1) ? v.H : v.D;
+        const int64_t strP = (P == 0) ? 1 : v.W, strQ = (Q == 1) ? v.W : v.W * v.H;
+        // offsets inside the volume (MAX_VISITS3 keeps a plane's pixels well within 2^13 of its centre: Entry::at);
+        // a plane outside of it draws nothing
+        flat = ca >= 0 && ca < da;
+        loP = (int)max(-(int64_t)cP, (int64_t)-8191);
+        hiP = (int)min(nP - 1 - cP, (int64_t)8191);
+        loQ = (int)max(-(int64_t)cQ, (int64_t)-8191);
+        hiQ = (int)min(nQ - 1 - cQ, (int64_t)8191);
+        if (!flat) hiP = loP - 1;
+        te = ps.te;
+        for (int k = 0; k < 3; k++) ne[k] = ps.ne[k];
+        const bool one = flip1 != flip2;   // the first step: along (a + 2) % 3 when exactly one axis is flipped
+        alongP = (a == 1) ? one : !one;
+        const int spanP = (P == 0) ? L->span[0] : L->span[1], spanQ = (Q == 1) ? L->span[1] : L->span[2];
+        side = (a != 0 && flat && spanP < 32 && spanQ < 32) ? (2 * spanP + 1) * (2 * spanQ + 1) : 0;
+        if (quad == 0) {
+            Plane &p = plane[wave][pl];
+            p.centre = ((L->frame * v.D + ps.cur[2]) * v.H + ps.cur[1]) * v.W + ps.cur[0];
+            p.line = ps.line;
+            p.spanP = spanP;
+            p.spanQ = spanQ;
+            p.sP = (int32_t)strP;
+            p.sQ = (int32_t)strQ;
+        }
+    }
+    // patches one after the other (a plane whose patch does not fit has none)
+    {
+        int x = side;
+#pragma unroll
+        for (int d = 1; d < FILL_PLANES; d <<= 1) {
+            const int y = __shfl_up(x, d, FILL_PLANES);
+            if (pl >= d) x += y;
+        }
+        if (quad == 0) plane[wave][pl].patch = (side > 0 && x <= PATCH) ? x - side : -1;
+        const int all = min(__shfl(x, FILL_PLANES - 1, FILL_PLANES), PATCH);
+        for (int i = lane; i < all; i += 64) patch[wave][i] = (Bits)~(Bits)0;   // (a NaN that no value has)
+    }
+    wave_fence();
+    auto put = [&](T pte, const T *pne, uint32_t at) {
+        const Plane &p = plane[wave][at >> 28];
+        const Rec3<T> &R = rec[p.line];
+        const T e = err3(R, pte, nerr3(R, pne));
+        if (!(e <= T(1))) return;
+        const T val = pixel_value<K>(e, max_val);
+        const int qP = (int)((at >> 14) & 0x3fffu) - 8192, qQ = (int)(at & 0x3fffu) - 8192;
+        if (p.patch >= 0 && abs(qP) <= p.spanP && abs(qQ) <= p.spanQ)
+            patch[wave][p.patch + (qQ + p.spanQ) * (2 * p.spanP + 1) + qP + p.spanP] = patch_bits(val);
+        else
+            apply_atomic<OV>(out + (p.centre + (int64_t)qP * p.sP + (int64_t)qQ * p.sQ), val);
+    };
+    int q_head = 0, q_tail = 0;   // the wave's queue (uniform over the wave)
+    auto drain = [&](int n) {
+        wave_fence();
+        if (lane < n) {
+            const Entry e = queue[wave][(q_head + lane) & (FILL_QUEUE - 1)];
+            put(e.te, e.ne, e.at);
+        }
+        q_head += n;
+        wave_fence();
+    };
+    auto push = [&](bool mine) {
+        const uint64_t m = __ballot(mine);
+        if (m == 0) return;
+        if (mine) {
+            Entry &e = queue[wave][(q_tail + __popcll(m & below)) & (FILL_QUEUE - 1)];
+            e.te = te;
+            for (int k = 0; k < 3; k++) e.ne[k] = ne[k];
+            e.at = ((uint32_t)pl << 28) | ((uint32_t)(oP + 8192) << 14) | (uint32_t)(oQ + 8192);
+        }
+        q_tail += __popcll(m);
+        if (q_tail - q_head >= 64) drain(64);
+    };
+    // the plane's centre, without the band test
+    push(go && quad == 0 && loP <= 0 && hiP >= 0 && loQ <= 0 && hiQ >= 0);
+    // the quadrant's first pixel
+    te += alongP ? stP : stQ;
+    for (int k = 0; k < 3; k++) ne[k] += alongP ? iP[k] : iQ[k];
+    oP = alongP ? dP : 0;
+    oQ = alongP ? 0 : dQ;
+    int dir = 0;           // 0: the walk's own pixel, 1: a ray along Q, 2: a ray along P
+    bool nP = false, nQ = false;
+    while (__ballot(go)) {
+        const T s2 = ne[0] * ne[0] + ne[1] * ne[1] + ne[2] * ne[2];
+        bool in = go && s2 < s_in;
+        if (go && !in && !(s2 > s_out)) in = nerr3(*L, ne) < L->w2;
+        if (in && (count == cap || walks == cap)) {
+            atomicOr(flags, FLAG_STUCK);
+            go = in = false;
+        }
+        push(in && oP >= loP && oP <= hiP && oQ >= loQ && oQ <= hiQ);
+        // the next candidate: from the pixel before or from the walk's
+        const bool walk = dir == 0;
+        go = go && (in || !walk);
+        if (walk) {
+            // the walk's pixel: keep it, and its next step (it3_update)
+            xte = te;
+            for (int k = 0; k < 3; k++) xne[k] = ne[k];
+            xP = oP;
+            xQ = oQ;
+            const T w = (plane_q == 0) ? ne[0] : ((plane_q == 1) ? ne[1] : ne[2]);
+            const T gP = (plane_q == 0) ? iP[0] : ((plane_q == 1) ? iP[1] : iP[2]);
+            const T gQ = (plane_q == 0) ? iQ[0] : ((plane_q == 1) ? iQ[1] : iQ[2]);
+            const T eP = w + gP, eQ = w + gQ, eb = eP + gQ;
+            const bool qb = m_abs(eQ) < m_abs(eP);
+            const bool both = m_abs(eb) < m_abs(qb ? eQ : eP);
+            nP = !qb || both;
+            nQ = qb || both;
+        }
+        const bool on = in && !walk;                 // the ray goes on
+        second = !in && dir == 1 && nQ;              // the ray along P comes next
+        const bool step = !walk && !in && !second;   // the walk's next step
+        const bool mP = on ? dir == 2 : (walk ? !nP : (second || nP));
+        const bool mQ = on ? dir == 1 : (walk ? nP : (!second && nQ));
+        count = on ? count + 1 : 0;
+        walks += step ? 1 : 0;
+        te = on ? te : xte;
+        te += mP ? stP : T(0);
+        te += mQ ? stQ : T(0);
+        for (int k = 0; k < 3; k++) {
+            ne[k] = on ? ne[k] : xne[k];
+            ne[k] += mP ? iP[k] : T(0);
+            ne[k] += mQ ? iQ[k] : T(0);
+        }
+        oP = (on ? oP : xP) + (mP ? dP : 0);
+        oQ = (on ? oQ : xQ) + (mQ ? dQ : 0);
+        dir = on ? dir : (walk ? (nP ? 1 : 2) : (second ? 2 : 0));
+    }
+    drain(q_tail - q_head);
+    // the patches' rows
+    for (int k = 0; k < FILL_PLANES; k++) {
+        if (first + k >= n_states) break;
+        const bool used = __shfl(side, k, 64) > 0;
+        if (!used) continue;
+        const Plane &p = plane[wave][k];
+        if (p.patch < 0) continue;
+        const int n = 2 * p.spanP + 1, all = n * (2 * p.spanQ + 1);
+        const float rn = 1.0f / (float)n;
+        T *const o = out + p.centre;
+        for (int i = lane; i < all; i += 64) {
+            const Bits bits = patch[wave][p.patch + i];
+            if (bits == (Bits)~(Bits)0) continue;
+            const int y = (int)(((float)i + 0.5f) * rn), x = i - y * n;
+            apply_atomic<OV>(o + ((int64_t)(x - p.spanP) * p.sP + (int64_t)(y - p.spanQ) * p.sQ), patch_value(bits));
+        }
+    }
 }
 
 // accumulate_lines, mixed overlaps: the lines of terms [t0, t0 + nb) drawn
@@ -602,12 +906,12 @@ static void launch_draw3(int kernel, T *out, const T *lines, int64_t n, const I 
     }
 }
 
-template <typename T, typename I, int OV>
-static void launch_fill3(int kernel, T *out, const T *lines, const PlaneState<T> *states, int64_t n_states,
-                         int64_t n_lines, const I *idxs, const Vol3 &v, T mv, int *flags, hipStream_t st)
+template <typename T, int OV>
+static void launch_fill3(int kernel, T *out, const Rec3<T> *rec, const PlaneState<T> *states, int64_t n_states,
+                         const Vol3 &v, T mv, int *flags, hipStream_t st)
 {
-    const unsigned g = (unsigned)grid_for(4 * n_states, D3_NT);   // four lanes per plane
-#define CBX_FILL3(KK) k_fill3<T, I, KK, OV><<<g, D3_NT, 0, st>>>(out, lines, states, n_states, n_lines, idxs, v, mv, flags)
+    const unsigned g = (unsigned)((n_states + FILL_PLANES * (FILL_NT / 64) - 1) / (FILL_PLANES * (FILL_NT / 64)));
+#define CBX_FILL3(KK) k_fill3<T, KK, OV><<<g, FILL_NT, 0, st>>>(out, rec, states, n_states, v, mv, flags)
     switch (kernel) {
     case K_BIWEIGHT: CBX_FILL3(K_BIWEIGHT); break;
     case K_GAUSSIAN: CBX_FILL3(K_GAUSSIAN); break;
@@ -619,31 +923,42 @@ static void launch_fill3(int kernel, T *out, const T *lines, const PlaneState<T>
 }
 
 // validation, the draw, then its step-budget flag (inside an open Workspace).
-// Above MAX_PLANES recorded planes the single-kernel walk (four lanes per
-// line) runs instead of the two phases.
+// Above MAX_PLANES recorded planes, or with strides or widths that the fills'
+// 32-bit offsets do not hold, the single-kernel walk (four lanes per line)
+// runs instead of the two phases.
 template <typename T, typename I>
 static int draw3_run(T *out, const Vol3 &v, const T *lines, int64_t n_lines, const I *idxs, T max_val, int kernel,
                      int overlap, hipStream_t st)
 {
     DevBuf<int> flags;
-    CBX_HIP(flags.alloc(1, st));
-    int rc = validate3(lines, n_lines, idxs, v, flags.ptr, st);
-    if (rc) return rc;
-    // planes of every line: offsets by a scan of their bounds
     DevBuf<int64_t> ub, off;
+    DevBuf<Rec3<T>> rec;
+    CBX_HIP(flags.alloc(1, st));
     CBX_HIP(ub.alloc((size_t)n_lines + 1, st));
     CBX_HIP(off.alloc((size_t)n_lines + 1, st));
-    k_plane_bound<T><<<grid_for(n_lines + 1, D3_NT), D3_NT, 0, st>>>(lines, n_lines, ub.ptr);
+    CBX_HIP(rec.alloc((size_t)n_lines, st));
+    {
+        void *const zp[1] = {flags.ptr};
+        const int64_t zw[1] = {1};
+        CBX_HIP(zero_words(st, 1, zp, zw));
+    }
+    // checks, records and the planes of every line: offsets by a scan of their bounds
+    k_setup3<T, I><<<grid_for(n_lines + 1, D3_NT), D3_NT, 0, st>>>(lines, n_lines, idxs, v, flags.ptr, ub.ptr, rec.ptr);
     CBX_HIP(hipGetLastError());
     CBX_HIP(exclusive_scan_i64(ub.ptr, off.ptr, n_lines + 1, st));
     uint64_t total = 0;
+    int rc;
     {
-        const void *src[1] = {off.ptr + n_lines};
-        const int nb[1] = {8};
-        CBX_HIP(read_device_values(st, 1, src, nb, &total));
+        uint64_t hv[2];
+        const void *src[2] = {off.ptr + n_lines, flags.ptr};
+        const int nb[2] = {8, 4};
+        CBX_HIP(read_device_values(st, 2, src, nb, hv));
+        total = hv[0];
+        if ((rc = flags3_status((int)hv[1]))) return rc;
     }
+    if (max_val != max_val) max_val = (T)NAN;   // (k_fill3's patches keep one pattern for themselves)
     DevBuf<PlaneState<T>> states;
-    const bool two_phase = total <= (uint64_t)MAX_PLANES;
+    const bool two_phase = total <= (uint64_t)MAX_PLANES && v.W * v.H < (int64_t(1) << 31) && n_lines < INT_MAX;
     if (two_phase && total > 0) CBX_HIP(states.alloc((size_t)total, st));
     {
         KernelTimer timer("draw3", st);
@@ -652,11 +967,9 @@ static int draw3_run(T *out, const Vol3 &v, const T *lines, int64_t n_lines, con
                 k_walk3_main<T><<<grid_for(n_lines, D3_NT), D3_NT, 0, st>>>(lines, n_lines, off.ptr, states.ptr,
                                                                            flags.ptr);
                 if (overlap == 0)
-                    launch_fill3<T, I, 0>(kernel, out, lines, states.ptr, (int64_t)total, n_lines, idxs, v, max_val,
-                                          flags.ptr, st);
+                    launch_fill3<T, 0>(kernel, out, rec.ptr, states.ptr, (int64_t)total, v, max_val, flags.ptr, st);
                 else
-                    launch_fill3<T, I, 1>(kernel, out, lines, states.ptr, (int64_t)total, n_lines, idxs, v, max_val,
-                                          flags.ptr, st);
+                    launch_fill3<T, 1>(kernel, out, rec.ptr, states.ptr, (int64_t)total, v, max_val, flags.ptr, st);
             }
         } else if (overlap == 0) {
             launch_draw3<T, I, 0>(kernel, out, lines, n_lines, idxs, v, max_val, flags.ptr, st);
