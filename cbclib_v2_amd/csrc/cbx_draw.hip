@@ -905,40 +905,411 @@ __device__ __forceinline__ void pixel_grad(const GradConst &C, int x, int y, dou
 template <int TILE>
 constexpr int tile_pitch() { return TILE + 4; }
 
-// The fills of one column for the float fast path (both halves and the
-// centre), with the forward's band test and inclusion decisions (err_fast);
-// lines with L.safe only.
-template <int K, int TILE>
-__device__ __forceinline__ void adj_column_fast(const LineSetup<float> &L, const GradConst &C, const float *gt, int cs,
-                                                float Te0, float Ne0, int c, int X0, int Y0, int s_lo, int s_hi,
-                                                double *acc)
+// The sums of one column's gradient terms.  With (a, b) the line's long and
+// short axes, r = p - p0, t the exact tangent, q = r_a t_b - r_b t_a and T = r t
+// (both linear along the column), Tc = T clamped to [0, |t|^2] and o = T - Tc, a
+// pixel's vector from its projection is (q (t_b, -t_a) + o (t_a, t_b)) / |t|^2,
+// its dist^2 is (q^2 + o^2) / |t|^2 and its ts is Tc / |t|^2.  The terms of
+// pixel_grad are constants of the line times these sums:
+//   s[0] = sum h q,  s[1] = sum h q Tc,  s[2] = sum g k,
+//   s[3] = sum h o,  s[4] = sum h o Tc   (zero for columns within the ends)
+// with h = g f, k = f u (u = dist^2 / w^2, ku = 1 / (|t| w)^2); triangular
+// profiles: h = g / r, k = r = sqrt(q^2 + o^2).
+template <int K>
+__device__ __forceinline__ void add_inside(double *s, float g, double q, double T, double ku)
 {
-    const float LL = L.LL, ea = L.ea, nlim = L.nlim;
-    const int a = L.axis, b = 1 - a;
-    auto visit = [&](int s, float T, float N) {
-        if (!(err_fast(L, LL, ea, T, N) <= 1.0f)) return;
-        const int x = (a == 0) ? c : s, y = (a == 0) ? s : c;
-        const float gv = gt[(y - Y0) * tile_pitch<TILE>() + (x - X0)];
-        if (gv != 0.0f) pixel_grad<K>(C, x, y, (double)gv, acc);
-    };
-    if (cs >= s_lo && cs < s_hi) visit(cs, Te0, Ne0);
-    const int sb = pick(L.st, b);
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-        const int dir = half ? -sb : sb;
-        const float dT = (dir > 0) ? pick(L.t, b) : -pick(L.t, b), dN = (dir > 0) ? pick(L.nv, b) : -pick(L.nv, b);
-        const int nsteps = (dir > 0) ? (s_hi - 1 - cs) : (cs - s_lo);
-        const int jin = (dir > 0) ? (s_lo - cs) : (cs - s_hi + 1);
-        float Te = Te0, Ne = Ne0;
-        for (int j = 1; j <= nsteps; j++) {
-            Te += dT;
-            Ne += dN;
-            if (!(__builtin_fabsf(Ne) < nlim)) break;
-            if (j >= jin) visit(cs + j * dir, Te, Ne);
-        }
+    const double gv = (double)g;
+    if constexpr (K == K_TRIANGULAR) {
+        const double p = (q > 0.0) ? gv : ((q < 0.0) ? -gv : 0.0);
+        s[0] += p;
+        s[1] = __builtin_fma(p, T, s[1]);
+        s[2] = __builtin_fma(gv, __builtin_fabs(q), s[2]);
+    } else {
+        const double u = q * q * ku;
+        double h = gv;
+        if constexpr (K == K_BIWEIGHT) h = __builtin_fma(-u, gv, gv);
+        if constexpr (K == K_GAUSSIAN) h = gv * ::exp(-4.5 * u);
+        const double p = h * q;
+        s[0] += p;
+        s[1] = __builtin_fma(p, T, s[1]);
+        s[2] = __builtin_fma(h, u, s[2]);
     }
 }
 
+template <int K>
+__device__ __forceinline__ void add_clamped(double *s, float g, double q, double T, double mag, double ku)
+{
+    const double gv = (double)g;
+    const double Tc = (T < 0.0) ? 0.0 : ((T > mag) ? mag : T), o = T - Tc;
+    const double r2 = __builtin_fma(q, q, o * o);
+    double h = gv, k;
+    if constexpr (K == K_TRIANGULAR) {
+        k = sqrt(r2);
+        h = (k > 0.0) ? gv / k : 0.0;
+        s[2] = __builtin_fma(gv, k, s[2]);
+    } else {
+        k = r2 * ku;
+        if constexpr (K == K_BIWEIGHT) h = __builtin_fma(-k, gv, gv);
+        if constexpr (K == K_GAUSSIAN) h = gv * ::exp(-4.5 * k);
+        s[2] = __builtin_fma(h, k, s[2]);
+    }
+    const double p = h * q, e = h * o;
+    s[0] += p;
+    s[1] = __builtin_fma(p, Tc, s[1]);
+    s[3] += e;
+    s[4] = __builtin_fma(e, Tc, s[4]);
+}
+
+// x of the lane at a fixed place of the row of 16 (CTRL: a DPP control), and the
+// sum of x over the SEG lanes of an item, in the same order in every lane
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <int SEG>
+__device__ __forceinline__ double item_sum(double x)
+{
+    static_assert(SEG == 8 || SEG == 16, "lanes of one row");
+    x += dpp_move<0xb1>(x);    // lanes 1, 0, 3, 2
+    x += dpp_move<0x4e>(x);    // lanes 2, 3, 0, 1
+    x += dpp_move<0x141>(x);   // mirrored within 8
+    if constexpr (SEG == 16) x += dpp_move<0x140>(x);   // mirrored within 16
+    return x;
+}
+
+// Per-item record of k_adjoint_fast in LDS.
+struct AdjRec {
+    double q0, T0;      // q and T at column 0 and short-axis coordinate 0
+    double la, lb;      // t_a, t_b (exact: from the end points)
+    double ku;          // 1 / (|t| w)^2
+    float inv;          // 1 / nb: nb is the normal error's change per +1 along the short axis
+    float hm, hp;       // half height of the band in steps: decided inside, decided outside
+    float cap, far;     // interior columns: cap < Te < far
+    int32_t base;       // LDS index of column 0 at short-axis coordinate 0
+    int32_t line;
+    int32_t meta;       // FR_* bits, columns from bit 16
+};
+
+// Adjoint of the float lines.  One workgroup per tile, NT / 64 independent
+// waves (the only barrier is after the tile of dLoss/dImage is in LDS), each
+// with chunks of up to CHW items: phase 1 replays one item's walk per lane;
+// phase 2a gives a lane one interior column, its pixels counted beforehand as
+// in the tile kernel of the draws and its terms reduced to three sums;
+// phase 2b takes the columns within the width of a line's end from a compacted
+// list, one half per lane, with the error of every pixel and the terms of
+// pixels beyond the end.  Lane i collects item i: the columns of phase 2a in a
+// fixed tree, those of phase 2b in their order, so a partial does not depend on
+// where its item stands in the list.
+//
+// Bound by vector instruction issue: the gradient of 160 000 biweight lines
+// (widths 2 to 6, 32 frames of 1024^2) takes 620 us, of which its 313 M wave
+// instructions need 510 at the issue rate; with one lane per column and the
+// full terms (25 double operations, two divisions per column) 983 us.  Chunks of
+// 16 items leave half the lanes of phase 2b idle (838 against 688 us with 32,
+// before the sums of phase 2b were shared with 2a); 192 / SEG fill four
+// workgroups of 40 KB per CU.
+template <int K, int TILE, int SEG, int NT, int CHW>
+__global__ void __launch_bounds__(NT, 4)
+k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, Geometry g,
+               const int *__restrict__ tile_off, const int2 *__restrict__ pairs,
+               const Segment<float> *__restrict__ segs, const LineSetup<float> *__restrict__ setup,
+               const LineLite *__restrict__ lite, const int *__restrict__ slot_base, float max_val,
+               double *__restrict__ partial, int *__restrict__ flags)
+{
+    constexpr int NW = NT / 64, PX = TILE * TILE, PITCH = tile_pitch<TILE>(), NREC = CHW * SEG;
+    constexpr int IPR = 64 / SEG;   // items per round of phase 2a
+    constexpr int BATCH = 32;       // columns per round of phase 2b
+    static_assert(CHW <= 64 && NREC <= 256, "one lane per item, column numbers of 8 bits");
+    union Sums {   // per wave: the items' sums of phase 2a, then the columns' of phase 2b
+        double item[CHW][3];
+        double col[BATCH][5];
+    };
+    __shared__ float gt[TILE * PITCH];
+    __shared__ int32_t rS[NW][NREC];
+    __shared__ float rN[NW][NREC], rT[NW][NREC];
+    __shared__ AdjRec arec[NW][CHW];
+    __shared__ uint8_t caps[NW][NREC];
+    __shared__ Sums sums[NW];
+
+    const int tile = blockIdx.x;
+    const int beg = tile_off[tile * LIST_SUBS], end = tile_off[(tile + 1) * LIST_SUBS];
+    // a plan whose last draw failed (capacity, bad idxs) has no valid lists
+    const int fl = *flags;
+    if (fl || beg == end) return;
+    int64_t f;
+    int tx, ty;
+    tile_coords(g, tile, f, tx, ty);
+    const int X0 = tx * TILE, Y0 = ty * TILE;
+    const int X1 = min(X0 + TILE, g.W), Y1 = min(Y0 + TILE, g.H);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // the tile of dLoss/dImage: every load issued before the LDS writes
+    const float *const fg = grad + ((f * g.H + Y0) * (int64_t)g.W + X0);
+    constexpr int PP = PX / NT;
+    float gv[PP];
+#pragma unroll
+    for (int j = 0; j < PP; j++) {
+        const int i = tid + j * NT;
+        const int y = i / TILE, x = i % TILE;
+        gv[j] = (y < Y1 - Y0 && x < X1 - X0) ? __builtin_nontemporal_load(fg + ((int64_t)y * g.W + x)) : 0.0f;
+    }
+    // equal chunks, the same number of turns for every wave
+    const int turns = (end - beg + NW * CHW - 1) / (NW * CHW);
+    const int size = (end - beg + turns * NW - 1) / (turns * NW);
+    Segment<float> sg;
+    LineLite L;
+    float ln[5];
+    int sbase;
+    auto take = [&](const int2 &it) {
+        sg = segs[it.x];
+        L = lite[it.y];
+        sbase = slot_base[it.x];
+        for (int k = 0; k < 5; k++) ln[k] = lines[5 * (int64_t)it.y + k];
+    };
+    // (lanes without an item load the list's last)
+    take(pairs[min(beg + wave * size + lane, end - 1)]);
+#pragma unroll
+    for (int j = 0; j < PP; j++) {
+        const int i = tid + j * NT;
+        gt[(i / TILE) * PITCH + (i % TILE)] = gv[j];
+    }
+    __syncthreads();
+
+    int32_t *const wS = rS[wave];
+    float *const wN = rN[wave], *const wT = rT[wave];
+    AdjRec *const wR = arec[wave];
+    uint8_t *const wC = caps[wave];
+    Sums &wX = sums[wave];
+    const uint64_t below = (1ull << lane) - 1ull;
+
+    for (int t = 0; t < turns; t++) {
+        const int first = beg + (t * NW + wave) * size;
+        const int n = min(size, end - first);
+        if (n <= 0) break;
+        const int2 np = pairs[min(first + NW * size + lane, end - 1)];   // the next turn's items
+        // phase 1 (as in k_tiles_fast)
+        const bool ax = L.meta & FR_AXIS;
+        const double la = (double)ln[ax ? 3 : 2] - (double)ln[ax ? 1 : 0];
+        const double lb = (double)ln[ax ? 2 : 3] - (double)ln[ax ? 0 : 1];
+        const double inv_mag = 1.0 / (la * la + lb * lb), inv_w = 1.0 / (double)ln[4];
+        const int64_t out_at = (int64_t)sbase + ((ax ? tx : ty) - (sg.lo >> g.tile_log));
+        if (lane < n) {
+            const bool pa = L.meta & FR_SA, pb = L.meta & FR_SB;
+            const bool p0 = ax ? pb : pa, p1 = ax ? pa : pb;   // steps along x and y
+            const float t0 = L.t[0], t1 = L.t[1];
+            const float nb = ax ? t1 : -t0, na = __builtin_fabsf(nb);
+            const int c0 = ax ? sg.c[1] : sg.c[0];
+            const double ra = (double)c0 - (double)ln[ax ? 1 : 0], rb = -(double)ln[ax ? 0 : 1];
+            AdjRec R;
+            R.q0 = ra * lb - rb * la;
+            R.T0 = ra * la + rb * lb;
+            R.la = la;
+            R.lb = lb;
+            R.ku = inv_mag * (inv_w * inv_w);
+            R.inv = __builtin_amdgcn_rcpf(nb);
+            const float h = L.nlim * __builtin_fabsf(R.inv), tol = h * (8e-6f + 3e-7f * h);
+            R.hm = h - tol;
+            R.hp = h + tol;
+            // (the walk's tangent error drifts from the exact one: a margin keeps T within [0, |t|^2])
+            const float drift = L.LL * 6e-8f * (4.0f * __builtin_amdgcn_sqrtf(L.LL) + 64.0f);
+            R.cap = ((L.meta & FR_SAFE) && L.nlim < 64.0f * na) ? L.cap + drift : __builtin_inff();
+            R.far = L.LL - (L.cap + drift);
+            R.base = ax ? (c0 - Y0) * PITCH - X0 : (c0 - X0) - Y0 * PITCH;
+            R.line = sg.line;
+            R.meta = L.meta | (sg.ncols << 16);
+            wR[lane] = R;
+            const float dx = p0 ? t1 : -t1, dy = p1 ? -t0 : t0;
+            const float ux = p0 ? t0 : -t0, uy = p1 ? t1 : -t1;
+            const int sb = pb ? 1 : -1;
+            float Te = sg.Te, Ne = sg.Ne;
+            int s = ax ? sg.c[0] : sg.c[1];
+            int slot = lane * SEG, it = 0;
+            const int stop = slot + sg.ncols;
+            for (; slot < stop && it < 4 * SEG + 16; it++) {
+                wS[slot] = s;
+                wN[slot] = Ne;
+                wT[slot] = Te;
+                const float ex = Ne + dx, ey = Ne + dy, exy = ex + dy;
+                const bool yb = __builtin_fabsf(ey) < __builtin_fabsf(ex);
+                const float m = yb ? ey : ex;
+                const bool both = __builtin_fabsf(exy) < __builtin_fabsf(m);
+                const bool nx = !yb || both, ny = yb || both;
+                Te += nx ? ux : 0.0f;
+                Te += ny ? uy : 0.0f;
+                Ne = both ? exy : m;
+                s += (ax ? nx : ny) ? sb : 0;
+                slot += (ax ? ny : nx) ? 1 : 0;
+            }
+            if (slot < stop) atomicOr(flags, FLAG_STUCK);   // still walking after the step budget
+        }
+        take(np);
+        wave_sync();
+        // phase 2a
+        int ncap = 0, cap_lo = 0, cap_hi = 0;   // lane i: item i's columns in the list
+        for (int u0 = 0; u0 < n * SEG; u0 += 64) {
+            const int u = u0 + lane, i = u / SEG, k = u % SEG;
+            bool cap = false;
+            double v[3] = {0.0, 0.0, 0.0};
+            if (u < n * SEG) {
+                const AdjRec &R = wR[i];
+                const int meta = R.meta;
+                if (k < (meta >> 16)) {
+                    const float Te = wT[u], Ne = wN[u];
+                    const float jc = -Ne * R.inv;
+                    cap = !(Te > R.cap && Te < R.far && __builtin_fabsf(jc) <= 1.0f);
+                    if (!cap) {
+                        const int cs = wS[u];
+                        const bool rx = meta & FR_AXIS;
+                        const int kk = (meta & FR_SA) ? k : -k;
+                        const int sst = rx ? 1 : PITCH;
+                        const int at = R.base + kk * (rx ? PITCH : 1) + cs * sst;
+                        const int w0 = (rx ? X0 : Y0) - cs, w1 = (rx ? X1 : Y1) - 1 - cs;
+                        const double ra = R.la, rb = R.lb, ku = R.ku;
+                        const double q0 = __builtin_fma((double)kk, rb, __builtin_fma(-(double)cs, ra, R.q0));
+                        const double T0 = __builtin_fma((double)kk, ra, __builtin_fma((double)cs, rb, R.T0));
+                        const float f0 = __builtin_ceilf(jc - R.hm), f1 = __builtin_floorf(jc + R.hm);
+                        const int j0 = (int)f0, j1 = (int)f1;
+                        const int ja = max(j0, w0), m = min(j1, w1) - ja + 1;
+                        double jd = (double)ja, sums3[3] = {0.0, 0.0, 0.0};
+                        const float *p = gt + (at + ja * sst);
+                        for (int j = 0; j < m; j++) {
+                            // (sums3[1] with j in place of T)
+                            add_inside<K>(sums3, *p, __builtin_fma(-jd, ra, q0), jd, ku);
+                            jd += 1.0;
+                            p += sst;
+                        }
+                        // the undecided pixels next to the band's ends (fill_interior)
+                        const float g0 = __builtin_ceilf(jc - R.hp), g1 = __builtin_floorf(jc + R.hp);
+                        if (g0 < f0 || g1 > f1) {
+                            const LineSetup<float> G = setup[R.line];
+                            const float nb = rx ? G.nv[0] : G.nv[1];
+                            for (int j = (int)g0; j <= (int)g1; j++) {
+                                if ((j >= j0 && j <= j1) || j < w0 || j > w1) continue;
+                                float N = Ne;
+                                const float dN = (j < 0) ? -nb : nb;
+                                for (int z = 0; z < abs(j); z++) N += dN;
+                                if (j != 0 && !(__builtin_fabsf(N) < G.nlim)) continue;
+                                if (err_fast(G, G.LL, G.ea, 0.0f, N) <= 1.0f)
+                                    add_inside<K>(sums3, gt[at + j * sst], __builtin_fma(-(double)j, ra, q0), (double)j,
+                                                  ku);
+                            }
+                        }
+                        v[0] = sums3[0];
+                        v[1] = __builtin_fma(T0, sums3[0], rb * sums3[1]);
+                        v[2] = sums3[2];
+                    }
+                }
+            }
+            const uint64_t cm = __ballot(cap);
+            if (cap) wC[ncap + __popcll(cm & below)] = (uint8_t)u;
+            // the SEG lanes of one item hold its columns
+#pragma unroll
+            for (int j = 0; j < 3; j++) v[j] = item_sum<SEG>(v[j]);
+            if (k == 0 && i < CHW)
+                for (int j = 0; j < 3; j++) wX.item[i][j] = v[j];
+            if (lane / IPR == u0 / 64) {
+                const int from = (lane % IPR) * SEG;
+                cap_lo = ncap + __popcll(cm & ((1ull << from) - 1ull));
+                cap_hi = cap_lo + __popcll((cm >> from) & ((1ull << SEG) - 1ull));
+            }
+            ncap += __popcll(cm);
+        }
+        wave_sync();
+        double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};   // lane i: item i's sums
+        if (lane < n)
+            for (int j = 0; j < 3; j++) acc[j] = wX.item[lane][j];
+        // phase 2b
+        for (int v0 = 0; v0 < ncap; v0 += BATCH) {
+            wave_sync();
+            const int v = v0 + (lane >> 1), half = lane & 1;
+            double w[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+            if (v < ncap) {
+                const int slot = wC[v], i = slot / SEG, k = slot % SEG;
+                const AdjRec &R = wR[i];
+                const int meta = R.meta, cs = wS[slot];
+                const LineSetup<float> &G = setup[R.line];
+                const bool rx = meta & FR_AXIS;
+                const int kk = (meta & FR_SA) ? k : -k, sst = rx ? 1 : PITCH;
+                const int at = R.base + kk * (rx ? PITCH : 1);   // (at short-axis coordinate 0)
+                const int s_lo = rx ? X0 : Y0, s_hi = rx ? X1 : Y1;
+                const double ra = R.la, rb = R.lb, ku = R.ku, mag = ra * ra + rb * rb;
+                const double qk = __builtin_fma((double)kk, rb, R.q0), Tk = __builtin_fma((double)kk, ra, R.T0);
+                auto add = [&](int s) {
+                    const float p = gt[at + s * sst];
+                    const double sd = (double)s;
+                    if (p != 0.0f)
+                        add_clamped<K>(w, p, __builtin_fma(-sd, ra, qk), __builtin_fma(sd, rb, Tk), mag, ku);
+                };
+                if (meta & FR_SAFE) {
+                    // the centre goes with half 0
+                    const float LL = G.LL, ea = G.ea, nlim = G.nlim;
+                    const int sb = (meta & FR_SB) ? 1 : -1, dir = half ? -sb : sb;
+                    const float tb = rx ? G.t[0] : G.t[1], nb = rx ? G.nv[0] : G.nv[1];
+                    const float dT = (dir > 0) ? tb : -tb, dN = (dir > 0) ? nb : -nb;
+                    float Te = wT[slot], Ne = wN[slot];
+                    if (half == 0 && cs >= s_lo && cs < s_hi && err_fast(G, LL, ea, Te, Ne) <= 1.0f) add(cs);
+                    const int nsteps = (dir > 0) ? (s_hi - 1 - cs) : (cs - s_lo);
+                    const int jin = (dir > 0) ? (s_lo - cs) : (cs - s_hi + 1);
+                    for (int j = 1; j <= nsteps; j++) {
+                        Te += dT;
+                        Ne += dN;
+                        if (!(__builtin_fabsf(Ne) < nlim)) break;
+                        if (j >= jin && err_fast(G, LL, ea, Te, Ne) <= 1.0f) add(cs + j * dir);
+                    }
+                } else if (half == 0) {
+                    const ColRec<float> cr = {cs, wT[slot], wN[slot]};
+                    fill_column(G, cr, s_lo, s_hi, [&](int s, float Te, float Ne) {
+                        if (err_of(G, Te, Ne) <= 1.0f) add(s);
+                    });
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 5; j++) {
+                w[j] += dpp_move<0xb1>(w[j]);
+                if (half == 0) wX.col[lane >> 1][j] = w[j];
+            }
+            wave_sync();
+            for (int z = max(cap_lo, v0); z < min(cap_hi, v0 + BATCH); z++)
+#pragma unroll
+                for (int j = 0; j < 5; j++) acc[j] += wX.col[z - v0][j];
+        }
+        // the constants of the sums, and out
+        if (lane < n) {
+            const double mv = (double)max_val;
+            double ch, cw;   // GradConst's cc, cw with the powers of |t|
+            if constexpr (K == K_TRIANGULAR) {
+                const double inv_len = sqrt(inv_mag);
+                ch = mv * inv_w * inv_len;
+                cw = mv * (inv_w * inv_w) * inv_len;
+            } else {
+                constexpr double kp = (K == K_BIWEIGHT) ? -1.875
+                                                        : ((K == K_PARABOLIC) ? -0.75 : -4.5 * 0.3989422804014327);
+                ch = -2.0 * kp * mv * (inv_w * inv_w) * inv_mag;
+                cw = -2.0 * kp * mv * inv_w;
+            }
+            // (no product of an infinite constant with an empty sum)
+            auto times = [](double c, double x) { return (x != 0.0) ? c * x : 0.0; };
+            const double e1 = times(ch, acc[0]), e2 = times(ch * inv_mag, acc[1]);
+            const double o1 = times(ch, acc[3]), o2 = times(ch * inv_mag, acc[4]);
+            const double a1 = times(lb, e1) + times(la, o1), b1 = times(lb, o1) - times(la, e1);
+            const double a2 = times(lb, e2) + times(la, o2), b2 = times(lb, o2) - times(la, e2);
+            double *p = partial + 5 * out_at;
+            p[0] = ax ? b1 : a1;
+            p[1] = ax ? a1 : b1;
+            p[2] = ax ? b2 : a2;
+            p[3] = ax ? a2 : b2;
+            p[4] = times(cw, acc[2]);
+        }
+        wave_sync();
+    }
+}
+
+// Adjoint of the double lines: one lane per column, the full terms.
 template <typename T, int K, int TILE, int SEG, int NT, int CH>
 __global__ void __launch_bounds__(NT)
 k_adjoint_tiles(const T *__restrict__ grad, const T *__restrict__ lines, Geometry g, const int *__restrict__ tile_off,
@@ -1008,23 +1379,13 @@ k_adjoint_tiles(const T *__restrict__ grad, const T *__restrict__ lines, Geometr
                     const int c = pick(sg.c, a) + k * pick(L.st, a);
                     const int s_lo = (a == 0) ? Y0 : X0, s_hi = (a == 0) ? Y1 : X1;
                     const GradConst C = grad_const<K>(L, lines + 5 * (int64_t)hdr[wave][i].line, max_val);
-                    bool done = false;
-                    if constexpr (sizeof(T) == 4) {
-                        if (L.safe) {
-                            adj_column_fast<K, TILE>(L, C, (const float *)gt, cr.s, cr.Te, cr.Ne, c, X0, Y0, s_lo,
-                                                     s_hi, acc);
-                            done = true;
-                        }
-                    }
-                    if (!done) {
-                        fill_column(L, cr, s_lo, s_hi, [&](int s, T Te, T Ne) {
-                            const T err = err_of(L, Te, Ne);
-                            if (!(err <= T(1))) return;
-                            const int x = (a == 0) ? c : s, y = (a == 0) ? s : c;
-                            const T gv = gt[(y - Y0) * tile_pitch<TILE>() + (x - X0)];
-                            if (gv != T(0)) pixel_grad<K>(C, x, y, (double)gv, acc);
-                        });
-                    }
+                    fill_column(L, cr, s_lo, s_hi, [&](int s, T Te, T Ne) {
+                        const T err = err_of(L, Te, Ne);
+                        if (!(err <= T(1))) return;
+                        const int x = (a == 0) ? c : s, y = (a == 0) ? s : c;
+                        const T gv = gt[(y - Y0) * tile_pitch<TILE>() + (x - X0)];
+                        if (gv != T(0)) pixel_grad<K>(C, x, y, (double)gv, acc);
+                    });
                 }
             }
             // the SEG lanes of one item hold its columns: reduce them in a fixed tree
@@ -1878,18 +2239,21 @@ static void launch_adjoint(const T *grad, const T *lines, const SegmentPlan<T> &
                            T max_val, double *partial, hipStream_t st)
 {
     constexpr int NT = 256;
-    if (P.g.tile == 64 && P.g.seg == 16)
-        k_adjoint_tiles<T, K, 64, 16, NT, 16><<<(unsigned)P.n_tiles, NT, 0, st>>>(
-            grad, lines, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, slot_base, max_val, partial, P.flags.ptr);
-    else if (P.g.tile == 64)
-        k_adjoint_tiles<T, K, 64, 8, NT, 32><<<(unsigned)P.n_tiles, NT, 0, st>>>(
-            grad, lines, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, slot_base, max_val, partial, P.flags.ptr);
-    else if (P.g.seg == 16)
-        k_adjoint_tiles<T, K, 32, 16, NT, 16><<<(unsigned)P.n_tiles, NT, 0, st>>>(
-            grad, lines, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, slot_base, max_val, partial, P.flags.ptr);
-    else
-        k_adjoint_tiles<T, K, 32, 8, NT, 32><<<(unsigned)P.n_tiles, NT, 0, st>>>(
-            grad, lines, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, slot_base, max_val, partial, P.flags.ptr);
+    auto run = [&](auto tile, auto seg) {
+        if constexpr (sizeof(T) == 4)
+            k_adjoint_fast<K, tile(), seg(), NT, 192 / seg()><<<(unsigned)P.n_tiles, NT, 0, st>>>(
+                grad, lines, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, P.lite.ptr, slot_base, max_val,
+                partial, P.flags.ptr);
+        else
+            k_adjoint_tiles<T, K, tile(), seg(), NT, 256 / seg()><<<(unsigned)P.n_tiles, NT, 0, st>>>(
+                grad, lines, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, slot_base, max_val, partial,
+                P.flags.ptr);
+    };
+    using std::integral_constant;
+    if (P.g.tile == 64 && P.g.seg == 16) run(integral_constant<int, 64>{}, integral_constant<int, 16>{});
+    else if (P.g.tile == 64) run(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+    else if (P.g.seg == 16) run(integral_constant<int, 32>{}, integral_constant<int, 16>{});
+    else run(integral_constant<int, 32>{}, integral_constant<int, 8>{});
 }
 
 template <typename T, typename I>
