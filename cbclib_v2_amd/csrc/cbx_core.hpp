@@ -107,6 +107,7 @@ struct alignas(16) LineSetup {
     int8_t valid;  // 0: the line emits nothing
     int8_t safe;   // 1: quotients of its errors by len cannot be subnormal (see line_setup)
     int8_t kid;    // profile of the line (K_BIWEIGHT .. K_TRIANGULAR)
+    int8_t sub;    // sub-list of its items in a tile's list (list_class)
     T e0[2];       // tangent and normal errors at m0
     T p0[2];       // first end point (for the adjoint's closed-form derivatives)
 };
