@@ -998,6 +998,7 @@ struct AdjRec {
     float hm, hp;       // half height of the band in steps: decided inside, decided outside
     float cap, far;     // interior columns: cap < Te < far
     int32_t base;       // LDS index of column 0 at short-axis coordinate 0
+    int32_t s0;         // short-axis position at column 0
     int32_t line;
     int32_t meta;       // FR_* bits, columns from bit 16
 };
@@ -1037,8 +1038,7 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
         double col[BATCH][5];
     };
     __shared__ float gt[TILE * PITCH];
-    __shared__ int32_t rS[NW][NREC];
-    __shared__ float rN[NW][NREC], rT[NW][NREC];
+    __shared__ WaveCols<NREC> cols[NW];
     __shared__ AdjRec arec[NW][CHW];
     __shared__ uint8_t caps[NW][NREC];
     __shared__ Sums sums[NW];
@@ -1087,8 +1087,7 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
     }
     __syncthreads();
 
-    int32_t *const wS = rS[wave];
-    float *const wN = rN[wave], *const wT = rT[wave];
+    WaveCols<NREC> &wK = cols[wave];
     AdjRec *const wR = arec[wave];
     uint8_t *const wC = caps[wave];
     Sums &wX = sums[wave];
@@ -1106,10 +1105,7 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
         const double inv_mag = 1.0 / (la * la + lb * lb), inv_w = 1.0 / (double)ln[4];
         const int64_t out_at = (int64_t)sbase + ((ax ? tx : ty) - (sg.lo >> g.tile_log));
         if (lane < n) {
-            const bool pa = L.meta & FR_SA, pb = L.meta & FR_SB;
-            const bool p0 = ax ? pb : pa, p1 = ax ? pa : pb;   // steps along x and y
-            const float t0 = L.t[0], t1 = L.t[1];
-            const float nb = ax ? t1 : -t0, na = __builtin_fabsf(nb);
+            const float nb = ax ? L.t[1] : -L.t[0], na = __builtin_fabsf(nb);
             const int c0 = ax ? sg.c[1] : sg.c[0];
             const double ra = (double)c0 - (double)ln[ax ? 1 : 0], rb = -(double)ln[ax ? 0 : 1];
             AdjRec R;
@@ -1127,32 +1123,11 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
             R.cap = ((L.meta & FR_SAFE) && L.nlim < 64.0f * na) ? L.cap + drift : __builtin_inff();
             R.far = L.LL - (L.cap + drift);
             R.base = ax ? (c0 - Y0) * PITCH - X0 : (c0 - X0) - Y0 * PITCH;
+            R.s0 = ax ? sg.c[0] : sg.c[1];
             R.line = sg.line;
             R.meta = L.meta | (sg.ncols << 16);
             wR[lane] = R;
-            const float dx = p0 ? t1 : -t1, dy = p1 ? -t0 : t0;
-            const float ux = p0 ? t0 : -t0, uy = p1 ? t1 : -t1;
-            const int sb = pb ? 1 : -1;
-            float Te = sg.Te, Ne = sg.Ne;
-            int s = ax ? sg.c[0] : sg.c[1];
-            int slot = lane * SEG, it = 0;
-            const int stop = slot + sg.ncols;
-            for (; slot < stop && it < 4 * SEG + 16; it++) {
-                wS[slot] = s;
-                wN[slot] = Ne;
-                wT[slot] = Te;
-                const float ex = Ne + dx, ey = Ne + dy, exy = ex + dy;
-                const bool yb = __builtin_fabsf(ey) < __builtin_fabsf(ex);
-                const float m = yb ? ey : ex;
-                const bool both = __builtin_fabsf(exy) < __builtin_fabsf(m);
-                const bool nx = !yb || both, ny = yb || both;
-                Te += nx ? ux : 0.0f;
-                Te += ny ? uy : 0.0f;
-                Ne = both ? exy : m;
-                s += (ax ? nx : ny) ? sb : 0;
-                slot += (ax ? ny : nx) ? 1 : 0;
-            }
-            if (slot < stop) atomicOr(flags, FLAG_STUCK);   // still walking after the step budget
+            if (!replay_columns<SEG>(wK, L, sg, lane * SEG, sg.ncols)) atomicOr(flags, FLAG_STUCK);
         }
         take(np);
         wave_sync();
@@ -1166,11 +1141,11 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
                 const AdjRec &R = wR[i];
                 const int meta = R.meta;
                 if (k < (meta >> 16)) {
-                    const float Te = wT[u], Ne = wN[u];
+                    const float Te = wK.T[u], Ne = wK.N[u];
                     const float jc = -Ne * R.inv;
                     cap = !(Te > R.cap && Te < R.far && __builtin_fabsf(jc) <= 1.0f);
                     if (!cap) {
-                        const int cs = wS[u];
+                        const int cs = R.s0 + wK.centre(u);
                         const bool rx = meta & FR_AXIS;
                         const int kk = (meta & FR_SA) ? k : -k;
                         const int sst = rx ? 1 : PITCH;
@@ -1238,7 +1213,7 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
             if (v < ncap) {
                 const int slot = wC[v], i = slot / SEG, k = slot % SEG;
                 const AdjRec &R = wR[i];
-                const int meta = R.meta, cs = wS[slot];
+                const int meta = R.meta, cs = R.s0 + wK.centre(slot);
                 const LineSetup<float> &G = setup[R.line];
                 const bool rx = meta & FR_AXIS;
                 const int kk = (meta & FR_SA) ? k : -k, sst = rx ? 1 : PITCH;
@@ -1258,7 +1233,7 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
                     const int sb = (meta & FR_SB) ? 1 : -1, dir = half ? -sb : sb;
                     const float tb = rx ? G.t[0] : G.t[1], nb = rx ? G.nv[0] : G.nv[1];
                     const float dT = (dir > 0) ? tb : -tb, dN = (dir > 0) ? nb : -nb;
-                    float Te = wT[slot], Ne = wN[slot];
+                    float Te = wK.T[slot], Ne = wK.N[slot];
                     if (half == 0 && cs >= s_lo && cs < s_hi && err_fast(G, LL, ea, Te, Ne) <= 1.0f) add(cs);
                     const int nsteps = (dir > 0) ? (s_hi - 1 - cs) : (cs - s_lo);
                     const int jin = (dir > 0) ? (s_lo - cs) : (cs - s_hi + 1);
@@ -1269,7 +1244,7 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
                         if (j >= jin && err_fast(G, LL, ea, Te, Ne) <= 1.0f) add(cs + j * dir);
                     }
                 } else if (half == 0) {
-                    const ColRec<float> cr = {cs, wT[slot], wN[slot]};
+                    const ColRec<float> cr = {cs, wK.T[slot], wK.N[slot]};
                     fill_column(G, cr, s_lo, s_hi, [&](int s, float Te, float Ne) {
                         if (err_of(G, Te, Ne) <= 1.0f) add(s);
                     });

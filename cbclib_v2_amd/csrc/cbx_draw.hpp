@@ -183,6 +183,65 @@ __device__ __forceinline__ void fill_column(const LineSetup<T> &L, const ColRec<
     }
 }
 
+// A wave's column records in LDS: errors and centre (relative to the item's first
+// position along the short axis, in the low half of a word) of column u = slot.
+template <int NREC>
+struct WaveCols {
+    float N[NREC], T[NREC];
+    int32_t S[NREC];
+    __device__ __forceinline__ int centre(int u) const { return (int)*reinterpret_cast<const int16_t *>(&S[u]); }
+};
+
+// One lane replays one segment's walk and records its ncols columns from slot
+// `first` on; false if it does not end within the step budget.  A step per turn
+// of the loop; its column is recorded over and over until the step that leaves
+// it.  The loop is most of what a narrow line costs the tile kernels, so the
+// slot (as a byte offset) and the short-axis position share one register whose
+// increments along x and y are known before: 20 vector instructions a step, 31
+// with separate ones (962 000 lines in 16-column segments: tile kernel 2684 ->
+// 2540 us).
+template <int SEG, int NREC>
+__device__ __forceinline__ bool replay_columns(WaveCols<NREC> &w, const LineLite &L, const Segment<float> &sg,
+                                               int first, int ncols)
+{
+    static_assert(NREC * 4 <= 0xffff && 4 * SEG + 16 < 0x7fff, "two 16-bit halves");
+    const bool ax = L.meta & FR_AXIS, pa = L.meta & FR_SA, pb = L.meta & FR_SB;
+    const bool p0 = ax ? pb : pa, p1 = ax ? pa : pb;   // steps along x and y
+    const float t0 = L.t[0], t1 = L.t[1];
+    const float dx = p0 ? t1 : -t1, dy = p1 ? -t0 : t0;
+    const float ux = p0 ? t0 : -t0, uy = p1 ? t1 : -t1;
+    const uint32_t side = pb ? 0x10000u : 0xffff0000u;
+    const uint32_t ix = ax ? side : 4u, iy = ax ? 4u : side;
+    typedef __attribute__((address_space(3))) char lds_char;
+    typedef __attribute__((address_space(3))) float lds_float;
+    typedef __attribute__((address_space(3))) int16_t lds_short;
+    const uint32_t base = (uint32_t)(uintptr_t)(lds_char *)reinterpret_cast<char *>(&w);   // (LDS addresses: 16 bits)
+    float Te = sg.Te, Ne = sg.Ne;
+    uint32_t at = base + (uint32_t)first * 4u, o = at;
+    const uint32_t stop = o + (uint32_t)ncols * 4u;
+    int it = 0;
+    if (o < stop)
+        do {
+            *(lds_float *)(uintptr_t)o = Ne;
+            *(lds_float *)(uintptr_t)(o + NREC * 4) = Te;
+            *(lds_short *)(uintptr_t)(o + NREC * 8) = (int16_t)(at >> 16);
+            const float ex = Ne + dx, ey = Ne + dy, exy = ex + dy;
+            const bool yb = __builtin_fabsf(ey) < __builtin_fabsf(ex);
+            const float m = yb ? ey : ex;
+            const bool both = __builtin_fabsf(exy) < __builtin_fabsf(m);
+            const bool y_only = yb & !both, y = yb | both;
+            Te += y_only ? 0.0f : ux;
+            Te += y ? uy : 0.0f;
+            Ne = both ? exy : m;
+            at += y_only ? 0u : ix;
+            at += y ? iy : 0u;
+            o = at & 0xffffu;
+            it++;
+        } while ((o < stop) & (it < 4 * SEG + 16));
+    asm("" : "+v"(o));   // (compare once, here: not in every turn as part of the loop's masks)
+    return o >= stop;
+}
+
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 template <typename T>

@@ -66,9 +66,9 @@ __device__ __forceinline__ void tile_put(Acc *img, uint32_t *zb, int idx, V v)
 struct alignas(16) FillRec {
     float LL, ea, nlim;
     float tb, nb;     // tangent and normal components along the short axis b
-    int32_t c0;       // long-axis coordinate of the item's first column
+    int32_t c0;       // long-axis coordinate of the item's first column (k_tiles_fast: short-axis position there)
     int32_t line;
-    int32_t meta;     // FR_* bits, profile id in bits 8-15 (k_tiles_fast: mask of the interior columns in 16-31)
+    int32_t meta;     // FR_* bits, profile id in bits 8-15 (k_tiles_fast: columns from bit 16)
 };
 
 template <typename T>
@@ -476,20 +476,21 @@ __device__ __forceinline__ void fill_half(Acc *img, uint32_t *zb, const FillRec 
 template <int K>
 constexpr float interior_scale() { return K == K_GAUSSIAN ? 6.4921276840f : 1.0f; }   // exp(-4.5 u) = 2^(-k u)
 
+// (+ h: 0.5 where the value is then cut to an integer)
 template <int K>
-__device__ __forceinline__ float interior_value(float x, float c)
+__device__ __forceinline__ float interior_value(float x, float c, float h)
 {
     if constexpr (K == K_BIWEIGHT) {
         const float m = __builtin_fmaf(-x, x, 1.0f);
-        return c * (m * m);
+        return __builtin_fmaf(c * m, m, h);
     } else if constexpr (K == K_GAUSSIAN) {
-        return c * __builtin_amdgcn_exp2f(-(x * x));
+        return __builtin_fmaf(c, __builtin_amdgcn_exp2f(-(x * x)), h);
     } else if constexpr (K == K_PARABOLIC) {
-        return c * __builtin_fmaf(-x, x, 1.0f);
+        return __builtin_fmaf(-c * x, x, c + h);
     } else if constexpr (K == K_RECTANGULAR) {
-        return c;
+        return c + h;
     } else {
-        return __builtin_fmaf(-c, __builtin_fabsf(x), c);
+        return __builtin_fmaf(-c, __builtin_fabsf(x), c + h);
     }
 }
 
@@ -525,16 +526,16 @@ __device__ __forceinline__ void fill_interior(Acc *img, uint32_t *zb, const Inne
     const float x0 = Ne * I.rs;
     float jf = (float)a;
     Acc *q = img + (at + a * sstride);
-    for (int i = 0; i < n; i++) {
-        const float v = interior_value<K>(__builtin_fmaf(jf, I.dx, x0), c);
+    for (Acc *const e = q + max(n, 0) * sstride; q != e; q += sstride) {
+        const float x = __builtin_fmaf(jf, I.dx, x0);
         if constexpr (OV == 2) {
-            const uint32_t u = __float2uint_rn(v);
+            // (rounded to nearest: below 2^23 the sum with 0.5 is exact, above it the value is whole)
+            const uint32_t u = (uint32_t)interior_value<K>(x, c, 0.5f);
             atomicAdd(q, fast_positive<K>() ? u : max(1u, u));
         } else {
-            atomicMax(q, ord_enc(v));
+            atomicMax(q, ord_enc(interior_value<K>(x, c, 0.0f)));
         }
         jf += 1.0f;
-        q += sstride;
     }
     // the undecided pixels next to the band's ends
     const float g0 = __builtin_ceilf(jc - I.hp), g1 = __builtin_floorf(jc + I.hp);
@@ -564,12 +565,12 @@ __device__ __forceinline__ void fill_interior(Acc *img, uint32_t *zb, const Inne
 // overlaps another's fills.
 //
 // Bound by vector instruction issue: 64 frames of 2048^2 with 128 000 gaussian
-// lines take 0.59 ms (292 M wave instructions, 48 % of the issue rate; the
-// image alone is 0.46 ms at a copy's rate), 32 of 1024^2 with 160 000 biweight
-// lines 0.35 ms, 256 of 1024^2 with 962 000 lines of mixed profiles 2.8 ms.
-// With one tested, sequential loop per half column (k_tiles' fills) and one
-// wave replaying the walks of the whole workgroup the same took 0.66, 0.60 and
-// 5.1 ms: 60 % of the instructions were the loop's tests, masks and idle lanes.
+// lines take 0.59 ms (the image alone is 0.46 ms at a copy's rate), 32 of 1024^2
+// with 160 000 biweight lines 0.32 ms (170 M wave instructions, 0.28 ms at the
+// issue rate), 256 of 1024^2 with 962 000 lines of mixed profiles 2.5 ms (1311 M,
+// 2.1 ms).  With one tested, sequential loop per half column (k_tiles' fills) and
+// one wave replaying the walks of the whole workgroup the same took 0.66, 0.60
+// and 5.1 ms: 60 % of the instructions were the loop's tests, masks and idle lanes.
 template <int K, int OV, int TILE, int SEG, int NT, int CHW>
 __global__ void __launch_bounds__(NT, 4)
 k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_off, const int2 *__restrict__ pairs,
@@ -579,10 +580,13 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
     static_assert(OV == 1 || OV == 2, "max codes or fixed-point sums");
     static_assert(CHW <= 64, "one lane per item");
     constexpr int NW = NT / 64, PX = TILE * TILE, NREC = CHW * SEG;
-    __shared__ alignas(16) uint32_t img[PX];
-    __shared__ uint32_t zb[OV == 2 ? PX / 32 : 1];
-    __shared__ int32_t rS[NW][NREC];
-    __shared__ float rN[NW][NREC], rT[NW][NREC];
+    // Rows 4 words apart in the banks: the columns of a steep line add to one x in
+    // consecutive rows, which share a bank with a pitch of TILE (160 000 lines of
+    // widths 2 to 6: 333 -> 321 us; conflict cycles a third fewer).
+    constexpr int PITCH = TILE + 4, LP = TILE * PITCH;
+    __shared__ alignas(16) uint32_t img[LP];
+    __shared__ uint32_t zb[OV == 2 ? LP / 32 : 1];
+    __shared__ WaveCols<NREC> cols[NW];
     __shared__ FillRec frec[NW][CHW];
     __shared__ InnerRec irec[NW][CHW];
     __shared__ uint16_t caps[NW][NREC];
@@ -647,14 +651,13 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
     take(pairs[min(beg + wave * size + lane, end - 1)]);
     auto clear = [&]() {
         uint4 *p = reinterpret_cast<uint4 *>(img);
-        for (int i = tid; i < PX / 4; i += NT) p[i] = make_uint4(0u, 0u, 0u, 0u);
+        for (int i = tid; i < LP / 4; i += NT) p[i] = make_uint4(0u, 0u, 0u, 0u);
         if constexpr (OV == 2)
-            for (int i = tid; i < PX / 32; i += NT) zb[i] = 0u;
+            for (int i = tid; i < LP / 32; i += NT) zb[i] = 0u;
     };
     clear();
 
-    int32_t *const wS = rS[wave];
-    float *const wN = rN[wave], *const wT = rT[wave];
+    WaveCols<NREC> &wK = cols[wave];
     FillRec *const wR = frec[wave];
     InnerRec *const wI = irec[wave];
     uint16_t *const wC = caps[wave];
@@ -677,8 +680,6 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
             {
                 const int meta = L.meta;
                 const bool ax = meta & FR_AXIS;
-                const bool pa = meta & FR_SA, pb = meta & FR_SB;
-                const bool p0 = ax ? pb : pa, p1 = ax ? pa : pb;   // steps along x and y
                 const float t0 = L.t[0], t1 = L.t[1];
                 int dst = lane;
                 if constexpr (K == K_MIXED) {
@@ -701,7 +702,7 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                     R.nlim = L.nlim;
                     R.tb = ax ? t0 : t1;
                     R.nb = nb;
-                    R.c0 = ax ? sg.c[1] : sg.c[0];
+                    R.c0 = ax ? sg.c[0] : sg.c[1];
                     R.line = sg.line;
                     R.meta = meta | ((L.term < 0 ? sg.ncols : 0) << 16);
                     wR[dst] = R;
@@ -717,33 +718,10 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                     // (thicker lines: the running sums drift further from the estimate)
                     I.cap = ((meta & FR_SAFE) && L.nlim < 64.0f * na) ? L.cap : __builtin_inff();
                     I.far = L.LL - L.cap;
-                    I.base = ax ? (sg.c[1] - Y0) * TILE - X0 : (sg.c[0] - X0) - Y0 * TILE;
+                    I.base = ax ? (sg.c[1] - Y0) * PITCH - X0 : (sg.c[0] - X0) - Y0 * PITCH;
                     wI[dst] = I;
-                    // a step per turn of the loop; its column is recorded over
-                    // and over until the step that leaves it
-                    const float dx = p0 ? t1 : -t1, dy = p1 ? -t0 : t0;
-                    const float ux = p0 ? t0 : -t0, uy = p1 ? t1 : -t1;
-                    const int sb = pb ? 1 : -1;
-                    float Te = sg.Te, Ne = sg.Ne;
-                    int s = ax ? sg.c[0] : sg.c[1];
-                    int slot = dst * SEG, it = 0;
-                    const int stop = slot + (L.term < 0 ? sg.ncols : 0);   // (a line of k_tiles_terms: no columns)
-                    for (; slot < stop && it < 4 * SEG + 16; it++) {
-                        wS[slot] = s;
-                        wN[slot] = Ne;
-                        wT[slot] = Te;
-                        const float ex = Ne + dx, ey = Ne + dy, exy = ex + dy;
-                        const bool yb = __builtin_fabsf(ey) < __builtin_fabsf(ex);
-                        const float m = yb ? ey : ex;
-                        const bool both = __builtin_fabsf(exy) < __builtin_fabsf(m);
-                        const bool nx = !yb || both, ny = yb || both;
-                        Te += nx ? ux : 0.0f;
-                        Te += ny ? uy : 0.0f;
-                        Ne = both ? exy : m;
-                        s += (ax ? nx : ny) ? sb : 0;
-                        slot += (ax ? ny : nx) ? 1 : 0;
-                    }
-                    if (slot < stop) atomicOr(flags, FLAG_STUCK);   // still walking after the step budget
+                    const int ncols = (L.term < 0) ? sg.ncols : 0;   // (a line of k_tiles_terms: no columns)
+                    if (!replay_columns<SEG>(wK, L, sg, dst * SEG, ncols)) atomicOr(flags, FLAG_STUCK);
                 }
             }
             take(np);
@@ -758,15 +736,15 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                     const int meta = wR[i].meta;
                     if (k < (meta >> 16)) {
                         const InnerRec I = wI[i];
-                        const float Te = wT[u], Ne = wN[u];
+                        const float Te = wK.T[u], Ne = wK.N[u];
                         const float jc = -Ne * I.inv;
                         cap = !(Te > I.cap && Te < I.far && __builtin_fabsf(jc) <= 1.0f);
                         if (!cap) {
-                            const int cs = wS[u];
+                            const int cs = wR[i].c0 + wK.centre(u);
                             const bool ax = meta & FR_AXIS;
                             const int kk = (meta & FR_SA) ? k : -k;
-                            const int sst = ax ? 1 : TILE;
-                            const int at = I.base + kk * (ax ? TILE : 1) + cs * sst;
+                            const int sst = ax ? 1 : PITCH;
+                            const int at = I.base + kk * (ax ? PITCH : 1) + cs * sst;
                             const int w0 = (ax ? X0 : Y0) - cs, w1 = (ax ? X1 : Y1) - 1 - cs;
                             if constexpr (K == K_MIXED) {
 #define CBX_INNER(KK) fill_interior<KK, OV>(img, zb, I, wR + i, setup, cs, Ne, jc, at, sst, w0, w1, vscale)
@@ -794,13 +772,13 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                 const int slot = wC[u >> 1], half = u & 1;
                 const int i = slot / SEG, k = slot % SEG;
                 const FillRec R = wR[i];
-                const int cs = wS[slot];
+                const int cs = R.c0 + wK.centre(slot);
                 const int a = R.meta & FR_AXIS;
-                const int c = R.c0 + ((R.meta & FR_SA) ? k : -k);
+                const int kk = (R.meta & FR_SA) ? k : -k;
                 const int s_lo = a ? X0 : Y0, s_hi = a ? X1 : Y1;
-                const int sstride = a ? 1 : TILE;
-                const int cbase = a ? (c - Y0) * TILE : c - X0;
-                fill_half<K, OV>(img, zb, R, setup, cs, wT[slot], wN[slot], half, cbase, sstride, s_lo, s_hi, vscale);
+                const int sstride = a ? 1 : PITCH;
+                const int cbase = wI[i].base + kk * (a ? PITCH : 1) + s_lo * sstride;
+                fill_half<K, OV>(img, zb, R, setup, cs, wK.T[slot], wK.N[slot], half, cbase, sstride, s_lo, s_hi, vscale);
             }
             wave_sync();
         }
@@ -813,13 +791,15 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                 // all LDS reads first (4 pixels and their zero bits per read),
                 // then branch-free updates
                 const float p2 = __int_as_float((127 - F) << 23);   // 2^-F, F <= 31
+                const uint32_t l4 = (uint32_t)tid * 4 / TILE * PITCH + (uint32_t)tid * 4 % TILE;
                 uint4 acc[PP / 4];
                 uint32_t zw[PP / 4];
 #pragma unroll
                 for (int j = 0; j < PP / 4; j++) {
-                    const int i = (tid + j * NT) * 4;
-                    acc[j] = *reinterpret_cast<const uint4 *>(&img[i]);
-                    zw[j] = zb[i >> 5] >> (i & 31);
+                    constexpr int ROWS = NT * 4 / TILE * PITCH;
+                    static_assert(!PREF || ROWS % 32 == 0, "whole words of zero bits");
+                    acc[j] = *reinterpret_cast<const uint4 *>(&img[l4 + j * ROWS]);
+                    zw[j] = zb[l4 / 32 + j * (ROWS / 32)] >> (l4 % 32);
                 }
 #pragma unroll
                 for (int j = 0; j < PP / 4; j++) {
@@ -832,9 +812,9 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                 uint32_t acc[PP], z[PP];
 #pragma unroll
                 for (int j = 0; j < PP; j++) {
-                    const int i = tid + j * NT;
-                    acc[j] = img[i];
-                    z[j] = (zb[i >> 5] >> (i & 31)) & 1u;
+                    const uint32_t li = (uint32_t)tid / TILE * PITCH + (uint32_t)tid % TILE + j * (NT / TILE * PITCH);
+                    acc[j] = img[li];
+                    z[j] = (zb[li >> 5] >> (li & 31)) & 1u;
                 }
 #pragma unroll
                 for (int j = 0; j < PP; j++) {
@@ -847,7 +827,7 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                 for (int i = tid; i < PX; i += NT) {
                     const int y = i / TILE, x = i % TILE;
                     if (y >= Y1 - Y0 || x >= X1 - X0) continue;
-                    const double add = fix_value(img[i], zb, i, scale, max_val, has);
+                    const double add = fix_value(img[y * PITCH + x], zb, y * PITCH + x, scale, max_val, has);
                     float *o = to + ((int64_t)y * g.W + x);
                     if (has) *o = (float)((double)*o + add);
                 }
@@ -883,7 +863,7 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
             for (int j = 0; j < B; j++) {
                 const int i = i0 + j * NT;
                 const int y = i / TILE, x = i % TILE;
-                e[j] = img[i];
+                e[j] = img[y * PITCH + x];
                 o[j] = to[(int64_t)min(y, Y1 - Y0 - 1) * g.W + min(x, X1 - X0 - 1)];
             }
 #pragma unroll
