@@ -10,10 +10,11 @@
 //
 // Layout: the array is viewed as rows along its last axis (R rows of W
 // elements) and packed one bit per element into 64-bit words, Wq = ceil(W/64)
-// words per row, bits beyond W zero.  Rows of a multiple of 64 elements at
-// 16-byte alignment are packed and unpacked one word per thread with four
-// 16-byte accesses (bytes to bits by a carry-free product); other rows one
-// word per wave: lane l owns element 64 j + l, the word is one ballot.  A dilation round is one
+// words per row, bits beyond W zero.  Bytes become bits (and bits bytes) 16 per
+// thread by carry-free products.  Rows of a multiple of 64 elements at 16-byte
+// alignment are one run of words; of other rows the words are read at any
+// alignment (aligned loads, shifted) and the bytes written in aligned pieces
+// across the ends of rows.  A dilation round is one
 // thread per word: the shifts are grouped by their row part (all axes but
 // the last); per group the source row's words j - 1, j, j + 1 are loaded once
 // and every x shift of the group is a funnel shift of them.  HBM traffic of
@@ -37,32 +38,31 @@ struct DilGeom {
     int nlead;                  // leading axes (ndim - 1)
     int32_t lead[DIL_MAX_DIM];  // their sizes
     int64_t rows, W, Wq;
-    int n_groups;
 };
 
-// group g: row shift lead_shift[g * nlead ..], flat row offset row_off[g],
-// x shifts dx[dx_off[g] .. dx_off[g + 1]); near[g] = 1 when every |dx| < 64
-struct DilGroups {
-    const int32_t *lead_shift;
-    const int64_t *row_off;
-    const int32_t *dx_off;
-    const int32_t *dx;
-    const int32_t *near;
+// The shifts in one array of words.  Group g: row shift lead(g)[0 .. nlead), flat
+// row offset row_off(g), x shifts dx(dx_off(g)) .. dx(dx_off(g + 1) - 1); near(g): every
+// |dx| < 64.
+struct DilTable {
+    const int32_t *w;
+    int n_groups, nlead;
+    __device__ __forceinline__ int64_t row_off(int g) const
+    {
+        return (int64_t)(((uint64_t)(uint32_t)w[2 * g + 1] << 32) | (uint32_t)w[2 * g]);
+    }
+    __device__ __forceinline__ int dx_off(int g) const { return w[2 * n_groups + g]; }
+    __device__ __forceinline__ int near(int g) const { return w[3 * n_groups + 1 + g]; }
+    __device__ __forceinline__ const int32_t *lead(int g) const { return w + 4 * n_groups + 1 + g * nlead; }
+    __device__ __forceinline__ int dx(int k) const { return w[(4 + nlead) * n_groups + 1 + k]; }
 };
 
-// one wave per word: word (r, j) of `bits` from the bytes of row r
-__global__ void __launch_bounds__(DIL_NT)
-k_pack_bits(const uint8_t *__restrict__ src, int64_t rows, int64_t W, int64_t Wq, uint64_t *__restrict__ bits)
-{
-    const int64_t word = (int64_t)blockIdx.x * (DIL_NT / 64) + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (word >= rows * Wq) return;   // uniform per wave
-    const int64_t r = word / Wq, j = word - r * Wq;
-    const int64_t x = j * 64 + lane;
-    const bool v = x < W && src[r * W + x] != 0;
-    const uint64_t b = __ballot(v);
-    if (lane == 0) bits[word] = b;
-}
+// Tables up to this size travel with the kernel's arguments (the usual
+// structures: 3 x 3 take 25 words, 5 x 5 x 5 201): five copies to the device took
+// 35 of a small dilation's 120 us.
+constexpr int DIL_SMALL = 256;
+struct DilSmall {
+    int32_t w[DIL_SMALL];
+};
 
 // bytes != 0 of a 32-bit word (4 elements) as 4 bits: the high bit of each
 // byte set when the byte is non-zero, then gathered by one product (the
@@ -114,16 +114,83 @@ k_unpack_words(const uint64_t *__restrict__ bits, uint32_t words, uint8_t *__res
     __builtin_nontemporal_store(q, reinterpret_cast<v4u *>(dst) + c);
 }
 
+// Rows of any length and alignment: one thread per 16 elements of a word, read as
+// five aligned 4-byte words shifted into place (byte by byte where those would
+// leave the array); the four lanes of a word join their 16 bits with shuffles.
+// (16 frames of 1062 x 1028: 32 us with one byte per lane and a ballot.)
 __global__ void __launch_bounds__(DIL_NT)
-k_unpack_bits(const uint64_t *__restrict__ bits, int64_t rows, int64_t W, int64_t Wq, uint8_t *__restrict__ dst)
+k_pack_rows(const uint8_t *__restrict__ src, uint32_t rows, int64_t W, uint32_t Wq, uint64_t *__restrict__ bits)
 {
-    const int64_t word = (int64_t)blockIdx.x * (DIL_NT / 64) + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (word >= rows * Wq) return;
-    const int64_t r = word / Wq, j = word - r * Wq;
-    const int64_t x = j * 64 + lane;
-    if (x >= W) return;
-    dst[r * W + x] = (uint8_t)((bits[word] >> lane) & 1u);
+    const uint32_t c = blockIdx.x * DIL_NT + threadIdx.x, word = c >> 2;
+    const uint32_t words = rows * Wq;
+    uint32_t h = 0;
+    if (word < words) {
+        const uint32_t r = word / Wq, j = word - r * Wq;
+        const int64_t x = (int64_t)j * 64 + 16 * (c & 3u), left = W - x;
+        if (left > 0) {
+            const uint8_t *const p = src + ((int64_t)r * W + x), *const end = src + (int64_t)rows * W;
+            const uint32_t off = (uint32_t)(uintptr_t)p & 3u;
+            const uint8_t *const q = p - off;
+            if (q >= src && q + 20 <= end) {
+                const uint32_t *const v = reinterpret_cast<const uint32_t *>(q);
+                const uint32_t v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3], v4 = v[4];
+                h = nz_nibble(__builtin_amdgcn_alignbyte(v1, v0, off)) |
+                    (nz_nibble(__builtin_amdgcn_alignbyte(v2, v1, off)) << 4) |
+                    (nz_nibble(__builtin_amdgcn_alignbyte(v3, v2, off)) << 8) |
+                    (nz_nibble(__builtin_amdgcn_alignbyte(v4, v3, off)) << 12);
+            } else {
+                for (int k = 0; k < 16 && k < left; k++) h |= (uint32_t)(p[k] != 0) << k;
+            }
+            if (left < 16) h &= (1u << left) - 1u;
+        }
+    }
+    const uint32_t h1 = __shfl_down(h, 1, 4), h2 = __shfl_down(h, 2, 4), h3 = __shfl_down(h, 3, 4);
+    if (word < words && (c & 3u) == 0)
+        bits[word] = (uint64_t)h | ((uint64_t)h1 << 16) | ((uint64_t)h2 << 32) | ((uint64_t)h3 << 48);
+}
+
+// Rows of any length and alignment: one thread per 16 aligned bytes of the
+// output, which may hold the end of one row and the start of the next ones
+// (31 us with one byte per lane).
+__global__ void __launch_bounds__(DIL_NT)
+k_unpack_rows(const uint64_t *__restrict__ bits, uint32_t rows, int64_t W, uint32_t Wq, double inv_W,
+              uint8_t *__restrict__ dst, uint32_t chunks)
+{
+    const uint32_t c = blockIdx.x * DIL_NT + threadIdx.x;
+    if (c >= chunks) return;
+    const int64_t first = (int64_t)c * 16 - (int64_t)((uintptr_t)dst & 15), P = (int64_t)rows * W;
+    const int lo = first < 0 ? (int)-first : 0;   // bytes of the chunk in front of the output
+    int64_t x = first + lo;
+    uint32_t r = (uint32_t)((double)x * inv_W);   // x < 2^36: at most one off
+    x -= (int64_t)r * W;
+    if (x < 0) {
+        r--;
+        x += W;
+    } else if (x >= W) {
+        r++;
+        x -= W;
+    }
+    uint32_t h = 0;
+    int n = lo;
+    while (n < 16 && r < rows) {
+        const uint64_t *const row = bits + (uint64_t)r * Wq;
+        const uint32_t j = (uint32_t)(x >> 6), sh = (uint32_t)x & 63u;
+        uint64_t v = row[j] >> sh;
+        if (sh > 48 && j + 1 < Wq) v |= row[j + 1] << (64 - sh);
+        const int take = (int)min((int64_t)(16 - n), W - x);
+        h |= ((uint32_t)v & ((1u << take) - 1u)) << n;
+        n += take;
+        x = 0;
+        r++;
+    }
+    uint8_t *const o = dst + first;
+    if (lo == 0 && first + 16 <= P) {
+        const v4u q = {nibble_bytes(h & 15u), nibble_bytes((h >> 4) & 15u), nibble_bytes((h >> 8) & 15u),
+                       nibble_bytes(h >> 12)};
+        __builtin_nontemporal_store(q, reinterpret_cast<v4u *>(o));
+    } else {
+        for (int k = lo; k < n; k++) o[k] = (uint8_t)((h >> k) & 1u);
+    }
 }
 
 __device__ __forceinline__ uint64_t word_at(const uint64_t *row, int64_t j, int64_t Wq)
@@ -158,9 +225,9 @@ __device__ __forceinline__ uint64_t near_shift(uint64_t wm, uint64_t w0, uint64_
 
 // one dilation round: Y = X | (M & OR_s X[. - s]); changed[workgroup] = 1
 // where a word changed
-__global__ void __launch_bounds__(DIL_NT)
-k_dilate_bits(const uint64_t *__restrict__ X, const uint64_t *__restrict__ M, DilGeom g, DilGroups grp,
-              uint64_t *__restrict__ Y, int *__restrict__ changed)   // changed: per-workgroup flags or NULL
+__device__ __forceinline__ void dilate_words(const uint64_t *__restrict__ X, const uint64_t *__restrict__ M,
+                                             const DilGeom &g, const DilTable &grp, uint64_t *__restrict__ Y,
+                                             int *__restrict__ changed)   // changed: per-workgroup flags or NULL
 {
     // 32-bit index arithmetic: the host keeps rows * Wq below 2^32
     const uint32_t word = blockIdx.x * DIL_NT + threadIdx.x;
@@ -184,8 +251,8 @@ k_dilate_bits(const uint64_t *__restrict__ X, const uint64_t *__restrict__ M, Di
     const uint64_t m = M ? M[word] : ~0ull;
     uint64_t acc = 0;
     if ((m & ~x) != 0) {   // some element could still join
-        for (int q = 0; q < g.n_groups; q++) {
-            const int32_t *s = grp.lead_shift + (int64_t)q * g.nlead;
+        for (int q = 0; q < grp.n_groups; q++) {
+            const int32_t *s = grp.lead(q);
             bool in = true;
 #pragma unroll
             for (int d = 0; d < DIL_MAX_DIM - 1; d++) {
@@ -195,14 +262,14 @@ k_dilate_bits(const uint64_t *__restrict__ X, const uint64_t *__restrict__ M, Di
                 }
             }
             if (!in) continue;
-            const uint64_t *row = X + ((int64_t)r - grp.row_off[q]) * (int64_t)Wq;
-            const int k0 = grp.dx_off[q], k1 = grp.dx_off[q + 1];
-            if (grp.near[q]) {
+            const uint64_t *row = X + ((int64_t)r - grp.row_off(q)) * (int64_t)Wq;
+            const int k0 = grp.dx_off(q), k1 = grp.dx_off(q + 1);
+            if (grp.near(q)) {
                 const uint64_t wm = word_at(row, (int64_t)j - 1, g.Wq), w0 = row[j];
                 const uint64_t wp = word_at(row, (int64_t)j + 1, g.Wq);
-                for (int k = k0; k < k1; k++) acc |= near_shift(wm, w0, wp, grp.dx[k]);
+                for (int k = k0; k < k1; k++) acc |= near_shift(wm, w0, wp, grp.dx(k));
             } else {
-                for (int k = k0; k < k1; k++) acc |= shifted_word(row, j, g.Wq, grp.dx[k]);
+                for (int k = k0; k < k1; k++) acc |= shifted_word(row, j, g.Wq, grp.dx(k));
             }
         }
     }
@@ -213,6 +280,21 @@ k_dilate_bits(const uint64_t *__restrict__ X, const uint64_t *__restrict__ M, Di
     // one flag per workgroup (stores to one address serialise), written
     // only when the host reads them
     if (changed && __ballot(y != x) != 0 && (threadIdx.x & 63) == 0) changed[blockIdx.x] = 1;
+}
+
+// (the table in device memory, or in the kernel's arguments)
+__global__ void __launch_bounds__(DIL_NT)
+k_dilate_bits(const uint64_t *__restrict__ X, const uint64_t *__restrict__ M, DilGeom g, DilTable grp,
+              uint64_t *__restrict__ Y, int *__restrict__ changed)
+{
+    dilate_words(X, M, g, grp, Y, changed);
+}
+
+__global__ void __launch_bounds__(DIL_NT)
+k_dilate_small(const uint64_t *__restrict__ X, const uint64_t *__restrict__ M, DilGeom g, int n_groups, DilSmall t,
+               uint64_t *__restrict__ Y, int *__restrict__ changed)
+{
+    dilate_words(X, M, g, DilTable{t.w, n_groups, g.nlead}, Y, changed);
 }
 
 // any non-zero among the n per-workgroup flags -> *out (one workgroup)
@@ -276,65 +358,61 @@ static int binary_dilation(const uint8_t *inp, const uint8_t *mask, int ndim, co
         const int32_t dx = (int32_t)s[ndim - 1];
         if (std::find(v.begin(), v.end(), dx) == v.end()) v.push_back(dx);
     }
-    std::vector<int32_t> h_lead, h_dx_off{0}, h_dx, h_near;
-    std::vector<int64_t> h_row_off;
-    for (auto &kv : groups) {
-        int64_t off = 0, stride = 1;
-        for (int d = g.nlead - 1; d >= 0; d--) {
-            off += kv.first[d] * stride;
-            stride *= shape[d];
+    // the words of DilTable
+    const int n_groups = (int)groups.size();
+    std::vector<int32_t> table(2 * (size_t)n_groups), near, lead, dx, dx_off{0};
+    {
+        size_t i = 0;
+        for (auto &kv : groups) {
+            int64_t off = 0, stride = 1;
+            for (int d = g.nlead - 1; d >= 0; d--) {
+                off += kv.first[d] * stride;
+                stride *= shape[d];
+            }
+            table[i++] = (int32_t)(uint32_t)(uint64_t)off;
+            table[i++] = (int32_t)(uint32_t)((uint64_t)off >> 32);
+            lead.insert(lead.end(), kv.first.begin(), kv.first.end());
+            bool all = true;
+            for (int32_t v : kv.second) all &= v > -64 && v < 64;
+            near.push_back(all ? 1 : 0);
+            dx.insert(dx.end(), kv.second.begin(), kv.second.end());
+            dx_off.push_back((int32_t)dx.size());
         }
-        h_lead.insert(h_lead.end(), kv.first.begin(), kv.first.end());
-        h_row_off.push_back(off);
-        bool near = true;
-        for (int32_t dx : kv.second) near &= dx > -64 && dx < 64;
-        h_near.push_back(near ? 1 : 0);
-        h_dx.insert(h_dx.end(), kv.second.begin(), kv.second.end());
-        h_dx_off.push_back((int32_t)h_dx.size());
+        for (const auto *v : {&dx_off, &near, &lead, &dx}) table.insert(table.end(), v->begin(), v->end());
     }
-    g.n_groups = (int)h_row_off.size();
+    const bool small = table.size() <= (size_t)DIL_SMALL;
 
     hipStream_t st = (hipStream_t)stream;
     Workspace ws(st);
     const int64_t words = g.rows * g.Wq;
-    const int64_t rounds = g.n_groups ? iterations : 0;
+    const int64_t rounds = n_groups ? iterations : 0;
     DevBuf<uint64_t> a, b, mb;
-    DevBuf<int32_t> d_lead, d_dx_off, d_dx, d_near;
-    DevBuf<int64_t> d_row_off;
+    DevBuf<int32_t> d_table;
     DevBuf<int> flags;
+    DilSmall small_table;
     CBX_HIP(a.alloc(words, st));
     if (rounds > 0) {
         CBX_HIP(b.alloc(words, st));
         if (mask) CBX_HIP(mb.alloc(words, st));
-        CBX_HIP(d_lead.alloc(std::max<size_t>(h_lead.size(), 1), st));
-        CBX_HIP(d_row_off.alloc(h_row_off.size(), st));
-        CBX_HIP(d_dx_off.alloc(h_dx_off.size(), st));
-        CBX_HIP(d_dx.alloc(h_dx.size(), st));
-        CBX_HIP(d_near.alloc(h_near.size(), st));
         if (rounds > 8) CBX_HIP(flags.alloc((size_t)grid_for(words, DIL_NT) + 1, st));
-        if (!h_lead.empty())
-            CBX_HIP(hipMemcpyAsync(d_lead.ptr, h_lead.data(), sizeof(int32_t) * h_lead.size(), hipMemcpyHostToDevice, st));
-        CBX_HIP(hipMemcpyAsync(d_row_off.ptr, h_row_off.data(), sizeof(int64_t) * h_row_off.size(),
-                               hipMemcpyHostToDevice, st));
-        CBX_HIP(hipMemcpyAsync(d_dx_off.ptr, h_dx_off.data(), sizeof(int32_t) * h_dx_off.size(),
-                               hipMemcpyHostToDevice, st));
-        CBX_HIP(hipMemcpyAsync(d_dx.ptr, h_dx.data(), sizeof(int32_t) * h_dx.size(), hipMemcpyHostToDevice, st));
-        CBX_HIP(hipMemcpyAsync(d_near.ptr, h_near.data(), sizeof(int32_t) * h_near.size(), hipMemcpyHostToDevice, st));
+        if (small) {
+            std::copy(table.begin(), table.end(), small_table.w);
+        } else {
+            CBX_HIP(d_table.alloc(table.size(), st));
+            CBX_HIP(hipMemcpyAsync(d_table.ptr, table.data(), sizeof(int32_t) * table.size(), hipMemcpyHostToDevice, st));
+        }
     }
-    const int wpb = DIL_NT / 64;
-    const unsigned pack_grid = (unsigned)((words + wpb - 1) / wpb);
     // whole words of 16-byte aligned rows: one thread per 16 bytes
     auto aligned = [&](const void *p) { return (g.W % 64) == 0 && ((uintptr_t)p & 15) == 0; };
     const unsigned quarter_grid = (unsigned)((4 * words + DIL_NT - 1) / DIL_NT);
     auto pack = [&](const uint8_t *src, uint64_t *dst) {
         if (aligned(src)) k_pack_words<<<quarter_grid, DIL_NT, 0, st>>>(src, (uint32_t)words, dst);
-        else k_pack_bits<<<pack_grid, DIL_NT, 0, st>>>(src, g.rows, g.W, g.Wq, dst);
+        else k_pack_rows<<<quarter_grid, DIL_NT, 0, st>>>(src, (uint32_t)g.rows, g.W, (uint32_t)g.Wq, dst);
     };
     KernelTimer timer("dilation", st);
     pack(inp, a.ptr);
     if (rounds > 0 && mask) pack(mask, mb.ptr);
     CBX_HIP(hipGetLastError());
-    const DilGroups grp{d_lead.ptr, d_row_off.ptr, d_dx_off.ptr, d_dx.ptr, d_near.ptr};
     uint64_t *cur = a.ptr, *nxt = b.ptr;
     // the rounds in batches of 8; a batch whose last round changed nothing
     // ends the dilation (the last round of a batch followed by another sets
@@ -349,7 +427,9 @@ static int binary_dilation(const uint8_t *inp, const uint8_t *mask, int ndim, co
                 k_clear_flags<<<grid_for(n_blocks, DIL_NT), DIL_NT, 0, st>>>(flags.ptr, n_blocks);
                 fl = flags.ptr;
             }
-            k_dilate_bits<<<n_blocks, DIL_NT, 0, st>>>(cur, mask ? mb.ptr : nullptr, g, grp, nxt, fl);
+            const uint64_t *const m = mask ? mb.ptr : nullptr;
+            if (small) k_dilate_small<<<n_blocks, DIL_NT, 0, st>>>(cur, m, g, n_groups, small_table, nxt, fl);
+            else k_dilate_bits<<<n_blocks, DIL_NT, 0, st>>>(cur, m, g, DilTable{d_table.ptr, n_groups, g.nlead}, nxt, fl);
             std::swap(cur, nxt);
         }
         CBX_HIP(hipGetLastError());
@@ -364,8 +444,13 @@ static int binary_dilation(const uint8_t *inp, const uint8_t *mask, int ndim, co
             if (hv == 0) break;
         }
     }
-    if (aligned(out)) k_unpack_words<<<quarter_grid, DIL_NT, 0, st>>>(cur, (uint32_t)words, out);
-    else k_unpack_bits<<<pack_grid, DIL_NT, 0, st>>>(cur, g.rows, g.W, g.Wq, out);
+    if (aligned(out)) {
+        k_unpack_words<<<quarter_grid, DIL_NT, 0, st>>>(cur, (uint32_t)words, out);
+    } else {
+        const int64_t chunks = (P + (int64_t)((uintptr_t)out & 15) + 15) / 16;   // < 2^32
+        k_unpack_rows<<<(unsigned)((chunks + DIL_NT - 1) / DIL_NT), DIL_NT, 0, st>>>(
+            cur, (uint32_t)g.rows, g.W, (uint32_t)g.Wq, 1.0 / (double)g.W, out, (uint32_t)chunks);
+    }
     CBX_HIP(hipGetLastError());
     return CBX_OK;
 }
