@@ -396,6 +396,11 @@ k_draw3(T *__restrict__ out, const T *__restrict__ lines, int64_t n_lines, const
 // as many steps each (one lane per line left most of a wave idle behind its
 // longest and widest line).
 
+//
+// The walk is a serial chain, so its time is the instructions of a step times the
+// longest line.  One loop for all long axes (walk3_main's, unrolled for each, left
+// a wave of mixed lines running three in turn), increments known before it, moves
+// by selects: 50 000 lines of up to 40 voxels 72 -> 29 us.
 template <typename T>
 __global__ void __launch_bounds__(D3_NT)
 k_walk3_main(const T *__restrict__ lines, int64_t n_lines, const int64_t *__restrict__ off,
@@ -405,28 +410,78 @@ k_walk3_main(const T *__restrict__ lines, int64_t n_lines, const int64_t *__rest
     if (i >= n_lines) return;
     const int64_t base = off[i], cap = off[i + 1] - base;
     if (cap == 0) return;
+    PlaneState<T> *const dst = states + base;
+    const int most = (int)min(cap, (int64_t)INT_MAX);
+    int k = 0;
     Line3<T> L;
-    int64_t k = 0;
     if (line3_setup(lines + 7 * i, L) == 1) {
-        auto plane = [&](const Iter3<T> &it) {
-            if (k == cap) {   // cannot happen: one plane per long-axis step
-                atomicOr(flags, FLAG_STUCK);
-                return;
-            }
-            PlaneState<T> ps;
-            ps.te = it.te;
-            for (int q = 0; q < 3; q++) {
-                ps.ne[q] = it.ne[q];
-                ps.cur[q] = (int32_t)it.cur[q];
-            }
-            ps.line = (int32_t)i;
-            states[base + k++] = ps;
+        Iter3<T> it;
+        it3_start(L, it);
+        const int s0 = (int)L.step[0], s1 = (int)L.step[1], s2 = (int)L.step[2];
+        const T t0 = (T)s0 * L.t[0], t1 = (T)s1 * L.t[1], t2 = (T)s2 * L.t[2];
+        // the normal errors' changes: pair (0,1) along 0, 1; (0,2) along 0, 2; (1,2) along 1, 2
+        const T a0 = (T)s0 * L.nrm[0][0], a1 = (T)s1 * L.nrm[0][1], b0 = (T)s0 * L.nrm[1][0], b2 = (T)s2 * L.nrm[1][2],
+                c1 = (T)s1 * L.nrm[2][1], c2 = (T)s2 * L.nrm[2][2];
+        // steps to the walk's end along each axis, and the budget of all of them
+        int l0 = (int)((L.m1[0] - L.m0[0]) * s0), l1 = (int)((L.m1[1] - L.m0[1]) * s1),
+            l2 = (int)((L.m1[2] - L.m0[2]) * s2);
+        int64_t budget = (int64_t)l0 + l1 + l2 + 64;
+        T te = it.te, na = it.ne[0], nb = it.ne[1], nc = it.ne[2];
+        int x = (int)it.cur[0], y = (int)it.cur[1], z = (int)it.cur[2];
+        // a pair's choice (it3_update): whether its first and second axis may step
+        auto choice = [](T n, T u, T v, bool &first, bool &second) {
+            const T ex = n + u, ey = n + v, exy = ex + v;
+            const bool q = m_abs(ey) < m_abs(ex);
+            const bool both = m_abs(exy) < m_abs(q ? ey : ex);
+            first = !q | both;
+            second = q | both;
         };
-        if (L.axis == 0) walk3_main<0>(L, flags, plane);
-        else if (L.axis == 1) walk3_main<1>(L, flags, plane);
-        else walk3_main<2>(L, flags, plane);
+        bool go = (l0 != 0) & (l1 != 0) & (l2 != 0);
+        while (go) {
+            bool a_0, a_1, b_0, b_2, c_1, c_2;
+            choice(na, a0, a1, a_0, a_1);
+            choice(nb, b0, b2, b_0, b_2);
+            choice(nc, c1, c2, c_1, c_2);
+            const bool m0 = a_0 & b_0, m1 = a_1 & c_1, m2 = b_2 & c_2;
+            if ((L.axis == 0) ? m0 : ((L.axis == 1) ? m1 : m2)) {
+                if (k == most) {   // cannot happen: one plane per long-axis step
+                    atomicOr(flags, FLAG_STUCK);
+                    break;
+                }
+                PlaneState<T> ps;
+                ps.te = te;
+                ps.ne[0] = na;
+                ps.ne[1] = nb;
+                ps.ne[2] = nc;
+                ps.cur[0] = x;
+                ps.cur[1] = y;
+                ps.cur[2] = z;
+                ps.line = (int32_t)i;
+                dst[k++] = ps;
+            }
+            if (budget-- == 0) {
+                atomicOr(flags, FLAG_STUCK);
+                break;
+            }
+            te += m0 ? t0 : T(0);
+            te += m1 ? t1 : T(0);
+            te += m2 ? t2 : T(0);
+            na += m0 ? a0 : T(0);
+            na += m1 ? a1 : T(0);
+            nb += m0 ? b0 : T(0);
+            nb += m2 ? b2 : T(0);
+            nc += m1 ? c1 : T(0);
+            nc += m2 ? c2 : T(0);
+            x += m0 ? s0 : 0;
+            y += m1 ? s1 : 0;
+            z += m2 ? s2 : 0;
+            l0 -= m0 ? 1 : 0;
+            l1 -= m1 ? 1 : 0;
+            l2 -= m2 ? 1 : 0;
+            go = (l0 != 0) & (l1 != 0) & (l2 != 0);
+        }
     }
-    for (; k < cap; k++) states[base + k].line = -1;
+    for (int64_t q = k; q < cap; q++) dst[q].line = -1;
 }
 
 // A line's constants for the fills of its planes: Line3's, and what turns their
