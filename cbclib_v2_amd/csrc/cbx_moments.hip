@@ -591,8 +591,14 @@ __device__ T logbinom(int64_t n, int64_t k, T p)
     T t = (T)(lgamma((double)(n + 1)) - lgamma((double)(k + 1)) - lgamma((double)(n - k + 1)) +
               (double)((T)k * log_p) + (double)((T)(n - k) * log_q));
     T tail = t;
+    // Past its mode the terms fall for good (the increment falls with i); once one
+    // is so small against the sum that 1 + exp(t - tail) rounds to 1, it and all
+    // that follow leave the sum as it is.
+    const T nil = sizeof(T) == 4 ? T(18) : T(38);
     for (int64_t i = k + 1; i < n + 1; ++i) {
-        t = (T)((double)t + (log((double)(n - i + 1)) - log((double)i) + (double)log_p - (double)log_q));
+        const double inc = log((double)(n - i + 1)) - log((double)i) + (double)log_p - (double)log_q;
+        t = (T)((double)t + inc);
+        if (inc < 0.0 && t < tail - nil) break;
         tail = dev_logaddexp(tail, t);
     }
     return tail;
