@@ -17,22 +17,25 @@
 //                     atomic per run of items into one sub-list.
 //  3. k_scan          item offsets per tile sub-list (one host read: the
 //                     item total, flags and slot count; plans read nothing).
-//  4. k_bin_slots     one lane per segment slot: the per-tile item lists.
-//  5. k_tiles         one workgroup per TILE x TILE pixel tile: one wave
-//                     resumes each item's walk from its checkpoint (phase 1,
-//                     column records into LDS), then all waves fill the
-//                     columns (phase 2), accumulating into an LDS tile with
-//                     LDS atomics (fixed point for float sums); the tile is
-//                     flushed to HBM once with a coalesced read-modify-write.
-//                     HBM traffic of the image: one read and one write per
-//                     touched tile.
+//  4. k_bin_slots     one lane per segment slot: the per-tile item lists, in
+//                     sub-lists of like cost (list_class).
+//  5. k_tiles_fast    (cbx_tiles.hip) one workgroup per TILE x TILE pixel tile of
+//                     float images, k_tiles of double images and exact values:
+//                     each item's walk is resumed from its checkpoint (phase 1,
+//                     column records into LDS) and its columns are filled (phase
+//                     2) into an LDS tile with LDS atomics (fixed point for float
+//                     sums); the tile is flushed to HBM once with a coalesced
+//                     read-modify-write.  HBM traffic of the image: one read and
+//                     one write per touched tile.
 //
 // Ordered path (pixel lists, the deterministic mode, accumulate_lines with
 // different overlaps): k_segments walks twice (count, then write) so that a
 // line's segments are consecutive and lines keep their input order, and
 // k_tiles_ordered applies each pixel's terms in ascending line order, the
-// single-threaded reference's order.  The adjoint (k_adjoint_tiles,
-// k_line_grad) runs on the tile path's segments and lists.
+// single-threaded reference's order.  accumulate_lines of float lines in short
+// terms takes the tile path instead (k_term_order, k_tiles_terms).  The adjoint
+// (k_adjoint_fast, k_adjoint_tiles for doubles, k_line_grad) runs on the tile
+// path's segments and lists.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1015,8 +1018,8 @@ struct AdjRec {
 // where its item stands in the list.
 //
 // Bound by vector instruction issue: the gradient of 160 000 biweight lines
-// (widths 2 to 6, 32 frames of 1024^2) takes 620 us, of which its 313 M wave
-// instructions need 510 at the issue rate; with one lane per column and the
+// (widths 2 to 6, 32 frames of 1024^2) takes 584 us, of which its 289 M wave
+// instructions need 470 at the issue rate; with one lane per column and the
 // full terms (25 double operations, two divisions per column) 983 us.  Chunks of
 // 16 items leave half the lanes of phase 2b idle (838 against 688 us with 32,
 // before the sums of phase 2b were shared with 2a); 192 / SEG fill four

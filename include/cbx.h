@@ -61,8 +61,9 @@ CBX_API int cbx_kernel_id(const char *name);
 
 /*
  * Launch options of draw_lines (NULL = automatic).  `tile` is the side of the
- * square pixel tile one workgroup accumulates in LDS (32 or 64), `seg` the
- * number of long-axis columns per walk checkpoint (8 or 16).  `deterministic`
+ * square pixel tile one workgroup accumulates in LDS (32 or 64; 0 = 64, or 32
+ * where the frames have few tiles), `seg` the number of long-axis columns per
+ * walk checkpoint (8 or 16; 0 = 8).  `deterministic`
  * = 1 accumulates every pixel in ascending line order starting from the value
  * already in `out`, which is the single-threaded reference's order: the
  * result is then bit-identical to bresenham.draw_lines(..., num_threads=1).
@@ -134,9 +135,8 @@ CBX_API int cbx_draw_pixels_f64(int64_t n_frames, int64_t height, int64_t width,
  * (n_frames x height x width, in place) with `out_overlap`
  * (CBX_SUM | CBX_MAX each).  A term or frame index out of range ->
  * CBX_EINDEX.  Equal overlaps are draw_lines with idxs = frames[terms]; mixed
- * overlaps reduce each term per pixel tile in the reference's line order and
- * add (or max) the tile into its frame with atomics, so terms sharing a frame
- * pixel combine in no fixed order.  opts as for draw_lines (the tile path of
+ * overlaps reduce each term per pixel tile and add (or max) it into its frame,
+ * so terms sharing a frame pixel combine in no fixed order.  opts as for draw_lines (the tile path of
  * equal overlaps);
  * opts->kernels is not accepted.  Replaces bresenham.accumulate_lines
  * (bresenham.cpp:151-309, bound at 326-327) and
