@@ -476,21 +476,20 @@ __device__ __forceinline__ void fill_half(Acc *img, uint32_t *zb, const FillRec 
 template <int K>
 constexpr float interior_scale() { return K == K_GAUSSIAN ? 6.4921276840f : 1.0f; }   // exp(-4.5 u) = 2^(-k u)
 
-// (+ h: 0.5 where the value is then cut to an integer)
 template <int K>
-__device__ __forceinline__ float interior_value(float x, float c, float h)
+__device__ __forceinline__ float interior_value(float x, float c)
 {
     if constexpr (K == K_BIWEIGHT) {
         const float m = __builtin_fmaf(-x, x, 1.0f);
-        return __builtin_fmaf(c * m, m, h);
+        return c * (m * m);
     } else if constexpr (K == K_GAUSSIAN) {
-        return __builtin_fmaf(c, __builtin_amdgcn_exp2f(-(x * x)), h);
+        return c * __builtin_amdgcn_exp2f(-(x * x));
     } else if constexpr (K == K_PARABOLIC) {
-        return __builtin_fmaf(-c * x, x, c + h);
+        return c * __builtin_fmaf(-x, x, 1.0f);
     } else if constexpr (K == K_RECTANGULAR) {
-        return c + h;
+        return c;
     } else {
-        return __builtin_fmaf(-c, __builtin_fabsf(x), c + h);
+        return __builtin_fmaf(-c, __builtin_fabsf(x), c);
     }
 }
 
@@ -527,13 +526,14 @@ __device__ __forceinline__ void fill_interior(Acc *img, uint32_t *zb, const Inne
     float jf = (float)a;
     Acc *q = img + (at + a * sstride);
     for (Acc *const e = q + max(n, 0) * sstride; q != e; q += sstride) {
-        const float x = __builtin_fmaf(jf, I.dx, x0);
+        const float v = interior_value<K>(__builtin_fmaf(jf, I.dx, x0), c);
         if constexpr (OV == 2) {
-            // (rounded to nearest: below 2^23 the sum with 0.5 is exact, above it the value is whole)
-            const uint32_t u = (uint32_t)interior_value<K>(x, c, 0.5f);
+            // (not cut after adding 0.5 inside the value's product, one instruction
+            // less: from 2^23 on that sum is rounded itself)
+            const uint32_t u = __float2uint_rn(v);
             atomicAdd(q, fast_positive<K>() ? u : max(1u, u));
         } else {
-            atomicMax(q, ord_enc(interior_value<K>(x, c, 0.0f)));
+            atomicMax(q, ord_enc(v));
         }
         jf += 1.0f;
     }
