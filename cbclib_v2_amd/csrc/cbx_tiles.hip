@@ -164,8 +164,8 @@ __device__ __forceinline__ float fold_fix(float o, uint32_t acc, uint32_t zbit, 
 // pixel values: F >= 22, so that eight faint terms stay within 1e-6 max_val.
 constexpr int FIX_ROUND = 1023;
 
-// Tile kernel of the double images, of exact values and of sums of non-finite
-// values.  The workgroup takes its tile's items ((segment, line) pairs)
+// Tile kernel of the double images, of exact values and of non-finite values.
+// The workgroup takes its tile's items ((segment, line) pairs)
 // in chunks of CH <= NT: phase 1 gives each of CH threads one item (the walk
 // replay, column records into LDS); phase 2 gives each thread one (item,
 // column, half) unit of the fills at a time.  The first chunk's loads and
@@ -1081,6 +1081,23 @@ void run_tiles_terms(float *out, const SegmentPlan<float> &P, float max_val, int
 template void run_tiles_terms<CBX_PROFILE>(float *, const SegmentPlan<float> &, float, int, hipStream_t);
 #endif
 
+template <int K, int OV, int TILE, int SEG>
+static void launch_fast(float *out, const SegmentPlan<float> &P, float max_val, int threads, int chunk, bool,
+                        hipStream_t st)
+{
+#define CBX_TILES_FAST(NT, CHW)                                                                                 \
+    k_tiles_fast<K, OV, TILE, SEG, NT, CHW><<<(unsigned)P.n_tiles, NT, 0, st>>>(                               \
+        out, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, P.lite.ptr, max_val, P.flags.ptr)
+    // 256 records per wave: four workgroups' areas fit a CU's LDS and the tile's few items spread over
+    // its waves (64 frames of 2048^2, seg 8: 24 / 32 / 48 items 0.604 / 0.592 / 0.721 ms; 256 of 1024^2,
+    // seg 16: 8 / 16 / 24 / 32 items 3.72 / 2.80 / 3.07 / 2.89 ms)
+    if (threads == 64) CBX_TILES_FAST(64, 64);
+    else if (threads == 128) CBX_TILES_FAST(128, 32);
+    else if (chunk == 64) CBX_TILES_FAST(256, (SEG == 8 ? 32 : 16));
+    else CBX_TILES_FAST(256, (SEG == 8 ? 64 : 32));
+#undef CBX_TILES_FAST
+}
+
 template <typename T, int K, int OV, int TILE, int SEG>
 static void launch_tiles(T *out, const SegmentPlan<T> &P, T max_val, int threads, int chunk, bool fast,
                          hipStream_t st)
@@ -1088,46 +1105,18 @@ static void launch_tiles(T *out, const SegmentPlan<T> &P, T max_val, int threads
 #define CBX_TILES(NT, CH, FST)                                                                                  \
     k_tiles<T, K, OV, TILE, SEG, NT, CH, FST><<<(unsigned)P.n_tiles, NT, 0, st>>>(                             \
         out, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, max_val, P.flags.ptr)
-#define CBX_TILES_FAST(NT, CHW)                                                                                 \
-    k_tiles_fast<K, OV, TILE, SEG, NT, CHW><<<(unsigned)P.n_tiles, NT, 0, st>>>(                               \
-        out, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, P.lite.ptr, max_val, P.flags.ptr)
-    if constexpr (sizeof(T) == 4 && OV != 0) {
-        if (OV == 2 || fast) {
-            // 256 records per wave: four workgroups' areas fit a CU's LDS and the tile's few items spread over
-            // its waves (64 frames of 2048^2, seg 8: 24 / 32 / 48 items 0.604 / 0.592 / 0.721 ms; 256 of 1024^2,
-            // seg 16: 8 / 16 / 24 / 32 items 3.72 / 2.80 / 3.07 / 2.89 ms)
-            if (threads == 64) CBX_TILES_FAST(64, 64);
-            else if (threads == 128) CBX_TILES_FAST(128, 32);
-            else if (chunk == 64) CBX_TILES_FAST(256, (SEG == 8 ? 32 : 16));
-            else CBX_TILES_FAST(256, (SEG == 8 ? 64 : 32));
-            return;
-        }
-    }
-    if constexpr (OV != 2) {
-        if (fast) {
-            if (threads == 64) CBX_TILES(64, 64, true);
-            else if (threads == 128) CBX_TILES(128, 64, true);
-            else if (chunk == 64) CBX_TILES(256, 64, true);
-            else CBX_TILES(256, 256, true);
-        } else {
-            if (threads == 64) CBX_TILES(64, 64, false);
-            else if (threads == 128) CBX_TILES(128, 64, false);
-            else if (chunk == 64) CBX_TILES(256, 64, false);
-            else CBX_TILES(256, 256, false);
-        }
+    if (fast) {
+        if (threads == 64) CBX_TILES(64, 64, true);
+        else if (threads == 128) CBX_TILES(128, 64, true);
+        else if (chunk == 64) CBX_TILES(256, 64, true);
+        else CBX_TILES(256, 256, true);
+    } else {
+        if (threads == 64) CBX_TILES(64, 64, false);
+        else if (threads == 128) CBX_TILES(128, 64, false);
+        else if (chunk == 64) CBX_TILES(256, 64, false);
+        else CBX_TILES(256, 256, false);
     }
 #undef CBX_TILES
-#undef CBX_TILES_FAST
-}
-
-template <typename T, int K, int OV>
-static void launch_tiles_k(T *out, const SegmentPlan<T> &P, T max_val, int threads, int chunk, bool fast,
-                           hipStream_t st)
-{
-    if (P.g.tile == 64 && P.g.seg == 16) launch_tiles<T, K, OV, 64, 16>(out, P, max_val, threads, chunk, fast, st);
-    else if (P.g.tile == 64) launch_tiles<T, K, OV, 64, 8>(out, P, max_val, threads, chunk, fast, st);
-    else if (P.g.seg == 16) launch_tiles<T, K, OV, 32, 16>(out, P, max_val, threads, chunk, fast, st);
-    else launch_tiles<T, K, OV, 32, 8>(out, P, max_val, threads, chunk, fast, st);
 }
 
 template <typename T, int K>
@@ -1137,16 +1126,24 @@ void run_tiles_profile(T *out, const SegmentPlan<T> &P, T max_val, int overlap, 
     const int threads = (opts && opts->threads) ? opts->threads : 256;
     const bool fast = !(opts && opts->exact_values);
     const int chunk = (opts && opts->chunk) ? opts->chunk : 64;
-    // float sums on the fast path accumulate in fixed point, unless max_val
-    // is not finite (inf * 0 must stay NaN, as in the reference)
+    const Geometry &g = P.g;
+#define CBX_SHAPE(FN, ...)                                                                                      \
+    ((g.tile == 64) ? ((g.seg == 16) ? FN<__VA_ARGS__, 64, 16> : FN<__VA_ARGS__, 64, 8>)                        \
+                    : ((g.seg == 16) ? FN<__VA_ARGS__, 32, 16> : FN<__VA_ARGS__, 32, 8>))(                      \
+        out, P, max_val, threads, chunk, fast, st)
+    // k_tiles_fast takes max_val out of the sum and out of the profile's
+    // differences: not where it is no finite number (inf * 0 and inf - inf are
+    // NaN, where max_val * K(x) is inf)
     if constexpr (sizeof(T) == 4) {
-        if (overlap == 0 && fast && std::isfinite(max_val)) {
-            launch_tiles_k<T, K, 2>(out, P, max_val, threads, chunk, fast, st);
+        if (fast && std::isfinite(max_val)) {
+            if (overlap == 0) CBX_SHAPE(launch_fast, K, 2);
+            else CBX_SHAPE(launch_fast, K, 1);
             return;
         }
     }
-    if (overlap == 0) launch_tiles_k<T, K, 0>(out, P, max_val, threads, chunk, fast, st);
-    else launch_tiles_k<T, K, 1>(out, P, max_val, threads, chunk, fast, st);
+    if (overlap == 0) CBX_SHAPE(launch_tiles, T, K, 0);
+    else CBX_SHAPE(launch_tiles, T, K, 1);
+#undef CBX_SHAPE
 }
 
 template void run_tiles_profile<float, CBX_PROFILE>(float *, const SegmentPlan<float> &, float, int,
