@@ -100,7 +100,6 @@ __device__ __forceinline__ LineLite line_lite(const LineSetup<float> &L)
     r.cap = J * (m_abs(pick(L.t, b)) * 1.00001f + L.LL * 2.4e-7f);
     r.meta = a | (pick(L.st, a) > 0 ? FR_SA : 0) | (pick(L.st, b) > 0 ? FR_SB : 0) | (L.safe ? FR_SAFE : 0) |
              ((int)(uint8_t)L.kid << 8);
-    r.term = -1;
     return r;
 }
 
@@ -287,8 +286,7 @@ template <typename T, typename I>
 __global__ void __launch_bounds__(256)
 k_setup_lines(const T *__restrict__ lines, const I *__restrict__ idxs, const uint8_t *__restrict__ kernels,
               int kernel, int64_t n_lines, Geometry g, LineSetup<T> *__restrict__ setup,
-              LineLite *__restrict__ lite, const int32_t *__restrict__ line_term,
-              unsigned long long *__restrict__ counters, int *__restrict__ flags)
+              LineLite *__restrict__ lite, unsigned long long *__restrict__ counters, int *__restrict__ flags)
 {
     const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int ub = 0;
@@ -296,11 +294,7 @@ k_setup_lines(const T *__restrict__ lines, const I *__restrict__ idxs, const uin
         LineSetup<T> L;
         setup_line(lines, idxs, kernels, kernel, l, g, L, flags);
         setup[l] = L;
-        if constexpr (sizeof(T) == 4) {
-            LineLite r = line_lite(L);
-            if (line_term) r.term = line_term[l];
-            lite[l] = r;
-        }
+        if constexpr (sizeof(T) == 4) lite[l] = line_lite(L);
         ub = segment_bound(L, g);
     }
 #pragma unroll
@@ -1549,10 +1543,10 @@ static std::atomic<int64_t> g_slot_hint{0};
 template <typename T, typename I>
 static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs, const uint8_t *kernels,
                                 int kernel, int64_t n_lines, int64_t n_frames, int64_t H, int64_t W, int tile,
-                                int seg, hipStream_t st, int64_t *line_base = nullptr, bool slot_tiles = false,
-                                const int32_t *line_term = nullptr)
+                                int seg, hipStream_t st, int64_t *line_base = nullptr, bool slot_tiles = false, bool skip_neg = false)
 {
     Geometry &g = P.g;
+    g.skip_neg = skip_neg ? 1 : 0;
     g.n_frames = n_frames;
     g.H = (int32_t)H;
     g.W = (int32_t)W;
@@ -1578,8 +1572,7 @@ static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs
     }
     const int blk = 256;
     k_setup_lines<T, I><<<grid_for(n_lines, blk), blk, 0, st>>>(lines, idxs, kernels, kernel, n_lines, g,
-                                                               P.setup.ptr, P.lite.ptr, line_term, counters.ptr,
-                                                               P.flags.ptr);
+                                                               P.setup.ptr, P.lite.ptr, counters.ptr, P.flags.ptr);
     CBX_HIP(hipGetLastError());
     uint64_t hv[3];
     int fl = 0, rc = 0;
@@ -1963,39 +1956,48 @@ __device__ __forceinline__ double point_segment2(double px, double py, double ax
     return dx * dx + dy * dy;
 }
 
-// line_term[i] = the term of line i if another line of it may draw one of line
-// i's pixels, else -1.  Every pixel of a line lies within its width of the
-// segment, up to the drift of the float walk: lines further apart than both
-// widths plus 1 px plus 1e-4 of their lengths share none.  (A line that draws
-// nothing, e.g. a NaN end point, touches none.)
+// Splits the lines: one that another line of its term may touch (draw a pixel of)
+// keeps its term in `touching` and gets frame -1, one alone in its pixels gets
+// -1 in `touching` and keeps its frame; *n_touching counts the former.  Every pixel
+// of a line lies within its width of the segment, up to the drift of the float
+// walk: lines further apart than both widths plus 1 px plus 1e-4 of their lengths
+// share none.  (A line that draws nothing, e.g. a NaN end point, touches none.)
 template <typename T, typename I>
-__global__ void k_term_touch(const T *__restrict__ lines, const I *__restrict__ terms, const int *__restrict__ off,
-                             const int *__restrict__ order, int64_t n_lines, int32_t *__restrict__ line_term)
+__global__ void __launch_bounds__(256)
+k_term_touch(const T *__restrict__ lines, const I *__restrict__ terms, const int *__restrict__ off,
+             const int *__restrict__ order, int64_t n_lines, I *__restrict__ frame, I *__restrict__ touching,
+             int *__restrict__ n_touching)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n_lines) return;
-    const int t = (int)terms[i];
-    const T *a = lines + 5 * i;
-    const double ax = a[0], ay = a[1], bx = a[2], by = a[3], wa = a[4];
-    const double la = fabs(bx - ax) + fabs(by - ay);
     bool touch = false;
-    for (int k = off[t]; k < off[t + 1] && !touch; k++) {
-        const int j = order[k];
-        if (j == (int)i) continue;
-        const T *b = lines + 5 * (int64_t)j;
-        const double cx = b[0], cy = b[1], dx = b[2], dy = b[3];
-        const double r = wa + (double)b[4] + 1.0 + 1e-4 * (la + fabs(dx - cx) + fabs(dy - cy));
-        if (!(fmax(cx, dx) + r >= fmin(ax, bx) && fmin(cx, dx) - r <= fmax(ax, bx) && fmax(cy, dy) + r >= fmin(ay, by) &&
-              fmin(cy, dy) - r <= fmax(ay, by)))
-            continue;
-        // the segments cross, or the distance is an end point's
-        const double o1 = (bx - ax) * (cy - ay) - (by - ay) * (cx - ax), o2 = (bx - ax) * (dy - ay) - (by - ay) * (dx - ax);
-        const double o3 = (dx - cx) * (ay - cy) - (dy - cy) * (ax - cx), o4 = (dx - cx) * (by - cy) - (dy - cy) * (bx - cx);
-        const double d2 = fmin(fmin(point_segment2(ax, ay, cx, cy, dx, dy), point_segment2(bx, by, cx, cy, dx, dy)),
-                               fmin(point_segment2(cx, cy, ax, ay, bx, by), point_segment2(dx, dy, ax, ay, bx, by)));
-        touch = (o1 * o2 <= 0.0 && o3 * o4 <= 0.0) || d2 <= r * r;
+    if (i < n_lines) {
+        const int t = (int)terms[i];
+        const T *a = lines + 5 * i;
+        const double ax = a[0], ay = a[1], bx = a[2], by = a[3], wa = a[4];
+        const double la = fabs(bx - ax) + fabs(by - ay);
+        for (int k = off[t]; k < off[t + 1] && !touch; k++) {
+            const int j = order[k];
+            if (j == (int)i) continue;
+            const T *b = lines + 5 * (int64_t)j;
+            const double cx = b[0], cy = b[1], dx = b[2], dy = b[3];
+            const double r = wa + (double)b[4] + 1.0 + 1e-4 * (la + fabs(dx - cx) + fabs(dy - cy));
+            if (!(fmax(cx, dx) + r >= fmin(ax, bx) && fmin(cx, dx) - r <= fmax(ax, bx) &&
+                  fmax(cy, dy) + r >= fmin(ay, by) && fmin(cy, dy) - r <= fmax(ay, by)))
+                continue;
+            // the segments cross, or the distance is an end point's
+            const double o1 = (bx - ax) * (cy - ay) - (by - ay) * (cx - ax);
+            const double o2 = (bx - ax) * (dy - ay) - (by - ay) * (dx - ax);
+            const double o3 = (dx - cx) * (ay - cy) - (dy - cy) * (ax - cx);
+            const double o4 = (dx - cx) * (by - cy) - (dy - cy) * (bx - cx);
+            const double d2 = fmin(fmin(point_segment2(ax, ay, cx, cy, dx, dy), point_segment2(bx, by, cx, cy, dx, dy)),
+                                   fmin(point_segment2(cx, cy, ax, ay, bx, by), point_segment2(dx, dy, ax, ay, bx, by)));
+            touch = (o1 * o2 <= 0.0 && o3 * o4 <= 0.0) || d2 <= r * r;
+        }
+        touching[i] = touch ? (I)t : (I)(-1);
+        if (touch) frame[i] = (I)(-1);
     }
-    line_term[i] = touch ? t : -1;
+    const int n = __syncthreads_count(touch);
+    if (threadIdx.x == 0 && n) atomicAdd(n_touching, n);
 }
 
 // The ids of the plan tiles that hold items (in no fixed order), one atomic
@@ -2035,22 +2037,30 @@ static void launch_accumulate(int kernel, T *out, const SegmentPlan<T> &P, T max
 // accumulate_lines (bresenham.cpp:151-256): lines grouped into terms, each
 // term reduced over its lines (in_overlap), terms reduced into frames
 // (out_overlap).  Equal overlaps compose to draw_lines with idxs =
-// frames[terms] on the tile path.  So do mixed overlaps for every line that no
-// other line of its term can touch (k_term_touch), with out_overlap; the others
-// follow term by term in the same frame tiles (k_tiles_terms).  Double images
-// and terms of many lines (MAX_TERM_LINES) bin the lines by (term,
+// frames[terms] on the tile path.  Different overlaps bin the lines by (term,
 // tile) and run the ordered tile kernel in accumulate mode: each term tile
 // is reduced in LDS in reference line order from zero, like the reference's
 // term buffer, and its touched pixels are combined into frame frames[term]
 // with atomics (bresenham.cpp:230-248).  Terms reach a frame in no fixed
 // order, as under the reference's OpenMP loop over terms.
+//
+// In float images most lines of a term usually share no pixel with another line
+// of it (k_term_touch).  The reduction over such a line is the line, so those
+// go to the frames by the tile kernel with exact values, which is cheaper
+// than a (term, tile) list each; a sum of them is rounded once instead of once
+// a term.
 // (term, tile) pairs of one mixed-overlap accumulate plan at most
 constexpr int64_t MAX_TERM_TILES = int64_t(1) << 24;
-// Mixed overlaps of float images whose terms hold at most this many lines go by
-// frame tiles (k_term_touch compares every pair of a term's lines: 256 x the
-// lines; 64 000 lines in 4000 terms of 16 and 16 frames of 512^2 take 1.37 ms by
-// (term, tile) lists and 0.23 ms by frame tiles).
+// k_term_touch compares every pair of a term's lines (this many times the lines):
+// terms of more lines leave all lines to the (term, tile) lists.
 constexpr int64_t MAX_TERM_LINES = 256;
+// A second plan and its launches take 70 us, and its tile kernel a workgroup per
+// tile; a line alone saves some 20 ns of (term, tile) lists.  So it is made for at
+// least this many such lines in at least this many tiles.  All lists / split, us, lines
+// of 10 to 60 px: 1000, 4000 and 8000 lines in 1024 tiles 178 / 210, 249 / 242 and
+// 336 / 264, 64 000 lines 1420 / 480; 16 000 lines in 81, 100 and 144 tiles 475 / 537,
+// 485 / 493 and 504 / 440; 64 000 lines in 49 tiles 1330 / 1970.
+constexpr int64_t LONE_MIN_LINES = 4096, LONE_MIN_TILES = 128;
 
 // term of each line within the batch [t0, t1), or -1 (a line of another batch)
 template <typename I>
@@ -2085,10 +2095,15 @@ static int accumulate_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W,
     hipStream_t st = (hipStream_t)stream;
     const int64_t n_chk = n_lines > n_terms ? n_lines : n_terms;
     const bool same = in_overlap == out_overlap;
-    // different overlaps of float images: by frame tiles, unless a term is large
-    // (below), a tile index would not fit or max_val is not finite
-    bool by_tile = !same && sizeof(T) == 4 && std::isfinite(max_val) && n_lines > 0 && n_terms > 0 &&
-                   n_frames * ((H + 63) / 64) * ((W + 63) / 64) < (int64_t(1) << 31) / LIST_SUBS;
+    // lines alone in their pixels by frame tiles (LONE_MIN_LINES), unless a term is
+    // large (surely so where the terms hold more lines on average, else counted
+    // below), a tile index would not fit or max_val is not finite
+    int tile = 0, seg = 0;
+    resolve_opts<T>(nullptr, n_frames, H, W, n_lines, false, tile, seg);
+    const int64_t n_tiles = n_frames * ((H + tile - 1) / tile) * ((W + tile - 1) / tile);
+    bool by_tile = !same && sizeof(T) == 4 && std::isfinite(max_val) && n_lines >= LONE_MIN_LINES &&
+                   n_lines <= MAX_TERM_LINES * n_terms && n_tiles >= LONE_MIN_TILES &&
+                   n_tiles < (int64_t(1) << 31) / LIST_SUBS;
     DevBuf<I> comp;
     DevBuf<int32_t> frames32;
     DevBuf<int> cnt, rank;
@@ -2123,36 +2138,36 @@ static int accumulate_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W,
                                            (in_overlap == 1 && max_val < T(0)) ? T(0) : max_val, kernel,
                                            in_overlap, opts, stream);
 
-    if constexpr (sizeof(T) == 4) {
+    // lines alone in their pixels: a plan of their own over the frames, drawn after the others
+    SegmentPlan<T> lone;
+    DevBuf<I> touching;
+    int64_t n_touching = n_lines;
+    if (by_tile) {
+        DevBuf<int> off, order, n_dev;
+        CBX_HIP(touching.alloc(n_lines, st));
+        CBX_HIP(off.alloc(n_terms + 1, st));
+        CBX_HIP(order.alloc(n_lines, st));
+        CBX_HIP(n_dev.alloc(1, st));
+        void *const zp[1] = {n_dev.ptr};
+        const int64_t zw[1] = {1};
+        CBX_HIP(zero_words(st, 1, zp, zw));
+        CBX_HIP(exclusive_scan_total_i32(cnt.ptr, nullptr, off.ptr, n_terms, st));
+        const unsigned grid = (unsigned)grid_for(n_lines, 256);
+        k_term_order<I><<<grid, 256, 0, st>>>(terms, off.ptr, rank.ptr, n_lines, order.ptr);
+        k_term_touch<T, I><<<grid, 256, 0, st>>>(lines, terms, off.ptr, order.ptr, n_lines, comp.ptr, touching.ptr,
+                                                 n_dev.ptr);
+        CBX_HIP(hipGetLastError());
+        const void *src[1] = {n_dev.ptr};
+        const int nb[1] = {4};
+        uint64_t hv = 0;
+        CBX_HIP(read_device_values(st, 1, src, nb, &hv));
+        n_touching = (int64_t)hv;
+        by_tile = n_lines - n_touching >= LONE_MIN_LINES;
         if (by_tile) {
-            DevBuf<int> off, order;
-            DevBuf<int32_t> line_term;
-            CBX_HIP(off.alloc(n_terms + 1, st));
-            CBX_HIP(order.alloc(n_lines, st));
-            CBX_HIP(line_term.alloc(n_lines, st));
-            CBX_HIP(exclusive_scan_total_i32(cnt.ptr, nullptr, off.ptr, n_terms, st));
-            const unsigned grid = (unsigned)grid_for(n_lines, 256);
-            k_term_order<I><<<grid, 256, 0, st>>>(terms, off.ptr, rank.ptr, n_lines, order.ptr);
-            k_term_touch<T, I><<<grid, 256, 0, st>>>(lines, terms, off.ptr, order.ptr, n_lines, line_term.ptr);
-            CBX_HIP(hipGetLastError());
-            // a term's buffer starts at zero: with max_val < 0 its maximum is 0
-            const T mv = (in_overlap == 1 && max_val < T(0)) ? T(0) : max_val;
-            SegmentPlan<T> P;
-            if ((rc = build_plan_unordered<T, I>(P, lines, comp.ptr, nullptr, kernel, n_lines, n_frames, H, W, 64, 8, st,
-                                                 nullptr, false, line_term.ptr)))
+            // (checks every line: a call that fails leaves `out` untouched)
+            if ((rc = build_plan_unordered<T, I>(lone, lines, comp.ptr, nullptr, kernel, n_lines, n_frames, H, W, tile,
+                                                 seg, st, nullptr, false, true)))
                 return rc;
-            if (P.n_segs == 0) return CBX_OK;
-            KernelTimer timer("accumulate_tiles", st);
-            run_tiles<T>(out, P, kernel, out_overlap, mv, nullptr, st);
-            switch (kernel) {
-            case K_BIWEIGHT: run_tiles_terms<K_BIWEIGHT>(out, P, mv, in_overlap, st); break;
-            case K_GAUSSIAN: run_tiles_terms<K_GAUSSIAN>(out, P, mv, in_overlap, st); break;
-            case K_PARABOLIC: run_tiles_terms<K_PARABOLIC>(out, P, mv, in_overlap, st); break;
-            case K_RECTANGULAR: run_tiles_terms<K_RECTANGULAR>(out, P, mv, in_overlap, st); break;
-            default: run_tiles_terms<K_TRIANGULAR>(out, P, mv, in_overlap, st); break;
-            }
-            CBX_HIP(hipGetLastError());
-            return CBX_OK;
         }
     }
 
@@ -2162,20 +2177,29 @@ static int accumulate_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W,
     // memory the next batch reuses.
     const int64_t per_frame = ((H + 31) / 32) * ((W + 31) / 32);
     const int64_t batch = std::max<int64_t>(1, std::min<int64_t>(n_terms, MAX_TERM_TILES / per_frame));
+    const I *const of_terms = by_tile ? touching.ptr : terms;
     DevBuf<I> bterms;
-    if (batch < n_terms) CBX_HIP(bterms.alloc(n_lines, st));
-    for (int64_t t0 = 0; t0 < n_terms; t0 += batch) {
+    if (batch < n_terms && n_touching > 0) CBX_HIP(bterms.alloc(n_lines, st));
+    for (int64_t t0 = 0; t0 < n_terms && n_touching > 0; t0 += batch) {
         const int64_t t1 = std::min(n_terms, t0 + batch);
         Workspace inner(st);
-        const I *bidx = terms;
+        const I *bidx = of_terms;
         if (batch < n_terms) {
-            k_term_batch<I><<<grid_for(n_lines, 256), 256, 0, st>>>(terms, n_lines, t0, t1, bterms.ptr);
+            k_term_batch<I><<<grid_for(n_lines, 256), 256, 0, st>>>(of_terms, n_lines, t0, t1, bterms.ptr);
             CBX_HIP(hipGetLastError());
             bidx = bterms.ptr;
         }
-        if ((rc = accumulate_batch<T, I>(out, lines, n_lines, bidx, t1 - t0, batch < n_terms, frames32.ptr + t0, H,
-                                         W, max_val, kernel, in_overlap, st)))
+        if ((rc = accumulate_batch<T, I>(out, lines, n_lines, bidx, t1 - t0, by_tile || batch < n_terms, frames32.ptr + t0,
+                                         H, W, max_val, kernel, in_overlap, st)))
             return rc;
+    }
+    if (by_tile && lone.n_segs > 0) {
+        KernelTimer timer("accumulate_lone", st);
+        cbx_draw_opts exact{};
+        exact.exact_values = 1;
+        // a term's buffer starts at zero: with max_val < 0 its maximum is 0
+        run_tiles<T>(out, lone, kernel, out_overlap, (in_overlap == 1 && max_val < T(0)) ? T(0) : max_val, &exact, st);
+        CBX_HIP(hipGetLastError());
     }
     return CBX_OK;
 }
@@ -2425,8 +2449,7 @@ static int plan_draw(cbx_plan *pl, float *out, const float *lines, int64_t n_lin
                                                          P.tile_cur.ptr, pl->scan_state.ptr,
                                                          (int64_t)pl->scan_state.n);
     k_setup_lines<float, int32_t><<<grid_for(n_lines, blk), blk, 0, st>>>(lines, idxs, kernels, kernel, n_lines, g,
-                                                                         P.setup.ptr, P.lite.ptr, nullptr, pl->counters.ptr,
-                                                                         P.flags.ptr);
+                                                                         P.setup.ptr, P.lite.ptr, pl->counters.ptr, P.flags.ptr);
     k_walk_lines<float><<<grid_for(n_lines, blk), blk, 0, st>>>(n_lines, g, P.setup.ptr, P.segs.ptr, P.n_segs,
                                                                 pl->counters.ptr, P.tile_cnt.ptr, P.flags.ptr,
                                                                 pl->line_base.ptr);

@@ -29,8 +29,6 @@ struct alignas(16) LineLite {
     float nlim;       // band limit
     float cap;        // a column with cap < Te < LL - cap has no tangential overshoot at any of its pixels
     int32_t meta;     // FR_* bits, profile id in bits 8-15
-    int32_t term;     // accumulate_lines with different overlaps: the line's term when another line of it
-                      // may touch this one, else (and in every other draw) -1
 };
 constexpr int FR_AXIS = 1, FR_SA = 2, FR_SB = 4, FR_SAFE = 8;
 
@@ -41,7 +39,7 @@ struct Geometry {
     int32_t tile_log, seg_log;
     int32_t ntx, nty;
     uint32_t m_frame = 0, m_ntx = 0;   // tile_coords: 2^32 / (tiles per frame), 2^32 / ntx, rounded down
-    int32_t skip_neg = 0;   // 1: a line with a negative frame draws nothing (accumulate_lines term batches)
+    int32_t skip_neg = 0;   // 1: a line with a negative frame draws nothing (accumulate_lines: another plan's lines)
 };
 
 // The unordered plan's item list of tile t is split into LIST_SUBS sub-lists by
@@ -264,11 +262,5 @@ struct SegmentPlan {
 template <typename T, int K>
 void run_tiles_profile(T *out, const SegmentPlan<T> &P, T max_val, int overlap, const cbx_draw_opts *opts,
                        hipStream_t st);
-
-// accumulate_lines with different overlaps, after run_tiles_profile has drawn the
-// lines alone in their pixels (LineLite::term < 0): the other lines, term by term
-// (k_tiles_terms; plans of 64-pixel tiles and 8-column segments).
-template <int K>
-void run_tiles_terms(float *out, const SegmentPlan<float> &P, float max_val, int in_overlap, hipStream_t st);
 
 } // namespace cbx

@@ -704,7 +704,7 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                     R.nb = nb;
                     R.c0 = ax ? sg.c[0] : sg.c[1];
                     R.line = sg.line;
-                    R.meta = meta | ((L.term < 0 ? sg.ncols : 0) << 16);
+                    R.meta = meta | (sg.ncols << 16);
                     wR[dst] = R;
                     InnerRec I;
                     I.inv = __builtin_amdgcn_rcpf(nb);
@@ -720,8 +720,7 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                     I.far = L.LL - L.cap;
                     I.base = ax ? (sg.c[1] - Y0) * PITCH - X0 : (sg.c[0] - X0) - Y0 * PITCH;
                     wI[dst] = I;
-                    const int ncols = (L.term < 0) ? sg.ncols : 0;   // (a line of k_tiles_terms: no columns)
-                    if (!replay_columns<SEG>(wK, L, sg, dst * SEG, ncols)) atomicOr(flags, FLAG_STUCK);
+                    if (!replay_columns<SEG>(wK, L, sg, dst * SEG, sg.ncols)) atomicOr(flags, FLAG_STUCK);
                 }
             }
             take(np);
@@ -876,210 +875,6 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
         }
     }
 }
-
-// accumulate_lines with different overlaps: the lines of a tile whose term has
-// another line that may touch them (LineLite::term >= 0), one term after the
-// other.  Their items are collected from the tile's list, ordered by term
-// (and place in the list), and their walks replayed 64 at a time; a term's
-// items are then drawn into an LDS tile from zero with the inner overlap
-// (max: order-preserving codes; sum: fixed point, F = clz of the term's items
-// here) and its touched pixels folded into the tile's current values, held in
-// registers, with the outer overlap.  Lines alone in their term's pixels never
-// come here (the reduction over one line is the line): k_tiles_fast has drawn
-// them before.  A term has at most MAX_TERM_LINES (256) lines and a line at most
-// 8 segments in a 64-pixel tile, so the items of one term always fit
-// TERM_ITEMS; where those of all terms do not, terms are taken by their low
-// bits, as many as it needs.  Bound by the latency of a tile's terms, one after
-// the other: 65 us for 4000 terms of 16 lines of up to 60 px in 16 frames of
-// 512^2 (6 % of the lines touch another of their term); 95 us when every term
-// searched the tile's list and replayed its own walks.
-constexpr int TERM_ITEMS = 2304;
-
-template <int K, int IN_OV>
-__global__ void __launch_bounds__(256)
-k_tiles_terms(float *__restrict__ out, Geometry g, const int *__restrict__ tile_off, const int2 *__restrict__ pairs,
-              const Segment<float> *__restrict__ segs, const LineSetup<float> *__restrict__ setup,
-              const LineLite *__restrict__ lite, float max_val, int *__restrict__ flags)
-{
-    constexpr int TILE = 64, SEG = 8, NT = 256, PX = TILE * TILE, PP = PX / NT, CH = 64;
-    constexpr int OV = (IN_OV == 1) ? 1 : 2;   // codes or fixed point in the term's tile
-    __shared__ uint32_t img[PX];
-    __shared__ uint32_t zb[PX / 32];
-    __shared__ int32_t rS[CH * SEG];
-    __shared__ float rN[CH * SEG], rT[CH * SEG];
-    __shared__ FillRec frec[CH];
-    __shared__ int32_t place[TERM_ITEMS], key[TERM_ITEMS];   // item (place in the tile's list) and its term
-    __shared__ uint16_t order[TERM_ITEMS];
-    __shared__ int32_t s_n;
-
-    const int tile = blockIdx.x;
-    const int beg = tile_off[tile * LIST_SUBS], end = tile_off[(tile + 1) * LIST_SUBS];
-    if (*flags || beg == end) return;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const uint64_t below = (1ull << lane) - 1ull;
-    const int n_items = end - beg;
-    for (int i = tid; i < PX; i += NT) img[i] = 0u;
-    for (int i = tid; i < PX / 32; i += NT) zb[i] = 0u;
-
-    int64_t f;
-    int tx, ty;
-    tile_coords(g, tile, f, tx, ty);
-    const int X0 = tx * TILE, Y0 = ty * TILE;
-    const int X1 = min(X0 + TILE, g.W), Y1 = min(Y0 + TILE, g.H);
-    float *const to = out + ((f * g.H + Y0) * (int64_t)g.W + X0);
-    float pre[PP];
-    bool drawn = false;
-    for (int bits = 0, low = 0;;) {
-        // the items of the terms whose `bits` low bits are `low`
-        __syncthreads();
-        if (tid == 0) s_n = 0;
-        __syncthreads();
-        for (int w = 0; w < n_items; w += NT) {
-            const int i = w + tid;
-            const int t = (i < n_items) ? lite[pairs[beg + i].y].term : -1;
-            const bool hit = t >= 0 && (t & ((1 << bits) - 1)) == low;
-            const uint64_t m = __ballot(hit);
-            int at = 0;
-            if (lane == 0 && m) at = atomicAdd(&s_n, __popcll(m));
-            at = __shfl(at, 0, 64) + __popcll(m & below);
-            if (hit && at < TERM_ITEMS) {
-                place[at] = i;
-                key[at] = t;
-            }
-        }
-        __syncthreads();
-        const int n_all = s_n;
-        if (n_all > TERM_ITEMS && bits < 30) {
-            bits++;
-            continue;
-        }
-        const int n_hit = min(n_all, TERM_ITEMS);   // (one term's items: always fewer)
-        if (n_hit > 0 && !drawn) {
-            // the tile's current values (clamped into the frame: pixels
-            // outside it are not stored)
-            drawn = true;
-#pragma unroll
-            for (int j = 0; j < PP; j++) {
-                const int i = tid + j * NT;
-                const int y = min(i / TILE, Y1 - Y0 - 1), x = min(i % TILE, X1 - X0 - 1);
-                pre[j] = to[(int64_t)y * g.W + x];
-            }
-        }
-        for (int i = tid; i < n_hit; i += NT) {
-            const int t = key[i], p = place[i];
-            int rank = 0;
-            for (int j = 0; j < n_hit; j++) rank += (key[j] < t) | ((key[j] == t) & (place[j] < p));
-            order[rank] = (uint16_t)i;
-        }
-        int F = 0;
-        for (int c0 = 0; c0 < n_hit; c0 += CH) {
-            const int c1 = min(c0 + CH, n_hit);
-            __syncthreads();
-            if (tid < c1 - c0) {
-                const int2 it = pairs[beg + place[order[c0 + tid]]];
-                const Segment<float> sg = segs[it.x];
-                const LineSetup<float> L = setup[it.y];
-                const int a = L.axis;
-                frec[tid] = fill_rec(L, pick(sg.c, a), it.y);
-                WalkState<float> s;
-                s.c[0] = sg.c[0];
-                s.c[1] = sg.c[1];
-                s.Te = sg.Te;
-                s.Ne = sg.Ne;
-#pragma unroll
-                for (int k = 0; k < SEG; k++) rS[tid * SEG + k] = INT_MIN;
-                int k = 0;
-                for (int q = 0; q < 4 * SEG + 16 && k < sg.ncols; q++) {
-                    bool nx, ny;
-                    walk_next(L, s.Ne, nx, ny);
-                    if (a == 0 ? nx : ny) {
-                        rS[tid * SEG + k] = pick(s.c, 1 - a);
-                        rT[tid * SEG + k] = s.Te;
-                        rN[tid * SEG + k] = s.Ne;
-                        k++;
-                    }
-                    walk_step(L, s, nx, ny);
-                }
-                if (k < sg.ncols) atomicOr(flags, FLAG_STUCK);
-            }
-            __syncthreads();
-            // the terms of these items, one at a time
-            for (int g0 = c0, g1; g0 < c1; g0 = g1) {
-                const int t = key[order[g0]];
-                if (OV == 2 && (g0 == 0 || key[order[g0 - 1]] != t)) {
-                    int m = 1;
-                    while (g0 + m < n_hit && key[order[g0 + m]] == t) m++;
-                    F = __clz(m);
-                }
-                for (g1 = g0 + 1; g1 < c1 && key[order[g1]] == t;) g1++;
-                const float vscale = (OV == 2) ? __int_as_float((127 + F) << 23) : max_val;
-                for (int u = (g0 - c0) * SEG * 2 + tid; u < (g1 - c0) * SEG * 2; u += NT) {
-                    const int slot = u >> 1, half = u & 1;
-                    const int i = slot / SEG, k = slot % SEG;
-                    const int cs = rS[slot];
-                    if (cs == INT_MIN) continue;
-                    const FillRec R = frec[i];
-                    const int a = R.meta & FR_AXIS;
-                    const int c = R.c0 + ((R.meta & FR_SA) ? k : -k);
-                    fill_half<K, OV>(img, zb, R, setup, cs, rT[slot], rN[slot], half, a ? (c - Y0) * TILE : c - X0,
-                                     a ? 1 : TILE, a ? X0 : Y0, a ? X1 : Y1, vscale);
-                }
-                if (g1 == c1 && g1 < n_hit && key[order[g1]] == t) break;   // goes on in the next items
-                __syncthreads();
-                // the term's touched pixels into the frame's
-                const float p2 = __int_as_float((127 - F) << 23), zero = max_val * 0.0f;
-#pragma unroll
-                for (int j = 0; j < PP; j++) {
-                    const int i = tid + j * NT;
-                    const uint32_t e = img[i];
-                    const bool z = (OV == 2) && ((zb[i >> 5] >> (i & 31)) & 1u);
-                    if (e != 0u || z) {
-                        if constexpr (IN_OV == 1) {
-                            pre[j] += ord_dec(e);
-                        } else {
-                            const float v = e ? ((float)e * p2) * max_val : zero;
-                            pre[j] = (pre[j] < v) ? v : pre[j];   // std::max(out, term)
-                        }
-                        img[i] = 0u;
-                    }
-                }
-                if constexpr (OV == 2) {
-                    __syncthreads();
-                    for (int i = tid; i < PX / 32; i += NT) zb[i] = 0u;
-                }
-                __syncthreads();
-            }
-        }
-        // the next set of low bits: the sibling of the last set not yet taken
-        while (bits > 0 && ((low >> (bits - 1)) & 1)) {
-            bits--;
-            low &= (1 << bits) - 1;
-        }
-        if (bits == 0) break;
-        low |= 1 << (bits - 1);
-    }
-    if (!drawn) return;
-#pragma unroll
-    for (int j = 0; j < PP; j++) {
-        const int i = tid + j * NT;
-        if (i / TILE < Y1 - Y0 && i % TILE < X1 - X0) to[(int64_t)(i / TILE) * g.W + (i % TILE)] = pre[j];
-    }
-}
-
-#if CBX_PROFILE < 5
-template <int K>
-void run_tiles_terms(float *out, const SegmentPlan<float> &P, float max_val, int in_overlap, hipStream_t st)
-{
-    if (in_overlap == 1)
-        k_tiles_terms<K, 1><<<(unsigned)P.n_tiles, 256, 0, st>>>(out, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr,
-                                                                 P.setup.ptr, P.lite.ptr, max_val, P.flags.ptr);
-    else
-        k_tiles_terms<K, 0><<<(unsigned)P.n_tiles, 256, 0, st>>>(out, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr,
-                                                                 P.setup.ptr, P.lite.ptr, max_val, P.flags.ptr);
-}
-
-template void run_tiles_terms<CBX_PROFILE>(float *, const SegmentPlan<float> &, float, int, hipStream_t);
-#endif
 
 template <int K, int OV, int TILE, int SEG>
 static void launch_fast(float *out, const SegmentPlan<float> &P, float max_val, int threads, int chunk, bool,
