@@ -1907,14 +1907,11 @@ static int draw_pixels_impl(int64_t n_frames, int64_t H, int64_t W, const T *lin
 // accumulate_lines, step 1: range checks of terms and frames (bad[0]: a term
 // outside [0, n_terms), bad[1]: a frame outside [0, n_frames)), the frame of
 // every term as int32 (frames32, n_terms entries) and, when comp != nullptr,
-// the frame of every line, comp[i] = frames[terms[i]].  With cnt: also the lines
-// of every term (cnt), each line's place among them (rank, in no fixed order)
-// and the largest count (bad[2]).
+// the frame of every line, comp[i] = frames[terms[i]].
 template <typename I>
 __global__ void k_term_frames(const I *__restrict__ terms, const I *__restrict__ frames, int64_t n_lines,
                               int64_t n_terms, int64_t n_frames, I *__restrict__ comp,
-                              int32_t *__restrict__ frames32, int *__restrict__ bad, int *__restrict__ cnt,
-                              int *__restrict__ rank)
+                              int32_t *__restrict__ frames32, int *__restrict__ bad)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i < n_terms) {
@@ -1929,11 +1926,48 @@ __global__ void k_term_frames(const I *__restrict__ terms, const I *__restrict__
         if (t < 0 || (int64_t)t >= n_terms) atomicOr(bad, 1);
         else f = frames[t];
         if (comp) comp[i] = (f < 0 || (int64_t)f >= n_frames) ? I(0) : f;
-        if (cnt && t >= 0 && (int64_t)t < n_terms) {
-            const int r = atomicAdd(&cnt[t], 1);
-            rank[i] = r;
-            if (r + 1 > __hip_atomic_load(bad + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(bad + 2, r + 1);
+    }
+}
+
+// Lines of every term (cnt) and each line's place among them (rank, in no fixed
+// order), unless a term has more than `most` lines: then *many is set, counting
+// stops and what was counted is of no use.  The lines of one term in a wave take one
+// atomic.  Counters of few long terms share a cache line, whose atomics take 11 ns
+// each one after the other (300 000 shuffled lines of 20 terms, an atomic each:
+// 3.3 ms), so few workgroups run at a time and see what the ones before have found.
+constexpr int TERM_COUNT_BLOCKS = 64;
+
+template <typename I>
+__global__ void __launch_bounds__(256)
+k_term_count(const I *__restrict__ terms, int64_t n_lines, int64_t n_terms, int most, int *__restrict__ cnt,
+             int *__restrict__ rank, int *__restrict__ many)
+{
+    const int lane = threadIdx.x & 63;
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (int64_t i0 = blockIdx.x * (int64_t)256 + (threadIdx.x & ~63); i0 < n_lines; i0 += gridDim.x * (int64_t)256) {
+        const int64_t i = i0 + lane;
+        const int64_t t64 = (i < n_lines) ? (int64_t)terms[i] : -1;
+        if (__hip_atomic_load(many, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+        const bool ok = t64 >= 0 && t64 < n_terms;   // (others: k_term_frames)
+        const int t = ok ? (int)t64 : -1;
+        int lead = lane, place = 0, n = 0;
+        for (uint64_t rest = __ballot(ok); rest;) {
+            const int l = __builtin_ctzll(rest);
+            const uint64_t m = __ballot(t == __shfl(t, l, 64));
+            if ((m >> lane) & 1) {
+                lead = l;
+                place = __popcll(m & below);
+                n = __popcll(m);
+            }
+            rest &= ~m;
         }
+        int base = 0;
+        if (ok && lead == lane) {
+            base = atomicAdd(&cnt[t], n);
+            if (base + n > most) atomicOr(many, 1);
+        }
+        base = __shfl(base, lead, 64);
+        if (ok) rank[i] = base + place;
     }
 }
 
@@ -2120,7 +2154,10 @@ static int accumulate_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W,
         const int64_t zw[2] = {3, by_tile ? n_terms : 0};
         CBX_HIP(zero_words(st, 2, zp, zw));
         k_term_frames<I><<<grid_for(n_chk, 256), 256, 0, st>>>(terms, frames, n_lines, n_terms, n_frames,
-                                                                 comp.ptr, frames32.ptr, bad.ptr, cnt.ptr, rank.ptr);
+                                                                 comp.ptr, frames32.ptr, bad.ptr);
+        if (by_tile)
+            k_term_count<I><<<(unsigned)std::min<int64_t>(grid_for(n_lines, 256), TERM_COUNT_BLOCKS), 256, 0, st>>>(
+                terms, n_lines, n_terms, (int)MAX_TERM_LINES, cnt.ptr, rank.ptr, bad.ptr + 2);
         CBX_HIP(hipGetLastError());
         const void *src[3] = {bad.ptr, bad.ptr + 1, bad.ptr + 2};
         const int nb[3] = {4, 4, 4};
@@ -2128,7 +2165,7 @@ static int accumulate_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W,
         CBX_HIP(read_device_values(st, 3, src, nb, hv));
         if (hv[1]) return fail(CBX_EINDEX, "frames is outside of (0, n_frames)");
         if (hv[0]) return fail(CBX_EINDEX, "a term index is outside of (0, len(frames))");
-        by_tile = by_tile && (int64_t)hv[2] <= MAX_TERM_LINES;
+        by_tile = by_tile && hv[2] == 0;
     }
     if (n_lines == 0 || n_frames * H * W == 0) return CBX_OK;
     // max/max: the term buffer starts at zero and takes std::max(buffer, v),

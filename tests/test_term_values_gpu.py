@@ -32,9 +32,14 @@ def case(kind):
         'fewer': ((1, 360, 390), 4095, 2000, 60.0),       # too few lines
         'large': ((1, 360, 390), 5140, 20, 30.0),         # terms of 257 lines
         'small frame': ((1, 90, 70), 9000, 1500, 30.0),   # too few tiles
+        'at most': ((1, 360, 390), 5376, 40, 12.0),       # terms of up to 256 lines, in no order
+        'one more': ((1, 360, 390), 5377, 40, 12.0),      # a term of 257
     }[kind]
     lines = random_segments(rng, n, *shape[1:], 1.0, lmax, 0.4, 4.0, pad=5.0).astype(np.float32)
     terms = (np.arange(n) % n_terms).astype(np.int32)
+    if kind in ('at most', 'one more'):
+        terms = np.minimum(np.arange(n) // 256, 20).astype(np.int32)
+        rng.shuffle(terms)
     return shape, lines, terms, rng.integers(0, shape[0], n_terms).astype(np.int32)
 
 
@@ -45,7 +50,7 @@ def accumulated(shape, lines, terms, frames, kernel, modes):
 
 
 @pytest.mark.parametrize('kernel', ['biweight', 'gaussian', 'parabolic', 'rectangular', 'triangular'])
-@pytest.mark.parametrize('kind', ['spread', 'crossing', 'alone', 'fewer', 'large', 'small frame'])
+@pytest.mark.parametrize('kind', ['spread', 'crossing', 'alone', 'fewer', 'large', 'small frame', 'at most', 'one more'])
 def test_term_values(cuda, oracle, kind, kernel):
     shape, lines, terms, frames = case(kind)
     rtol = 3e-7 if kernel == 'gaussian' else 0.0
