@@ -1648,16 +1648,14 @@ static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs
 // tiles than the card has CUs (256); there tiles of 32 x 32 share the work of a
 // tile among four workgroups.  Measured for 64 / 32, us: doubles 154 / 114 at 64
 // tiles, 161 / 131 at 256; gradients 170 / 148 at 64, 178 / 163 at 256, 136 / 140 at
-// 704; float draws, whose tiles cost little, gain where a tile has some dozen lines
-// (79 / 61 with 5000 lines in 64 tiles, 118 / 114 with 1000) and lose where it has
-// fewer (82 / 85 with 700 in 88).
-template <typename T>
-static void resolve_opts(const cbx_draw_opts *o, int64_t n_frames, int64_t H, int64_t W, int64_t n_lines, bool gradient,
-                         int &tile, int &seg)
+// 704; float draws 79 / 61 with 5000 lines in 64 tiles, 118 / 114 with 1000, and
+// where a tile has a few lines only 75 / 78 (192 lines in 64 tiles, gradient 102 / 101).
+// The frames decide, not the lines or the pass, so that a plan, the eager draw and the
+// eager gradient of the same frames work on the same tiles and give the same bits.
+static void resolve_opts(const cbx_draw_opts *o, int64_t n_frames, int64_t H, int64_t W, int &tile, int &seg)
 {
     const double tiles = (double)n_frames * (double)((H + 63) / 64) * (double)((W + 63) / 64);
-    const bool few = tiles <= 256.0 && (gradient || sizeof(T) == 8 || (double)n_lines >= 12.0 * tiles);
-    tile = (o && o->tile) ? o->tile : (few ? 32 : 64);
+    tile = (o && o->tile) ? o->tile : (tiles <= 256.0 ? 32 : 64);
     seg = (o && o->seg) ? o->seg : 8;
 }
 
@@ -1851,7 +1849,7 @@ static int draw_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W, const
     int rc = check_common(n_frames, H, W, n_lines, idxs != nullptr, kernel, overlap);
     if (rc) return rc;
     int tile, seg;
-    resolve_opts<T>(opts, n_frames, H, W, n_lines, false, tile, seg);
+    resolve_opts(opts, n_frames, H, W, tile, seg);
     if ((rc = check_opts(tile, seg))) return rc;
     if (opts && !(opts->threads == 0 || opts->threads == 64 || opts->threads == 128 || opts->threads == 256))
         return fail(CBX_EVALUE, "threads must be 64, 128 or 256");
@@ -2133,7 +2131,7 @@ static int accumulate_lines_impl(T *out, int64_t n_frames, int64_t H, int64_t W,
     // large (surely so where the terms hold more lines on average, else counted
     // below), a tile index would not fit or max_val is not finite
     int tile = 0, seg = 0;
-    resolve_opts<T>(nullptr, n_frames, H, W, n_lines, false, tile, seg);
+    resolve_opts(nullptr, n_frames, H, W, tile, seg);
     const int64_t n_tiles = n_frames * ((H + tile - 1) / tile) * ((W + tile - 1) / tile);
     bool by_tile = !same && sizeof(T) == 4 && std::isfinite(max_val) && n_lines >= LONE_MIN_LINES &&
                    n_lines <= MAX_TERM_LINES * n_terms && n_tiles >= LONE_MIN_TILES &&
@@ -2320,7 +2318,7 @@ static int adjoint_impl(const T *grad, int64_t n_frames, int64_t H, int64_t W, c
     int rc = check_common(n_frames, H, W, n_lines, idxs != nullptr, kernel, 0);
     if (rc) return rc;
     int tile, seg;
-    resolve_opts<T>(opts, n_frames, H, W, n_lines, true, tile, seg);
+    resolve_opts(opts, n_frames, H, W, tile, seg);
     if ((rc = check_opts(tile, seg))) return rc;
     hipStream_t st = (hipStream_t)stream;
     if (n_lines == 0) return CBX_OK;
@@ -2401,7 +2399,7 @@ static int plan_create(cbx_plan **out_plan, int64_t n_frames, int64_t H, int64_t
     if (!(headroom >= 1.0) || headroom > 64.0) return fail(CBX_EVALUE, "headroom must be in [1, 64]");
     if (n_lines <= 0 || n_frames * H * W == 0) return fail(CBX_EVALUE, "a plan needs lines and a non-empty frame");
     int tile, seg;
-    resolve_opts<float>(opts, n_frames, H, W, n_lines, false, tile, seg);
+    resolve_opts(opts, n_frames, H, W, tile, seg);
     if ((rc = check_opts(tile, seg))) return rc;
     if (opts && !(opts->threads == 0 || opts->threads == 64 || opts->threads == 128 || opts->threads == 256))
         return fail(CBX_EVALUE, "threads must be 64, 128 or 256");
