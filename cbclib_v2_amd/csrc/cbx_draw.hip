@@ -143,10 +143,13 @@ __device__ __forceinline__ int fill_reach(const LineSetup<T> &L)
 // step emits the column it leaves, so a block's emitted columns are its first
 // ones, their centres lie between the block's first and last short-axis
 // positions and their errors below a bound of the whole line (fill_reach).
+// TRACK: the range from the emitted centres and errors themselves, which is a pixel
+// narrower for some segments.  The ordered mode takes it, which can sort only so many
+// segments of a tile.
 // 19 vector instructions per step: the walk of 1000 lines of up to 720 px takes
 // 71 us (131 with the bookkeeping in the step and a store ring), of 128 000
 // lines of up to 400 px 86 us (126).
-template <typename T, typename OnSeg>
+template <bool TRACK, typename T, typename OnSeg>
 __device__ __forceinline__ void walk_segments(const LineSetup<T> &L, int64_t l, const Geometry &g,
                                               int *__restrict__ flags, OnSeg on_seg)
 {
@@ -155,6 +158,8 @@ __device__ __forceinline__ void walk_segments(const LineSetup<T> &L, int64_t l, 
     const int da = ax ? g.H : g.W, db = ax ? g.W : g.H;
     const int sa = pick(L.st, a), sb = pick(L.st, b);
     const int R = fill_reach(L);
+    int q_first = 0, q_last = 0;   // TRACK: `side` at the block's first and last emitted column,
+    T n_most = T(0);               // and the largest |N| at one
     // signed increments along x and y
     const T dx = (L.st[0] > 0) ? L.nv[0] : -L.nv[0], dy = (L.st[1] > 0) ? L.nv[1] : -L.nv[1];
     const T ux = (L.st[0] > 0) ? L.t[0] : -L.t[0], uy = (L.st[1] > 0) ? L.t[1] : -L.t[1];
@@ -173,6 +178,13 @@ __device__ __forceinline__ void walk_segments(const LineSetup<T> &L, int64_t l, 
             const bool yb = m_abs(ey) < m_abs(ex);
             const T m = yb ? ey : ex;
             const bool both = m_abs(exy) < m_abs(m);
+            if constexpr (TRACK) {
+                const bool em = both | (yb == ax);   // a column is left
+                const T an = m_abs(Ne);
+                q_first = em ? max(q_first, side) : q_first;
+                q_last = em ? side : q_last;
+                n_most = (em & (an > n_most)) ? an : n_most;
+            }
             Te += (both | !yb) ? ux : T(0);
             Te += (both | yb) ? uy : T(0);
             Ne = both ? exy : m;
@@ -208,14 +220,27 @@ __device__ __forceinline__ void walk_segments(const LineSetup<T> &L, int64_t l, 
         cur.c[1] = ax ? c : s;
         cur.Te = Te;
         cur.Ne = Ne;
+        if constexpr (TRACK) {
+            q_first = 0;   // (`side` is positive at every step)
+            n_most = T(0);
+        }
         const int k = advance(k0);
         most = max(most, q - side);
         s += sb * (q - side);
         c += sa * k0;
         left = (side > 0) ? left - k0 : 0;
         cur.ncols = k0 - k;
-        cur.lo = max(min(s0, s) - R, 0);
-        cur.hi = min(max(s0, s) + R, db - 1);
+        int e0 = s0, e1 = s, r = R;
+        if constexpr (TRACK) {
+            e0 = s0 + sb * (q - q_first);
+            e1 = s0 + sb * (q - q_last);
+            // as fill_reach; one of the two pixels is for the rounding of up to 2886 steps
+            const double j = ((double)L.w * (double)L.len + (double)n_most) / (double)m_abs(pick(L.t, a));
+            const double reach = __builtin_floor(j) + 2.0 + __builtin_floor(1.2e-7 * j * j);
+            r = reach < 1073741824.0 ? (int)reach : 1073741824;
+        }
+        cur.lo = max(min(e0, e1) - r, 0);
+        cur.hi = min(max(e0, e1) + r, db - 1);
         if ((cur.ncols > 0) & (cur.lo <= cur.hi)) on_seg(cur, tl);
     }
     // (the tile kernels' replay stops after 4 SEG + 16 steps; a walk takes at
@@ -256,7 +281,7 @@ k_segments(const T *__restrict__ lines, const I *__restrict__ idxs, int kernel, 
     }
     const int base = WRITE ? seg_off[l] : 0;
     int nseg = 0;
-    walk_segments(L, l, g, flags, [&](const Segment<T> &cur, int tl) {
+    walk_segments<BIN>(L, l, g, flags, [&](const Segment<T> &cur, int tl) {
         const int sid = base + nseg;
         if (WRITE) segs[sid] = cur;
         if (BIN) {
@@ -396,7 +421,7 @@ k_walk_lines(int64_t n_lines, Geometry g, const LineSetup<T> *__restrict__ setup
     Segment<T> *const dst = segs + base;
     // (axis 0: the long axis runs along tile columns)
     const int fbase = L.frame * (g.nty * g.ntx), ml = (L.axis == 0) ? 1 : g.ntx, mb = (L.axis == 0) ? g.ntx : 1;
-    walk_segments(L, l, g, flags, [&](const Segment<T> &cur, int tl) {
+    walk_segments<false>(L, l, g, flags, [&](const Segment<T> &cur, int tl) {
         if (nseg < ub) dst[nseg] = cur;
         const int tb0 = cur.lo >> g.tile_log, tb1 = cur.hi >> g.tile_log;
         int li = (fbase + tl * ml + tb0 * mb) * LIST_SUBS + L.sub;
