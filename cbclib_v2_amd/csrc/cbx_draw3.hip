@@ -589,6 +589,14 @@ k_setup3(const T *__restrict__ lines, int64_t n_lines, const I *__restrict__ idx
             const double lim = (double)L.w2 * (double)L.len * (double)L.len, tol = sizeof(T) == 4 ? 4e-6 : 1e-13;
             R.in = (T)(lim * (1.0 - tol));
             R.out = (T)(lim * (1.0 + tol));
+            // Squares near the smallest normal number are not accurate to tol, nor is the
+            // correction of a quotient: the limits decide nothing then, and a reciprocal of 0
+            // makes div_rn divide.
+            if (!(lim > (sizeof(T) == 4 ? 1e-30 : 1e-290))) {
+                R.rlen = T(0);
+                R.in = T(0);
+                R.out = (T)__builtin_inf();
+            }
             const T ta = (a == 0) ? L.t[0] : ((a == 1) ? L.t[1] : L.t[2]);
             for (int k = 0; k < 3; k++) {
                 const float slope = (float)(L.t[k] / ta);
