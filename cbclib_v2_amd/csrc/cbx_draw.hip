@@ -2017,8 +2017,11 @@ __device__ __forceinline__ double point_segment2(double px, double py, double ax
 // keeps its term in `touching` and gets frame -1, one alone in its pixels gets
 // -1 in `touching` and keeps its frame; *n_touching counts the former.  Every pixel
 // of a line lies within its width of the segment, up to the drift of the float
-// walk: lines further apart than both widths plus 1 px plus 1e-4 of their lengths
-// share none.  (A line that draws nothing, e.g. a NaN end point, touches none.)
+// walk: lines further apart than both widths, 1 px, 1e-4 of their lengths and 2^-23
+// of the squares of lengths and widths share none.  (The errors' running sums reach
+// length^2 along the line, and width x length in a fill; each of as many additions as
+// there are pixels rounds them by at most 2^-24, and a pixel is `length` of them.)
+// (A line that draws nothing, e.g. a NaN end point, touches none.)
 template <typename T, typename I>
 __global__ void __launch_bounds__(256)
 k_term_touch(const T *__restrict__ lines, const I *__restrict__ terms, const int *__restrict__ off,
@@ -2037,7 +2040,8 @@ k_term_touch(const T *__restrict__ lines, const I *__restrict__ terms, const int
             if (j == (int)i) continue;
             const T *b = lines + 5 * (int64_t)j;
             const double cx = b[0], cy = b[1], dx = b[2], dy = b[3];
-            const double r = wa + (double)b[4] + 1.0 + 1e-4 * (la + fabs(dx - cx) + fabs(dy - cy));
+            const double lb = fabs(dx - cx) + fabs(dy - cy), ws = wa + (double)b[4];
+            const double r = ws + 1.0 + 1e-4 * (la + lb) + 1.2e-7 * (la * la + lb * lb + ws * ws);
             if (!(fmax(cx, dx) + r >= fmin(ax, bx) && fmin(cx, dx) - r <= fmax(ax, bx) &&
                   fmax(cy, dy) + r >= fmin(ay, by) && fmin(cy, dy) - r <= fmax(ay, by)))
                 continue;
