@@ -1151,7 +1151,9 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
             wR[lane] = R;
             if (!replay_columns<SEG>(wK, L, sg, lane * SEG, sg.ncols)) atomicOr(flags, FLAG_STUCK);
         }
-        take(np);
+        // (gaussian: after the fills, whose double exp needs the registers that the next
+        // items would hold; 20 spilled ones made 100 000 lines of 1 to 8 px 211 us, now 205)
+        if constexpr (K != K_GAUSSIAN) take(np);
         wave_sync();
         // phase 2a
         int ncap = 0, cap_lo = 0, cap_hi = 0;   // lane i: item i's columns in the list
@@ -1309,6 +1311,7 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
             p[3] = ax ? a2 : b2;
             p[4] = times(cw, acc[2]);
         }
+        if constexpr (K == K_GAUSSIAN) take(np);
         wave_sync();
     }
 }
