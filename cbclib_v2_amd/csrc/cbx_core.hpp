@@ -545,17 +545,6 @@ __device__ __forceinline__ bool pixel_eval(const LineSetup<double> &L, double Te
     return true;
 }
 
-// dK/du at u = err = (dist / w)^2 for the adjoint; the triangular profile is
-// handled through dist in the caller.
-template <int K>
-__device__ __forceinline__ float profile_du(float u, float kval)
-{
-    if constexpr (K == K_BIWEIGHT) return -1.875f * (1.0f - u);
-    else if constexpr (K == K_PARABOLIC) return -0.75f;
-    else if constexpr (K == K_GAUSSIAN) return -4.5f * kval;
-    else return 0.0f;
-}
-
 // order-preserving encodings for max accumulation in LDS integer atomics
 __device__ __forceinline__ uint32_t ord_enc(float v)
 {

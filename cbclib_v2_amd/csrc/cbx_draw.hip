@@ -929,8 +929,7 @@ __device__ __forceinline__ void pixel_grad(const GradConst &C, int x, int y, dou
 // per row.  The lanes of one item read the same short-axis coordinate in 8 or
 // 16 consecutive rows (steep lines); with a pitch of TILE (a multiple of the
 // bank count) those reads fall in one bank, with TILE + 4 in distinct banks.
-// (The tile kernel keeps a pitch of TILE: its padded variants measured slower,
-// see k_tiles.)
+// (k_tiles_fast pads its rows alike; k_tiles does not, where padding spilled.)
 template <int TILE>
 constexpr int tile_pitch() { return TILE + 4; }
 

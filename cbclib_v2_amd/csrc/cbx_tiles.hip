@@ -900,17 +900,19 @@ static void launch_tiles(T *out, const SegmentPlan<T> &P, T max_val, int threads
 #define CBX_TILES(NT, CH, FST)                                                                                  \
     k_tiles<T, K, OV, TILE, SEG, NT, CH, FST><<<(unsigned)P.n_tiles, NT, 0, st>>>(                             \
         out, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, max_val, P.flags.ptr)
-    if (fast) {
-        if (threads == 64) CBX_TILES(64, 64, true);
-        else if (threads == 128) CBX_TILES(128, 64, true);
-        else if (chunk == 64) CBX_TILES(256, 64, true);
-        else CBX_TILES(256, 256, true);
-    } else {
-        if (threads == 64) CBX_TILES(64, 64, false);
-        else if (threads == 128) CBX_TILES(128, 64, false);
-        else if (chunk == 64) CBX_TILES(256, 64, false);
-        else CBX_TILES(256, 256, false);
+    if constexpr (sizeof(T) == 4) {   // (the values of doubles are always exact)
+        if (fast) {
+            if (threads == 64) CBX_TILES(64, 64, true);
+            else if (threads == 128) CBX_TILES(128, 64, true);
+            else if (chunk == 64) CBX_TILES(256, 64, true);
+            else CBX_TILES(256, 256, true);
+            return;
+        }
     }
+    if (threads == 64) CBX_TILES(64, 64, false);
+    else if (threads == 128) CBX_TILES(128, 64, false);
+    else if (chunk == 64) CBX_TILES(256, 64, false);
+    else CBX_TILES(256, 256, false);
 #undef CBX_TILES
 }
 
