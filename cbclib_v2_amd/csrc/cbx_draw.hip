@@ -1080,11 +1080,18 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
     const float *const fg = grad + ((f * g.H + Y0) * (int64_t)g.W + X0);
     constexpr int PP = PX / NT;
     float gv[PP];
+    // (rows below the frame, which no fill reaches, are left out four of the wave's at a time)
+    auto inside = [&](int j) { return (wave * 64 + j * NT) / TILE < Y1 - Y0; };
+    static_assert(PP % 4 == 0, "groups of 4");
 #pragma unroll
-    for (int j = 0; j < PP; j++) {
-        const int i = tid + j * NT;
-        const int y = i / TILE, x = i % TILE;
-        gv[j] = (y < Y1 - Y0 && x < X1 - X0) ? __builtin_nontemporal_load(fg + ((int64_t)y * g.W + x)) : 0.0f;
+    for (int j0 = 0; j0 < PP; j0 += 4) {
+        if (!inside(j0)) continue;
+#pragma unroll
+        for (int j = j0; j < j0 + 4; j++) {
+            const int i = tid + j * NT;
+            const int y = i / TILE, x = i % TILE;
+            gv[j] = (y < Y1 - Y0 && x < X1 - X0) ? __builtin_nontemporal_load(fg + ((int64_t)y * g.W + x)) : 0.0f;
+        }
     }
     // equal chunks, the same number of turns for every wave
     const int turns = (end - beg + NW * CHW - 1) / (NW * CHW);
@@ -1102,9 +1109,13 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
     // (lanes without an item load the list's last)
     take(pairs[min(beg + wave * size + lane, end - 1)]);
 #pragma unroll
-    for (int j = 0; j < PP; j++) {
-        const int i = tid + j * NT;
-        gt[(i / TILE) * PITCH + (i % TILE)] = gv[j];
+    for (int j0 = 0; j0 < PP; j0 += 4) {
+        if (!inside(j0)) continue;
+#pragma unroll
+        for (int j = j0; j < j0 + 4; j++) {
+            const int i = tid + j * NT;
+            gt[(i / TILE) * PITCH + (i % TILE)] = gv[j];
+        }
     }
     __syncthreads();
 
@@ -1310,6 +1321,7 @@ k_adjoint_fast(const float *__restrict__ grad, const float *__restrict__ lines, 
             p[3] = ax ? a2 : b2;
             p[4] = times(cw, acc[2]);
         }
+        if (t + 1 == turns) break;   // (no items to wait for: 20 000 frames of 64^2, a line each, 195 -> 189 us)
         if constexpr (K == K_GAUSSIAN) take(np);
         wave_sync();
     }
@@ -1677,12 +1689,14 @@ static int build_plan_unordered(SegmentPlan<T> &P, const T *lines, const I *idxs
 // tiles, 161 / 131 at 256; gradients 170 / 148 at 64, 178 / 163 at 256, 136 / 140 at
 // 704; float draws 79 / 61 with 5000 lines in 64 tiles, 118 / 114 with 1000, and
 // where a tile has a few lines only 75 / 78 (192 lines in 64 tiles, gradient 102 / 101).
+// A frame of at most 32 x 32 is one tile either way, of which less is cleared, read and
+// written (20 000 frames of 16^2, a line each: 108 / 82, gradient 164 / 153).
 // The frames decide, not the lines or the pass, so that a plan, the eager draw and the
 // eager gradient of the same frames work on the same tiles and give the same bits.
 static void resolve_opts(const cbx_draw_opts *o, int64_t n_frames, int64_t H, int64_t W, int &tile, int &seg)
 {
     const double tiles = (double)n_frames * (double)((H + 63) / 64) * (double)((W + 63) / 64);
-    tile = (o && o->tile) ? o->tile : (tiles <= 256.0 ? 32 : 64);
+    tile = (o && o->tile) ? o->tile : ((tiles <= 256.0 || (H <= 32 && W <= 32)) ? 32 : 64);
     seg = (o && o->seg) ? o->seg : 8;
 }
 

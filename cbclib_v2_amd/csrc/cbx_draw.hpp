@@ -257,6 +257,16 @@ struct SegmentPlan {
     DevBuf<Segment<T>> segs;
 };
 
+// Tiles of a few items each, and more of them than run at a time (four workgroups on each
+// of 256 CUs): the tile kernel that holds less of a tile (FEW).  us without / with it for
+// 64 frames of 1024^2 with 2, 8, 12, 16 and 24 items in a tile: sums 123 / 109, 164 / 159,
+// 175 / 173, 182 / 186, 199 / 212; maxima 107 / 104, 146 / 141, 157 / 150, 167 / 160, 188 / 180.
+template <typename T>
+inline bool few_items(const SegmentPlan<T> &P)
+{
+    return P.n_tiles > 1024 && P.n_items < 12 * P.n_tiles;
+}
+
 // The tile kernel of one profile (CBX_PROFILE of cbx_tiles.hip; K_MIXED: per-line
 // profiles) over a built unordered plan.
 template <typename T, int K>

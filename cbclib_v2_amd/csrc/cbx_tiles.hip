@@ -571,8 +571,14 @@ __device__ __forceinline__ void fill_interior(Acc *img, uint32_t *zb, const Inne
 // 2.1 ms).  With one tested, sequential loop per half column (k_tiles' fills) and
 // one wave replaying the walks of the whole workgroup the same took 0.66, 0.60
 // and 5.1 ms: 60 % of the instructions were the loop's tests, masks and idle lanes.
-template <int K, int OV, int TILE, int SEG, int NT, int CHW>
-__global__ void __launch_bounds__(NT, 4)
+//
+// FEW: tiles of a few items, whose time is latency.  Half the records and no pixel
+// values held beside them, so that five workgroups fit a CU instead of four, and
+// only touched pixels are read and written, by the same operations.  20 000 frames of
+// 64^2 with a line each: call 138 -> 123 us (max 119 -> 115), 133 (119) with k_tiles'
+// fills; of 33 x 33 with two 175 -> 147 (158).
+template <int K, int OV, int TILE, int SEG, int NT, int CHW, bool FEW>
+__global__ void __launch_bounds__(NT, FEW ? 6 : 4)
 k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_off, const int2 *__restrict__ pairs,
              const Segment<float> *__restrict__ segs, const LineSetup<float> *__restrict__ setup,
              const LineLite *__restrict__ lite, float max_val, int *__restrict__ flags)
@@ -608,7 +614,7 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
     // pixels per load where rows allow it, else one (clamped into the frame:
     // pixels outside it are not stored)
     constexpr int PP = PX / NT;   // pixels per thread
-    constexpr bool PREF = OV == 2 && PP <= 16 && PP % 4 == 0;
+    constexpr bool PREF = OV == 2 && PP <= 16 && PP % 4 == 0 && !FEW;
     float pre[PREF ? PP : 1];
     if constexpr (PREF) {
         if (full) {
@@ -785,11 +791,36 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
         if constexpr (OV == 2) {
             // fold the round into the pixel values (registers or `out`)
             const double scale = ldexp((double)max_val, -F);
-            const float zero = max_val * 0.0f;
-            if (PREF && full) {
+            const float zero = max_val * 0.0f, p2 = __int_as_float((127 - F) << 23);   // 2^-F, F <= 31
+            if constexpr (FEW) {
+                // the touched pixels only, a batch's loads before its stores
+                constexpr int B = PP < 8 ? PP : 8;
+                int t0 = tid;
+                asm("" : "+v"(t0));   // (addresses are made here, not kept in registers through the round)
+#pragma unroll 1
+                for (int i0 = t0; i0 < (Y1 - Y0) * TILE; i0 += B * NT) {
+                    float o[B];
+                    uint32_t acc[B], z[B];
+#pragma unroll
+                    for (int j = 0; j < B; j++) {
+                        const int i = i0 + j * NT, y = i / TILE, x = i % TILE, li = y * PITCH + x;
+                        acc[j] = img[li];
+                        z[j] = (zb[li >> 5] >> (li & 31)) & 1u;
+                        // (pixels outside the frame are never touched)
+                        o[j] = (acc[j] | z[j]) ? to[(int64_t)y * g.W + x] : 0.0f;
+                    }
+#pragma unroll
+                    for (int j = 0; j < B; j++) {
+                        const int i = i0 + j * NT, y = i / TILE, x = i % TILE;
+                        if (!(acc[j] | z[j])) continue;
+                        const double add = acc[j] ? (double)acc[j] * scale : (double)zero;
+                        to[(int64_t)y * g.W + x] =
+                            full ? fold_fix(o[j], acc[j], z[j], p2, max_val, zero) : (float)((double)o[j] + add);
+                    }
+                }
+            } else if (PREF && full) {
                 // all LDS reads first (4 pixels and their zero bits per read),
                 // then branch-free updates
-                const float p2 = __int_as_float((127 - F) << 23);   // 2^-F, F <= 31
                 const uint32_t l4 = (uint32_t)tid * 4 / TILE * PITCH + (uint32_t)tid * 4 % TILE;
                 uint4 acc[PP / 4];
                 uint32_t zw[PP / 4];
@@ -854,8 +885,8 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
         }
     } else if constexpr (OV == 1) {
         // every value is requested before any is used; std::max(out, value)
-        constexpr int B = PP < 16 ? PP : 16;
-        for (int i0 = tid; i0 < PX; i0 += B * NT) {
+        constexpr int B = FEW ? (PP < 8 ? PP : 8) : (PP < 16 ? PP : 16);
+        for (int i0 = tid; i0 < (FEW ? (Y1 - Y0) * TILE : PX); i0 += B * NT) {
             float o[B];
             uint32_t e[B];
 #pragma unroll
@@ -863,7 +894,8 @@ k_tiles_fast(float *__restrict__ out, Geometry g, const int *__restrict__ tile_o
                 const int i = i0 + j * NT;
                 const int y = i / TILE, x = i % TILE;
                 e[j] = img[y * PITCH + x];
-                o[j] = to[(int64_t)min(y, Y1 - Y0 - 1) * g.W + min(x, X1 - X0 - 1)];
+                if constexpr (FEW) o[j] = e[j] ? to[(int64_t)y * g.W + x] : 0.0f;
+                else o[j] = to[(int64_t)min(y, Y1 - Y0 - 1) * g.W + min(x, X1 - X0 - 1)];
             }
 #pragma unroll
             for (int j = 0; j < B; j++) {
@@ -880,16 +912,17 @@ template <int K, int OV, int TILE, int SEG>
 static void launch_fast(float *out, const SegmentPlan<float> &P, float max_val, int threads, int chunk, bool,
                         hipStream_t st)
 {
-#define CBX_TILES_FAST(NT, CHW)                                                                                 \
-    k_tiles_fast<K, OV, TILE, SEG, NT, CHW><<<(unsigned)P.n_tiles, NT, 0, st>>>(                               \
+#define CBX_TILES_FAST(NT, CHW, FEW)                                                                            \
+    k_tiles_fast<K, OV, TILE, SEG, NT, CHW, FEW><<<(unsigned)P.n_tiles, NT, 0, st>>>(                               \
         out, P.g, P.tile_off.ptr, P.pairs.ptr, P.segs.ptr, P.setup.ptr, P.lite.ptr, max_val, P.flags.ptr)
     // 256 records per wave: four workgroups' areas fit a CU's LDS and the tile's few items spread over
     // its waves (64 frames of 2048^2, seg 8: 24 / 32 / 48 items 0.604 / 0.592 / 0.721 ms; 256 of 1024^2,
     // seg 16: 8 / 16 / 24 / 32 items 3.72 / 2.80 / 3.07 / 2.89 ms)
-    if (threads == 64) CBX_TILES_FAST(64, 64);
-    else if (threads == 128) CBX_TILES_FAST(128, 32);
-    else if (chunk == 64) CBX_TILES_FAST(256, (SEG == 8 ? 32 : 16));
-    else CBX_TILES_FAST(256, (SEG == 8 ? 64 : 32));
+    if (threads == 64) CBX_TILES_FAST(64, 64, false);
+    else if (threads == 128) CBX_TILES_FAST(128, 32, false);
+    else if (chunk == 64 && few_items(P)) CBX_TILES_FAST(256, 128 / SEG, true);
+    else if (chunk == 64) CBX_TILES_FAST(256, (SEG == 8 ? 32 : 16), false);
+    else CBX_TILES_FAST(256, (SEG == 8 ? 64 : 32), false);
 #undef CBX_TILES_FAST
 }
 
