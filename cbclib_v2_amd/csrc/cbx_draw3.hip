@@ -623,7 +623,7 @@ __device__ __forceinline__ unsigned long long patch_bits(double v) { return (uns
 __device__ __forceinline__ float patch_value(uint32_t b) { return __uint_as_float(b); }
 __device__ __forceinline__ double patch_value(unsigned long long b) { return __longlong_as_double((long long)b); }
 
-// Fills of the recorded planes.  A wave takes FILL_PLANES consecutive planes, one
+// Fills of the recorded planes.  A wave takes 2^planes_log consecutive planes, one
 // (plane, quadrant) per lane (fill3_quadrant's pixels: a walk away from the
 // line with, from each of its pixels, a ray along the other axis for each axis
 // that the next step moves).  Walk and rays are one loop, a candidate pixel of
@@ -644,17 +644,26 @@ __device__ __forceinline__ double patch_value(unsigned long long b) { return __l
 // the issue rate, for 50 000 lines of widths 1 to 3, 13 M voxels, in 16 volumes
 // of 64 x 128 x 128).  A wave's patch and queue limit the waves in flight: with
 // patches of 1536, 1024, 768, 640 values 526, 433, 387, 381 us (planes that
-// find no room in the patch are added directly, so not smaller still).
+// find no room in the patch are added directly, so not smaller still).  Planes
+// whose rows reach less than 2 steps from the centre have too few neighbours to
+// gather: 200 000 lines of widths 0.2 to 0.6 take 396 us with patches, 283 without
+// (349 with one lane per (plane, quadrant)).
 // For max hardly any voxel is written (most are below what is there), so its
 // patch is kept to the smallest planes: 525 us with the patches of the sums, 465
 // with 64 values; 20 000 lines of widths 2 to 6 in doubles 984 and 795.
 // One lane per (plane, quadrant) with atomics for every pixel took 623 us.
 constexpr int FILL_PLANES = 16, FILL_NT = 256, FILL_QUEUE = 128;
 
-template <typename T, int K, int OV>
+//
+// RAYS: for so few planes that the widest one's quadrant, its lane's chain of steps, is
+// the time.  While every lane of the wave is on a ray, its steps run in a loop of their
+// own (a third of the instructions): 50 lines of widths 10 to 25 743 -> 504 us.  With
+// full waves that seldom happens, and the second copy of the loop costs (50 000 lines
+// 423 -> 460).  One instance for all profiles (K_MIXED, the profile in kid).
+template <typename T, int K, int OV, bool RAYS>
 __global__ void __launch_bounds__(FILL_NT)
 k_fill3(T *__restrict__ out, const Rec3<T> *__restrict__ rec, const PlaneState<T> *__restrict__ states,
-        int64_t n_states, Vol3 v, T max_val, int *__restrict__ flags)
+        int64_t n_states, int planes_log, Vol3 v, T max_val, int kid, int *__restrict__ flags)
 {
     constexpr int NW = FILL_NT / 64, PATCH = (OV == 1) ? 64 : (sizeof(T) == 4 ? 768 : 512);
     using Bits = typename std::conditional<sizeof(T) == 4, uint32_t, unsigned long long>::type;
@@ -672,9 +681,10 @@ k_fill3(T *__restrict__ out, const Rec3<T> *__restrict__ rec, const PlaneState<T
     __shared__ Plane plane[NW][FILL_PLANES];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint64_t below = (1ull << lane) - 1ull;
-    const int64_t first = ((int64_t)blockIdx.x * NW + wave) * FILL_PLANES;
-    const int pl = lane & (FILL_PLANES - 1), quad = lane / FILL_PLANES;
-    const bool have = first + pl < n_states;
+    const int planes = 1 << planes_log;
+    const int64_t first = ((int64_t)blockIdx.x * NW + wave) << planes_log;
+    const int pl = lane & (planes - 1), quad = lane >> planes_log;
+    const bool have = quad < 4 && first + pl < n_states;
     PlaneState<T> ps;
     ps.line = -1;
     if (have) ps = states[first + pl];
@@ -729,7 +739,7 @@ k_fill3(T *__restrict__ out, const Rec3<T> *__restrict__ rec, const PlaneState<T
         const bool one = flip1 != flip2;   // the first step: along (a + 2) % 3 when exactly one axis is flipped
         alongP = (a == 1) ? one : !one;
         const int spanP = (P == 0) ? L->span[0] : L->span[1], spanQ = (Q == 1) ? L->span[1] : L->span[2];
-        side = (a != 0 && flat && spanP < 32 && spanQ < 32) ? (2 * spanP + 1) * (2 * spanQ + 1) : 0;
+        side = (a != 0 && flat && spanP >= 2 && spanP < 32 && spanQ < 32) ? (2 * spanP + 1) * (2 * spanQ + 1) : 0;
         if (quad == 0) {
             Plane &p = plane[wave][pl];
             p.centre = ((L->frame * v.D + ps.cur[2]) * v.H + ps.cur[1]) * v.W + ps.cur[0];
@@ -745,11 +755,11 @@ k_fill3(T *__restrict__ out, const Rec3<T> *__restrict__ rec, const PlaneState<T
         int x = side;
 #pragma unroll
         for (int d = 1; d < FILL_PLANES; d <<= 1) {
-            const int y = __shfl_up(x, d, FILL_PLANES);
+            const int y = __shfl_up(x, d, 64);   // (a quadrant's lanes are neighbours)
             if (pl >= d) x += y;
         }
         if (quad == 0) plane[wave][pl].patch = (side > 0 && x <= PATCH) ? x - side : -1;
-        const int all = min(__shfl(x, FILL_PLANES - 1, FILL_PLANES), PATCH);
+        const int all = min(__shfl(x, planes - 1, 64), PATCH);
         for (int i = lane; i < all; i += 64) patch[wave][i] = (Bits)~(Bits)0;   // (a NaN that no value has)
     }
     wave_fence();
@@ -764,7 +774,7 @@ k_fill3(T *__restrict__ out, const Rec3<T> *__restrict__ rec, const PlaneState<T
         const Rec3<T> &R = rec[p.line];
         const T e = err3(R, pte, nerr3(R, pne));
         if (!(e <= T(1))) return;
-        const T val = pixel_value<K>(e, max_val);
+        const T val = pixel_value_of<K>(kid, e, max_val);
         if (held)
             patch[wave][p.patch + (qQ + p.spanQ) * (2 * p.spanP + 1) + qP + p.spanP] = patch_bits(val);
         else
@@ -846,10 +856,28 @@ k_fill3(T *__restrict__ out, const Rec3<T> *__restrict__ rec, const PlaneState<T
         oP = (on ? oP : xP) + (mP ? dP : 0);
         oQ = (on ? oQ : xQ) + (mQ ? dQ : 0);
         dir = on ? dir : (walk ? (nP ? 1 : 2) : (second ? 2 : 0));
+        if constexpr (RAYS) {
+            if (__ballot(go && !on) != 0) continue;
+            const bool rP = dir == 2;
+            const T st = rP ? stP : stQ, i0 = rP ? iP[0] : iQ[0], i1 = rP ? iP[1] : iQ[1], i2 = rP ? iP[2] : iQ[2];
+            const int sP = rP ? dP : 0, sQ = rP ? 0 : dQ;
+            while (__ballot(go)) {
+                const T r2 = ne[0] * ne[0] + ne[1] * ne[1] + ne[2] * ne[2];
+                if (__ballot(go && !(r2 < s_in && count < cap)) != 0) break;   // (for the step above)
+                push(go && oP >= loP && oP <= hiP && oQ >= loQ && oQ <= hiQ);
+                count++;
+                te += st;
+                ne[0] += i0;
+                ne[1] += i1;
+                ne[2] += i2;
+                oP += sP;
+                oQ += sQ;
+            }
+        }
     }
     drain(q_tail - q_head);
     // the patches' rows
-    for (int k = 0; k < FILL_PLANES; k++) {
+    for (int k = 0; k < planes; k++) {
         if (first + k >= n_states) break;
         const bool used = __shfl(side, k, 64) > 0;
         if (!used) continue;
@@ -996,14 +1024,26 @@ template <typename T, int OV>
 static void launch_fill3(int kernel, T *out, const Rec3<T> *rec, const PlaneState<T> *states, int64_t n_states,
                          const Vol3 &v, T mv, int *flags, hipStream_t st)
 {
-    const unsigned g = (unsigned)((n_states + FILL_PLANES * (FILL_NT / 64) - 1) / (FILL_PLANES * (FILL_NT / 64)));
-#define CBX_FILL3(KK) k_fill3<T, KK, OV><<<g, FILL_NT, 0, st>>>(out, rec, states, n_states, v, mv, flags)
+    // Planes of a wave: 16, or fewer where that would leave SIMDs without a wave to
+    // work for the widest planes (us with 16 / 8 / 4 / 2 planes: 62 000 planes of widths 5 to
+    // 9 397 / 353 / 352 / 514, 15 000 of 10 to 25 1133 / 855 / 700 / 862, 3800 of them 1257 /
+    // 966 / 817 / 741, with RAYS and one 504; 2.8 M of 0.2 to 0.6 283 / 412 / 648 / 1100).
+    const bool rays = n_states < 8192;
+    const int planes_log = rays ? 0 : (n_states < 32768 ? 2 : (n_states < 131072 ? 3 : 4));
+    const int64_t per_group = (int64_t)(FILL_NT / 64) << planes_log;
+    const unsigned g = (unsigned)((n_states + per_group - 1) / per_group);
+#define CBX_FILL3(KK, RAYS)                                                                                     \
+    k_fill3<T, KK, OV, RAYS><<<g, FILL_NT, 0, st>>>(out, rec, states, n_states, planes_log, v, mv, kernel, flags)
+    if (rays) {
+        CBX_FILL3(K_MIXED, true);
+        return;
+    }
     switch (kernel) {
-    case K_BIWEIGHT: CBX_FILL3(K_BIWEIGHT); break;
-    case K_GAUSSIAN: CBX_FILL3(K_GAUSSIAN); break;
-    case K_PARABOLIC: CBX_FILL3(K_PARABOLIC); break;
-    case K_RECTANGULAR: CBX_FILL3(K_RECTANGULAR); break;
-    default: CBX_FILL3(K_TRIANGULAR); break;
+    case K_BIWEIGHT: CBX_FILL3(K_BIWEIGHT, false); break;
+    case K_GAUSSIAN: CBX_FILL3(K_GAUSSIAN, false); break;
+    case K_PARABOLIC: CBX_FILL3(K_PARABOLIC, false); break;
+    case K_RECTANGULAR: CBX_FILL3(K_RECTANGULAR, false); break;
+    default: CBX_FILL3(K_TRIANGULAR, false); break;
     }
 #undef CBX_FILL3
 }
