@@ -245,7 +245,7 @@ def workload_c3(args):
             "roofline": {"bound": "hbm", "achieved": round(fwd_bytes / (tile_avg * 1e-3) / 1e9, 2),
                          "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(fwd_bytes / (tile_avg * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                         "kernel": "k_tiles", "avg_launch_ms": round(tile_avg, 4), "bytes_per_launch": fwd_bytes},
+                         "kernel": "k_tiles_fast", "avg_launch_ms": round(tile_avg, 4), "bytes_per_launch": fwd_bytes},
             "config": {"workload": f"batched uneven forward: {F} frames of {H}x{W} f32, {N} segments (per-frame counts "
                                    "log-uniform in [100, 20000], seed 2), per-line triangular/gaussian, sum; "
                                    "step = zero + one plan draw replayed from a HIP graph",
@@ -306,7 +306,7 @@ def workload_c4(args):
     adj_gbs = adj_bytes / (adj_avg * 1e-3) / 1e9 if adj_n else 0.0
     return {"metric": "fwd+adjoint frames/s (C4)", "value": round(F / (ms * 1e-3), 2), "unit": "frames/s",
             "adjoint_roofline": {"bound": "hbm", "achieved": round(adj_gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                                 "frac": round(adj_gbs / HBM_PEAK_GBS, 4), "kernel": "k_adjoint_tiles",
+                                 "frac": round(adj_gbs / HBM_PEAK_GBS, 4), "kernel": "k_adjoint_fast",
                                  "bytes_per_launch": adj_bytes, "avg_launch_ms": round(adj_avg, 4)},
             "ms_per_step": round(ms, 4), "Mlines_per_s": round(N / (ms * 1e-3) / 1e6, 4),
             "config": {"workload": f"forward + adjoint: {F} frames of {H}x{W} f32, {N} segments ({per}/frame, "
@@ -748,8 +748,8 @@ def main() -> None:
                                "Structure([0,1,1],2)); step = zero + draw_lines + label",
                    "frames": F, "segments": N, "tile": args.tile or 64, "seg": args.seg or 8},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic('k_tiles'),
-                     "kernel": "k_tiles (draw_lines tile accumulation)",
+                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic('k_tiles_fast'),
+                     "kernel": "k_tiles_fast (draw_lines tile accumulation)",
                      "bytes_per_launch": fwd_bytes, "avg_launch_ms": round(tile_avg, 4), "launches": tiles_n},
         "fwd_Mlines_per_s": round(N / (acc['fwd'] / 2 * 1e-3) / 1e6, 4),
         "fwd_label_frames_per_s": round(F / (ms_step * 1e-3), 2),

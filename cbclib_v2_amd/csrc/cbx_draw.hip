@@ -32,8 +32,9 @@
 // different overlaps): k_segments walks twice (count, then write) so that a
 // line's segments are consecutive and lines keep their input order, and
 // k_tiles_ordered applies each pixel's terms in ascending line order, the
-// single-threaded reference's order.  accumulate_lines of float lines in short
-// terms takes the tile path instead (k_term_order, k_tiles_terms).  The adjoint
+// single-threaded reference's order.  Float lines of accumulate_lines that no
+// other line of their term can touch take the tile path with exact values
+// instead (k_term_touch).  The adjoint
 // (k_adjoint_fast, k_adjoint_tiles for doubles, k_line_grad) runs on the tile
 // path's segments and lists.
 #include <hip/hip_runtime.h>

@@ -566,9 +566,9 @@ __device__ __forceinline__ void fill_interior(Acc *img, uint32_t *zb, const Inne
 //
 // Bound by vector instruction issue: 64 frames of 2048^2 with 128 000 gaussian
 // lines take 0.59 ms (the image alone is 0.46 ms at a copy's rate), 32 of 1024^2
-// with 160 000 biweight lines 0.32 ms (170 M wave instructions, 0.28 ms at the
-// issue rate), 256 of 1024^2 with 962 000 lines of mixed profiles 2.5 ms (1311 M,
-// 2.1 ms).  With one tested, sequential loop per half column (k_tiles' fills) and
+// with 160 000 biweight lines 0.33 ms (175 M wave instructions, 0.28 ms at the
+// issue rate), 256 of 1024^2 with 972 000 lines of mixed profiles and 16-column
+// segments 2.6 ms (1356 M, 2.2 ms).  With one tested, sequential loop per half column (k_tiles' fills) and
 // one wave replaying the walks of the whole workgroup the same took 0.66, 0.60
 // and 5.1 ms: 60 % of the instructions were the loop's tests, masks and idle lanes.
 //

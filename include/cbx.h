@@ -62,8 +62,8 @@ CBX_API int cbx_kernel_id(const char *name);
 /*
  * Launch options of draw_lines (NULL = automatic).  `tile` is the side of the
  * square pixel tile one workgroup accumulates in LDS (32 or 64; 0 = 64, or 32
- * where the frames have few tiles), `seg` the number of long-axis columns per
- * walk checkpoint (8 or 16; 0 = 8).  `deterministic`
+ * where the frames have few tiles or are no larger; by the frames alone), `seg`
+ * the number of long-axis columns per walk checkpoint (8 or 16; 0 = 8).  `deterministic`
  * = 1 accumulates every pixel in ascending line order starting from the value
  * already in `out`, which is the single-threaded reference's order: the
  * result is then bit-identical to bresenham.draw_lines(..., num_threads=1).
